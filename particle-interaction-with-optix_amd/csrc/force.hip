@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) void k_pair_count(const float4* __restrict__ p
     rowcnt[__float_as_uint(pi.w)] = cnt;
 }
 
-// Pass 2: the partners' original indices, then each row sorted ascending.
+// Pass 2: the partners' original indices in walk order (sort_rows then orders each row).
 template <int PRED>
 __global__ __launch_bounds__(256) void k_pair_fill(const float4* __restrict__ pos, const uint32_t* __restrict__ cell_of,
                                                    const uint32_t* __restrict__ off, uint32_t n, GridGeom g,
@@ -175,8 +175,7 @@ __global__ __launch_bounds__(256) void k_pair_fill(const float4* __restrict__ po
     int32_t cx, cy, cz;
     cell_coords(g, cell_of[k], cx, cy, cz);
     const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx < g.g[0] - 1 ? cx + 1 : g.g[0] - 1;
-    const unsigned long long r0 = rows[i];
-    unsigned long long w = r0;
+    unsigned long long w = rows[i];
     for (int32_t zz = cz - 1; zz <= cz + 1; ++zz) {
         if (zz < 0 || zz >= g.g[2]) continue;
         for (int32_t yy = cy - 1; yy <= cy + 1; ++yy) {
@@ -188,16 +187,6 @@ __global__ __launch_bounds__(256) void k_pair_fill(const float4* __restrict__ po
                 if (t != k && pair_mult<PRED>(c, pi, pj, d2) > 0) cols[w++] = __float_as_uint(pj.w);
             }
         }
-    }
-    // insertion sort of the row (rows hold tens of entries)
-    for (unsigned long long a = r0 + 1; a < w; ++a) {
-        const uint32_t v = cols[a];
-        unsigned long long b = a;
-        while (b > r0 && cols[b - 1] > v) {
-            cols[b] = cols[b - 1];
-            --b;
-        }
-        cols[b] = v;
     }
 }
 
@@ -440,6 +429,7 @@ int pairs_cellgrid(lj_context* ctx, const float* x, const float* y, const float*
         LJ_FILL(LJ_PRED_AABB) LJ_FILL(LJ_PRED_CUSTOM) LJ_FILL(LJ_PRED_CUDALJ) LJ_FILL(LJ_PRED_SPHERE) LJ_FILL(LJ_PRED_TRIANGLE)
 #undef LJ_FILL
     }
+    sort_rows(rows, n, cols, s);
     LJ_HIP(ctx, hipGetLastError());
     return LJ_OK;
 }

@@ -504,15 +504,6 @@ __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_fill(const float4* __restri
             cols[w++] = __float_as_uint(pj.w);
     });
     if (!ok) atomicOr(overflow, 1);
-    for (unsigned long long a = r0 + 1; a < w; ++a) {
-        const uint32_t v = cols[a];
-        unsigned long long b = a;
-        while (b > r0 && cols[b - 1] > v) {
-            cols[b] = cols[b - 1];
-            --b;
-        }
-        cols[b] = v;
-    }
 }
 
 // Marks the results of a force call whose walk tripped its step guard: n_pairs =
@@ -760,6 +751,7 @@ int lj_lbvh_pairs(lj_context* ctx, const float* x, const float* y, const float* 
         LJ_F(LJ_PRED_AABB) LJ_F(LJ_PRED_CUSTOM) LJ_F(LJ_PRED_SPHERE) LJ_F(LJ_PRED_TRIANGLE)
 #undef LJ_F
     }
+    sort_rows(row_offsets, n, cols, s);
     LJ_HIP(ctx, hipGetLastError());
     return LJ_OK;
 }

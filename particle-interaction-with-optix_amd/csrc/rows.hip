@@ -1,0 +1,207 @@
+// rows.hip -- sorting the rows of a CSR neighbour list in place.
+//
+// The list calls append each particle's partners in walk order (cells, or the tree's
+// leaves) and promise rows in ascending index order.  The reference has no lists; its
+// OptiX programs visit a particle's partners in the order the hardware reports them
+// (SDK/optixMultiSphereAABB/optixLJ.cu:134-176).
+#include "lj_internal.h"
+
+namespace lj {
+
+namespace {
+
+constexpr int kSortThreads = 256;
+constexpr int kRowLanes = 16;                                // lanes of a row: one DPP row
+constexpr int kBlockRows = kSortThreads / kRowLanes;         // rows of a workgroup
+constexpr uint32_t kRegRow = 16 * kRowLanes;                 // longest row sorted in registers
+constexpr uint32_t kLdsRow = 4096;                           // longest row sorted in LDS
+
+// DPP controls of the lane exchanges inside 16 lanes.
+constexpr int kXor1 = 0xB1;         // quad_perm [1,0,3,2]
+constexpr int kXor2 = 0x4E;         // quad_perm [2,3,0,1]
+constexpr int kMirror4 = 0x1B;      // quad_perm [3,2,1,0]
+constexpr int kMirror16 = 0x140;    // row_mirror
+constexpr int kMirror8 = 0x141;     // row_half_mirror
+
+template <int CTRL>
+__device__ inline uint32_t from_lane(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+
+// One exchange across lanes: element r of a lane against element r (or, mirrored, K - 1
+// - r) of its partner; the lanes with `bit` clear keep the smaller one.
+template <int K, int CTRL, bool MIRROR>
+__device__ inline void cross(uint32_t (&a)[K], unsigned bit) {
+    const bool upper = (threadIdx.x & bit) != 0;
+    uint32_t o[K];
+#pragma unroll
+    for (int r = 0; r < K; ++r) o[r] = from_lane<CTRL>(a[MIRROR ? K - 1 - r : r]);
+#pragma unroll
+    for (int r = 0; r < K; ++r) a[r] = upper ? max(a[r], o[r]) : min(a[r], o[r]);
+}
+
+// Exchange with the lane 4 away: the two halves of each 8 lanes mirrored, then each
+// half mirrored back.
+template <int K>
+__device__ inline void cross4(uint32_t (&a)[K]) {
+    const bool upper = (threadIdx.x & 4u) != 0;
+    uint32_t o[K];
+#pragma unroll
+    for (int r = 0; r < K; ++r) o[r] = from_lane<kMirror4>(from_lane<kMirror8>(a[r]));
+#pragma unroll
+    for (int r = 0; r < K; ++r) a[r] = upper ? max(a[r], o[r]) : min(a[r], o[r]);
+}
+
+__device__ inline void order(uint32_t& lo, uint32_t& hi) {
+    const uint32_t x = lo, y = hi;
+    lo = min(x, y);
+    hi = max(x, y);
+}
+
+// The exchanges at distances D, D / 2, ..., 1 inside a lane's K elements.
+template <int K, int D>
+__device__ inline void within(uint32_t (&a)[K]) {
+    if constexpr (D >= 1) {
+#pragma unroll
+        for (int r = 0; r < K; ++r)
+            if ((r & D) == 0) order(a[r], a[r + D]);
+        within<K, D / 2>(a);
+    }
+}
+
+// Stages 2, 4, ..., K of the sort inside a lane: each first compares mirrored elements
+// of a block, then halves the distance, so every comparison puts the smaller first.
+template <int K, int S>
+__device__ inline void lane_stages(uint32_t (&a)[K]) {
+    if constexpr (S <= K) {
+#pragma unroll
+        for (int b = 0; b < K; b += S)
+#pragma unroll
+            for (int r = 0; r < S / 2; ++r) order(a[b + r], a[b + S - 1 - r]);
+        within<K, S / 4>(a);
+        lane_stages<K, S * 2>(a);
+    }
+}
+
+// Sorts the 16 K elements of a row, element lane K + r in register r of its lane
+// (Batcher's bitonic sort, "Sorting networks and their applications", AFIPS 1968, in
+// the form whose merges start with a mirrored comparison).
+template <int K>
+__device__ inline void sort_regs(uint32_t (&a)[K]) {
+    lane_stages<K, 2>(a);
+    cross<K, kXor1, true>(a, 1u);  // blocks of 2 lanes
+    within<K, K / 2>(a);
+    cross<K, kMirror4, true>(a, 2u);  // of 4
+    cross<K, kXor1, false>(a, 1u);
+    within<K, K / 2>(a);
+    cross<K, kMirror8, true>(a, 4u);  // of 8
+    cross<K, kXor2, false>(a, 2u);
+    cross<K, kXor1, false>(a, 1u);
+    within<K, K / 2>(a);
+    cross<K, kMirror16, true>(a, 8u);  // of 16
+    cross4<K>(a);
+    cross<K, kXor2, false>(a, 2u);
+    cross<K, kXor1, false>(a, 1u);
+    within<K, K / 2>(a);
+}
+
+// K consecutive entries at any 4-byte address as one store of up to 16 bytes each.
+struct __attribute__((packed, aligned(4))) Four {
+    uint32_t v[4];
+};
+
+template <int K>
+__device__ inline void sort_row(uint32_t* __restrict__ row, uint32_t m) {
+    const uint32_t lane = threadIdx.x % kRowLanes;
+    uint32_t a[K];
+    // striped loads (the order before the sort does not matter); places past the row's
+    // end hold the largest value and stay behind every entry
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        const uint32_t at = r * kRowLanes + lane;
+        a[r] = at < m ? row[at] : 0xffffffffu;
+    }
+    sort_regs<K>(a);
+    const uint32_t first = lane * K;
+#pragma unroll
+    for (int r = 0; r < K; r += 4) {
+        if (K >= 4 && first + r + 4 <= m) {
+            *reinterpret_cast<Four*>(row + first + r) = Four{{a[r], a[r + 1], a[r + 2], a[r + 3]}};
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4 && r + u < K; ++u)
+                if (first + r + u < m) row[first + r + u] = a[r + u];
+        }
+    }
+}
+
+// The same sort over v[0, m) by the whole workgroup, for memory that its threads share
+// (LDS or the row itself); a comparison with a place at or past m never exchanges.
+__device__ inline void block_sort(uint32_t* v, uint32_t m) {
+    uint32_t top = 2;
+    while (top < m) top <<= 1;  // m <= 2^31
+    for (uint32_t s = 2; s != 0 && s <= top; s <<= 1)
+        for (uint32_t d = s >> 1; d > 0; d >>= 1) {
+            for (uint32_t c = threadIdx.x; c < (top >> 1); c += kSortThreads) {
+                const uint32_t in = c & (d - 1u), lo = ((c - in) << 1) + in;
+                const uint32_t hi = d == (s >> 1) ? ((c - in) << 1) + (s - 1u) - in : lo + d;
+                if (hi < m) {
+                    const uint32_t x = v[lo], y = v[hi];
+                    if (x > y) {
+                        v[lo] = y;
+                        v[hi] = x;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+}
+
+// Sixteen lanes take a row of up to 256 entries into registers (the wave's four rows by
+// the longest of them), sort it with lane exchanges that need no LDS, and store it; a
+// longer row is sorted by the whole workgroup in LDS, or, above 4096 entries, where it
+// lies.  Bound by the list's bytes, read and written once: 500,009 rows of 72 entries (36M,
+// 290 MB moved) in 108 us, 2.7 TB/s.  As one thread's insertion sort in global memory, at
+// the end of the kernel that lists the partners, that kernel took 7172 us, and 479 us
+// without it.
+__global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long long* __restrict__ rows, uint32_t n,
+                                                            uint32_t* __restrict__ cols) {
+    __shared__ uint32_t stage[kLdsRow];
+    const uint32_t first = blockIdx.x * kBlockRows;
+    const uint32_t i = first + threadIdx.x / kRowLanes;
+    unsigned long long r0 = 0, len = 0;
+    if (i < n) {
+        r0 = rows[i];
+        len = rows[i + 1] - r0;
+    }
+    const bool fits = len <= kRegRow;
+    const uint32_t m = fits ? (uint32_t)len : 0u;
+    uint32_t* const row = cols + r0;
+    if (__any(m > 128u)) sort_row<16>(row, m);
+    else if (__any(m > 64u)) sort_row<8>(row, m);
+    else if (__any(m > 32u)) sort_row<4>(row, m);
+    else if (__any(m > 1u)) sort_row<2>(row, m);
+    if (!__syncthreads_or(!fits)) return;
+    for (uint32_t q = first; q < first + kBlockRows && q < n; ++q) {
+        const unsigned long long s0 = rows[q], sl = rows[q + 1] - s0;
+        if (sl <= kRegRow) continue;  // the same for every thread of the workgroup
+        if (sl <= kLdsRow) {
+            for (uint32_t t = threadIdx.x; t < sl; t += kSortThreads) stage[t] = cols[s0 + t];
+            __syncthreads();
+            block_sort(stage, (uint32_t)sl);
+            for (uint32_t t = threadIdx.x; t < sl; t += kSortThreads) cols[s0 + t] = stage[t];
+            __syncthreads();
+        } else {
+            // in place: __syncthreads orders the workgroup's own global accesses
+            block_sort(cols + s0, (uint32_t)sl);
+        }
+    }
+}
+
+}  // namespace
+
+void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {
+    if (n > 0) hipLaunchKernelGGL(k_sort_rows, dim3(div_up(n, kBlockRows)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols);
+}
+
+}  // namespace lj

@@ -434,3 +434,30 @@ def test_c3_precision_subsample(engine):
     # size-independent invariants: ordered pairs come in (i,j),(j,i) couples
     assert int(res["n_pairs"]) % 2 == 0
     assert int(res["n_pairs"]) == pytest.approx(70.3 * n, rel=0.02)
+
+
+ROW_LENGTHS = [0, 1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 4096, 4097]
+
+
+@pytest.mark.parametrize("lbvh", [False, True])
+def test_pair_rows_of_every_length_class(engine, lbvh):
+    """Groups of m + 1 particles within the cutoff of each other and of nobody else give
+    rows of m partners: lengths on both sides of every size class of the row sort (16
+    lanes of 2, 4, 8 and 16 registers, LDS, in place), in shuffled order.  A row is the
+    other members of its group in ascending order."""
+    rng = np.random.default_rng(5)
+    rc, step = 0.01, 0.05
+    group = np.concatenate([np.full(m + 1, g) for g, m in enumerate(ROW_LENGTHS)])
+    rng.shuffle(group)
+    n = group.size
+    at = np.stack([group % 19, group // 19, np.zeros_like(group)], 1) * step + 0.02
+    x, y, z = ((at + rng.uniform(0, 0.5 * rc, (n, 3))).astype(np.float32)).T
+    d = engine.to_device(x, y, z)
+    rows, cols = engine.pairs(*d, ljamd.make_params(rc), lbvh=lbvh)
+    rows, cols = rows.cpu().numpy(), cols.cpu().numpy()
+    assert np.array_equal(np.diff(rows), np.array(ROW_LENGTHS)[group])
+    members = [np.flatnonzero(group == g) for g in range(len(ROW_LENGTHS))]
+    for i in range(n):
+        row = cols[rows[i] : rows[i + 1]]
+        want = members[group[i]]
+        assert np.array_equal(row, want[want != i]), (i, ROW_LENGTHS[group[i]])
