@@ -13,6 +13,8 @@
 // itself is stencil_pairs in lj_stencil.h).
 #include <cmath>
 
+#include "lj_rows.h"
+#include "lj_sort.h"
 #include "lj_stencil.h"
 
 namespace lj {
@@ -134,60 +136,202 @@ __global__ __launch_bounds__(256) void k_finalize(const double* __restrict__ par
 }
 
 // ------------------------------------------------------------------ pair lists
-// Pass 1: number of accepted partners of each particle, stored by original index (a
-// partner with a multiplicity above one is listed once).
-template <int PRED>
-__global__ __launch_bounds__(256) void k_pair_count(const float4* __restrict__ pos, const uint32_t* __restrict__ cell_of,
-                                                    const uint32_t* __restrict__ off, uint32_t n, GridGeom g,
-                                                    PairConst c, uint32_t* __restrict__ rowcnt) {
-    const uint32_t k = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const float4 pi = pos[k];
-    int32_t cx, cy, cz;
-    cell_coords(g, cell_of[k], cx, cy, cz);
-    const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx < g.g[0] - 1 ? cx + 1 : g.g[0] - 1;
-    uint32_t cnt = 0;
-    for (int32_t zz = cz - 1; zz <= cz + 1; ++zz) {
-        if (zz < 0 || zz >= g.g[2]) continue;
-        for (int32_t yy = cy - 1; yy <= cy + 1; ++yy) {
-            if (yy < 0 || yy >= g.g[1]) continue;
-            const uint32_t row = (uint32_t)((zz * g.g[1] + yy) * g.g[0]);
-            for (uint32_t t = off[row + x0]; t < off[row + x1 + 1]; ++t) {
-                const float4 pj = pos[t];
-                const float d2 = dist2(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
-                if (t != k && pair_mult<PRED>(c, pi, pj, d2) > 0) ++cnt;
-            }
+// Sixteen lanes take a row of up to 256 entries into registers (the wave's four rows by
+// the longest of them), sort it with lane exchanges that need no LDS, and store it; a
+// longer row is sorted by the whole workgroup in LDS, or, above 4096 entries, where it
+// lies.  Bound by the list's bytes, read and written once: 500,009 rows of 72 entries (36M,
+// 290 MB moved) in 108 us, 2.7 TB/s.  As one thread's insertion sort in global memory, at
+// the end of the kernel that lists the partners, that kernel took 7172 us, and 479 us
+// without it.  LONG: the rows of up to kRegRow entries are sorted already, so a thread looks
+// at one row's length (with 16 lanes a row that took 15 us on those 500,009 rows).
+template <bool LONG>
+__global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long long* __restrict__ rows, uint32_t n,
+                                                            uint32_t* __restrict__ cols) {
+    constexpr uint32_t kBlock = LONG ? kSortThreads : kBlockRows;  // rows of a workgroup
+    __shared__ uint32_t stage[kLdsRow];
+    const uint32_t first = blockIdx.x * kBlock;
+    const uint32_t i = first + (LONG ? threadIdx.x : threadIdx.x / kRowLanes);
+    unsigned long long r0 = 0, len = 0;
+    if (i < n) {
+        r0 = rows[i];
+        len = rows[i + 1] - r0;
+    }
+    const bool fits = len <= kRegRow;
+    if constexpr (!LONG) sort_four_rows(cols + r0, cols + r0, fits ? (uint32_t)len : 0u);
+    if (!__syncthreads_or(!fits)) return;
+    for (uint32_t q = first; q < first + kBlock && q < n; ++q) {
+        const unsigned long long s0 = rows[q], sl = rows[q + 1] - s0;
+        if (sl <= kRegRow) continue;  // the same for every thread of the workgroup
+        if (sl <= kLdsRow) {
+            for (uint32_t t = threadIdx.x; t < sl; t += kSortThreads) stage[t] = cols[s0 + t];
+            __syncthreads();
+            block_sort(stage, (uint32_t)sl);
+            for (uint32_t t = threadIdx.x; t < sl; t += kSortThreads) cols[s0 + t] = stage[t];
+            __syncthreads();
+        } else {
+            // in place: __syncthreads orders the workgroup's own global accesses
+            block_sort(cols + s0, (uint32_t)sl);
         }
     }
-    rowcnt[__float_as_uint(pi.w)] = cnt;
 }
 
-// Pass 2: the partners' original indices in walk order (sort_rows then orders each row).
-template <int PRED>
-__global__ __launch_bounds__(256) void k_pair_fill(const float4* __restrict__ pos, const uint32_t* __restrict__ cell_of,
-                                                   const uint32_t* __restrict__ off, uint32_t n, GridGeom g,
-                                                   PairConst c, const unsigned long long* __restrict__ rows,
-                                                   uint32_t* __restrict__ cols) {
-    const uint32_t k = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const float4 pi = pos[k];
-    const uint32_t i = __float_as_uint(pi.w);
-    int32_t cx, cy, cz;
-    cell_coords(g, cell_of[k], cx, cy, cz);
-    const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx < g.g[0] - 1 ? cx + 1 : g.g[0] - 1;
-    unsigned long long w = rows[i];
-    for (int32_t zz = cz - 1; zz <= cz + 1; ++zz) {
-        if (zz < 0 || zz >= g.g[2]) continue;
-        for (int32_t yy = cy - 1; yy <= cy + 1; ++yy) {
-            if (yy < 0 || yy >= g.g[1]) continue;
-            const uint32_t row = (uint32_t)((zz * g.g[1] + yy) * g.g[0]);
-            for (uint32_t t = off[row + x0]; t < off[row + x1 + 1]; ++t) {
-                const float4 pj = pos[t];
-                const float d2 = dist2(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
-                if (t != k && pair_mult<PRED>(c, pi, pj, d2) > 0) cols[w++] = __float_as_uint(pj.w);
+// Partners from the rc grid.  A wave takes kPairSlots consecutive sorted slots; the ones
+// in one cell (a run) share the 27 cells' particles, whose slots are nine ranges, taken
+// as one sequence: the lanes hold up to kPairBatches x 64 of them in registers and test
+// each of the run's particles, wave-uniform, against all of them, so that a partner is
+// loaded once per run, a ballot is the answer for 64 candidates, and no lane waits for
+// another's longer walk.  FILL = false counts (a partner with a multiplicity above one
+// is listed once): rowcnt[original index].  FILL = true lists: four particles at a time
+// collect their partners' indices in LDS, and 16 lanes each sort them in registers and
+// store them; rows above kRegRow entries are stored unsorted (sort_long_rows follows).
+// Bound by VALU issue: 500,009 particles, 465 candidates and 72 partners each: count 92 us,
+// list 287 us (one thread per particle: 159 and 479 us, and 108 us more for the sort).
+constexpr int kPairThreads = 256;
+constexpr int kPairSlots = 16;
+constexpr int kPairBatches = 8;
+constexpr uint32_t kNoSlot = 0xffffffffu;
+constexpr uint32_t kPairChunk = kPairBatches * kWaveSize;
+// entries between the four lists of a wave: a row and 16 more, so that the four groups of
+// 16 lanes read different banks
+constexpr int kListStride = (int)kRegRow + kRowLanes;
+
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int PRED, bool FILL>
+__global__ __launch_bounds__(kPairThreads) void k_pairs(const float4* __restrict__ pos,
+                                                        const uint32_t* __restrict__ cell_of,
+                                                        const uint32_t* __restrict__ off, uint32_t n, GridGeom g,
+                                                        PairConst c, uint32_t* __restrict__ rowcnt,
+                                                        const unsigned long long* __restrict__ rows,
+                                                        uint32_t* __restrict__ cols) {
+    constexpr int kWaves = kPairThreads / kWaveSize;
+    // every predicate but the two distance ones can accept the particle itself
+    constexpr bool kSelf = PRED != LJ_PRED_AABB && PRED != LJ_PRED_CUSTOM;
+    __shared__ uint32_t lists[FILL ? kWaves : 1][FILL ? 4 * kListStride : 1];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const unsigned lane = __lane_id();
+    const uint32_t first = (xcd_block(blockIdx.x, gridDim.x) * kWaves + wave) * kPairSlots;
+    if (first >= n) return;  // the whole wave (no workgroup barrier below)
+    const uint32_t cnt = n - first < (uint32_t)kPairSlots ? n - first : (uint32_t)kPairSlots;
+    const uint32_t key = cell_of[first + (lane < cnt ? lane : cnt - 1u)];
+    uint32_t found = 0;  // lane q: partners of slot first + q
+    for (uint32_t j0 = 0; j0 < cnt;) {
+        // the run: slots j0 .. j1 - 1, one cell (the keys are sorted)
+        const uint32_t ck = __builtin_amdgcn_readlane(key, j0);
+        const uint32_t j1 = 64u - (uint32_t)__builtin_clzll(__ballot(lane < cnt && key == ck));
+        // its nine ranges of slots, one per lane; lanes 9 .. 63 hold empty ones
+        uint32_t b = 0, len = 0;
+        {
+            int32_t cx, cy, cz;
+            cell_coords(g, ck, cx, cy, cz);
+            const int32_t zz = cz + (int32_t)(lane / 3u) - 1, yy = cy + (int32_t)(lane % 3u) - 1;
+            if (lane < 9u && zz >= 0 && zz < g.g[2] && yy >= 0 && yy < g.g[1]) {
+                const uint32_t row = (uint32_t)((zz * g.g[1] + yy) * g.g[0]);
+                const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx < g.g[0] - 1 ? cx + 1 : g.g[0] - 1;
+                b = off[row + x0];
+                len = off[row + x1 + 1] - b;
             }
         }
+        // candidate t lies in range r at slot t + shift[r], r the last one with start[r] <= t
+        uint32_t start[9], shift[9], total = 0;
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            start[r] = total;
+            shift[r] = __builtin_amdgcn_readlane(b, r) - total;
+            total += __builtin_amdgcn_readlane(len, r);
+        }
+        float4 pj[kPairBatches];
+        uint32_t slot[kPairBatches];
+        // candidates base .. base + kPairChunk - 1 (fewer at the end) into the registers
+        auto load = [&](uint32_t base) {
+#pragma unroll
+            for (int u = 0; u < kPairBatches; ++u) {
+                if (base + u * kWaveSize >= total) break;
+                const uint32_t t = base + u * kWaveSize + lane;
+                const uint32_t tc = t < total ? t : total - 1u;
+                uint32_t s = tc + shift[0];
+#pragma unroll
+                for (int r = 1; r < 9; ++r) s = tc >= start[r] ? tc + shift[r] : s;
+                pj[u] = pos[s];
+                slot[u] = s;
+                // past the end: no predicate with a distance accepts a NaN
+                if (t >= total) {
+                    pj[u].x = __builtin_nanf("");
+                    slot[u] = kNoSlot;
+                }
+            }
+        };
+        // is this lane's candidate of batch u a partner of slot k (position pi)?
+        auto partner = [&](int u, uint32_t k, const float4& pi) {
+            const float d2 = dist2(pj[u].x - pi.x, pj[u].y - pi.y, pj[u].z - pi.z);
+            bool in = pair_mult<PRED>(c, pi, pj[u], d2) > 0;
+            if constexpr (kSelf) in = in && slot[u] != k && slot[u] != kNoSlot;
+            return in;
+        };
+        if constexpr (!FILL) {
+            for (uint32_t base = 0; base < total; base += kPairChunk) {
+                load(base);
+                for (uint32_t j = j0; j < j1; ++j) {
+                    const float4 pi = pos[first + j];
+                    uint32_t m = 0;
+#pragma unroll
+                    for (int u = 0; u < kPairBatches; ++u) {
+                        if (base + u * kWaveSize >= total) break;
+                        m += (uint32_t)__popcll(__ballot(partner(u, first + j, pi)));
+                    }
+                    found += lane == j ? m : 0u;
+                }
+            }
+        } else {
+            uint32_t* const list = lists[wave];
+            for (uint32_t jq = j0; jq < j1; jq += 4) {
+                unsigned long long r0[4];
+                uint32_t len4[4], at[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t j = jq + q < j1 ? jq + q : j1 - 1u;
+                    const uint32_t i = __float_as_uint(pos[first + j].w);
+                    r0[q] = rows[i];
+                    len4[q] = (uint32_t)(rows[i + 1] - r0[q]);
+                    at[q] = 0;
+                }
+                for (uint32_t base = 0; base < total; base += kPairChunk) {
+                    if (jq == j0 || total > kPairChunk) load(base);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        if (jq + q >= j1) break;
+                        const float4 pi = pos[first + jq + q];
+#pragma unroll
+                        for (int u = 0; u < kPairBatches; ++u) {
+                            if (base + u * kWaveSize >= total) break;
+                            const bool in = partner(u, first + jq + q, pi);
+                            const uint64_t m = __ballot(in);
+                            if (in) {
+                                const uint32_t w = at[q] + sortk::rank_below(m);
+                                const uint32_t v = __float_as_uint(pj[u].w);
+                                if (len4[q] <= kRegRow) list[q * kListStride + w] = v;
+                                else cols[r0[q] + w] = v;
+                            }
+                            at[q] += (uint32_t)__popcll(m);
+                        }
+                    }
+                }
+                wave_lds_sync();
+                const uint32_t q = lane / kRowLanes;
+                const unsigned long long rq = q == 0 ? r0[0] : q == 1 ? r0[1] : q == 2 ? r0[2] : r0[3];
+                uint32_t mq = q == 0 ? len4[0] : q == 1 ? len4[1] : q == 2 ? len4[2] : len4[3];
+                if (jq + q >= j1 || mq > kRegRow) mq = 0;
+                sort_four_rows(list + q * kListStride, cols + rq, mq);
+                wave_lds_sync();
+            }
+        }
+        j0 = j1;
     }
+    if (!FILL && lane < cnt) rowcnt[__float_as_uint(pos[first + lane].w)] = found;
 }
 
 __global__ __launch_bounds__(256) void k_unpack(const float4* __restrict__ pos, uint32_t n, float* __restrict__ xo,
@@ -399,11 +543,21 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
     return LJ_OK;
 }
 
-int pairs_cellgrid(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n, const lj_params* p,
-                   const GridGeom& g, const PairConst& c, unsigned long long* rows, uint32_t* cols,
-                   unsigned long long capacity, unsigned long long* needed, hipStream_t s) {
+static void sort_long_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {
+    if (n > 0)
+        hipLaunchKernelGGL(k_sort_rows<true>, dim3(div_up(n, kSortThreads)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols);
+}
+
+void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {
+    if (n > 0)
+        hipLaunchKernelGGL(k_sort_rows<false>, dim3(div_up(n, kBlockRows)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols);
+}
+
+static int pairs_cellgrid(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n,
+                          const GridGeom& g, const PairConst& c, unsigned long long* rows, uint32_t* cols,
+                          unsigned long long capacity, unsigned long long* needed, int predicate, hipStream_t s) {
     LJ_TRY(bin_particles(ctx, x, y, z, n, g, s));
-    const unsigned nb = div_up(n > 0 ? n : 1, 256);
+    const unsigned nb = div_up(n > 0 ? n : 1, (kPairThreads / kWaveSize) * kPairSlots);
     const float4* pos = ctx->bin.pos.as<float4>();
     const uint32_t* cell_of = ctx->bin.sorted_keys();
     const uint32_t* off = ctx->bin.offsets.as<uint32_t>();
@@ -411,11 +565,20 @@ int pairs_cellgrid(lj_context* ctx, const float* x, const float* y, const float*
     // row counts (u32, by original index) -> u64 offsets
     LJ_HIP(ctx, ctx->bin.rows.grow(((size_t)n + 1) * sizeof(uint32_t)));
     uint32_t* rowcnt = ctx->bin.rows.as<uint32_t>();
-    switch (p->predicate) {
-#define LJ_COUNT(P) case P: hipLaunchKernelGGL(k_pair_count<P>, dim3(nb), dim3(256), 0, s, pos, cell_of, off, nn, g, c, rowcnt); break;
-        LJ_COUNT(LJ_PRED_AABB) LJ_COUNT(LJ_PRED_CUSTOM) LJ_COUNT(LJ_PRED_CUDALJ) LJ_COUNT(LJ_PRED_SPHERE) LJ_COUNT(LJ_PRED_TRIANGLE)
-#undef LJ_COUNT
+#define LJ_PAIRS(P, FILL)                                                                                          \
+    case P:                                                                                                        \
+        hipLaunchKernelGGL((k_pairs<P, FILL>), dim3(nb), dim3(kPairThreads), 0, s, pos, cell_of, off, nn, g, c, rowcnt, \
+                           (const unsigned long long*)rows, cols);                                                 \
+        break;
+#define LJ_PAIRS_ALL(FILL)                                                                             \
+    switch (predicate) {                                                                               \
+        LJ_PAIRS(LJ_PRED_AABB, FILL)                                                                   \
+        LJ_PAIRS(LJ_PRED_CUSTOM, FILL)                                                                 \
+        LJ_PAIRS(LJ_PRED_CUDALJ, FILL)                                                                 \
+        LJ_PAIRS(LJ_PRED_SPHERE, FILL)                                                                 \
+        LJ_PAIRS(LJ_PRED_TRIANGLE, FILL)                                                               \
     }
+    LJ_PAIRS_ALL(false)
     LJ_TRY(scan_u32_to_u64(ctx, rowcnt, rows, n, s));
     unsigned long long total = 0;
     LJ_HIP(ctx, hipMemcpyAsync(&total, rows + n, sizeof total, hipMemcpyDeviceToHost, s));
@@ -424,12 +587,10 @@ int pairs_cellgrid(lj_context* ctx, const float* x, const float* y, const float*
     if (total > capacity)
         return fail(ctx, LJ_ERR_CAPACITY, "pair list needs %llu entries, capacity is %llu", total, capacity);
     if (total == 0) return LJ_OK;
-    switch (p->predicate) {
-#define LJ_FILL(P) case P: hipLaunchKernelGGL(k_pair_fill<P>, dim3(nb), dim3(256), 0, s, pos, cell_of, off, nn, g, c, (const unsigned long long*)rows, cols); break;
-        LJ_FILL(LJ_PRED_AABB) LJ_FILL(LJ_PRED_CUSTOM) LJ_FILL(LJ_PRED_CUDALJ) LJ_FILL(LJ_PRED_SPHERE) LJ_FILL(LJ_PRED_TRIANGLE)
-#undef LJ_FILL
-    }
-    sort_rows(rows, n, cols, s);
+    LJ_PAIRS_ALL(true)
+#undef LJ_PAIRS_ALL
+#undef LJ_PAIRS
+    sort_long_rows(rows, n, cols, s);  // the rows that k_pairs left unsorted
     LJ_HIP(ctx, hipGetLastError());
     return LJ_OK;
 }
@@ -488,7 +649,7 @@ int lj_pairs(lj_context* ctx, const float* x, const float* y, const float* z, in
     if (!row_offsets || (n > 0 && (!x || !y || !z)) || (capacity > 0 && !cols))
         return fail(ctx, LJ_ERR_INVALID_ARG, "NULL pointer argument");
     LJ_HIP(ctx, hipSetDevice(ctx->device));
-    return pairs_cellgrid(ctx, x, y, z, n, p, g, c, row_offsets, cols, capacity, needed, (hipStream_t)stream);
+    return pairs_cellgrid(ctx, x, y, z, n, g, c, row_offsets, cols, capacity, needed, p->predicate, (hipStream_t)stream);
 }
 
 int lj_reorder(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n, const lj_params* p,

@@ -195,7 +195,7 @@ int scan_u32(lj_context* ctx, const uint32_t* in, uint32_t* out, int64_t n, uint
 int scan_u32_to_u64(lj_context* ctx, const uint32_t* in, unsigned long long* out, int64_t n, hipStream_t s);
 
 // Sorts every row of a CSR list, cols[rows[i] .. rows[i + 1]) for i < n, ascending and
-// in place (rows.hip).
+// in place (force.hip).
 void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s);
 
 // Cell-grid pipelines (force.hip).

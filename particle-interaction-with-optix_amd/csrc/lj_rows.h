@@ -1,14 +1,15 @@
-// rows.hip -- sorting the rows of a CSR neighbour list in place.
+// lj_rows.h -- sorting the rows of a CSR neighbour list: 16 lanes a row in registers, or a
+// workgroup a row in the memory that holds it.
 //
-// The list calls append each particle's partners in walk order (cells, or the tree's
+// The list calls find each particle's partners in walk order (cells, or the tree's
 // leaves) and promise rows in ascending index order.  The reference has no lists; its
 // OptiX programs visit a particle's partners in the order the hardware reports them
 // (SDK/optixMultiSphereAABB/optixLJ.cu:134-176).
+#pragma once
+
 #include "lj_internal.h"
 
 namespace lj {
-
-namespace {
 
 constexpr int kSortThreads = 256;
 constexpr int kRowLanes = 16;                                // lanes of a row: one DPP row
@@ -110,8 +111,9 @@ struct __attribute__((packed, aligned(4))) Four {
     uint32_t v[4];
 };
 
+// Sorts from[0, m) (the row itself or a copy in LDS) into row[0, m), m <= 16 K.
 template <int K>
-__device__ inline void sort_row(uint32_t* __restrict__ row, uint32_t m) {
+__device__ inline void sort_row(const uint32_t* from, uint32_t* row, uint32_t m) {
     const uint32_t lane = threadIdx.x % kRowLanes;
     uint32_t a[K];
     // striped loads (the order before the sort does not matter); places past the row's
@@ -119,7 +121,7 @@ __device__ inline void sort_row(uint32_t* __restrict__ row, uint32_t m) {
 #pragma unroll
     for (int r = 0; r < K; ++r) {
         const uint32_t at = r * kRowLanes + lane;
-        a[r] = at < m ? row[at] : 0xffffffffu;
+        a[r] = at < m ? from[at] : 0xffffffffu;
     }
     sort_regs<K>(a);
     const uint32_t first = lane * K;
@@ -133,6 +135,14 @@ __device__ inline void sort_row(uint32_t* __restrict__ row, uint32_t m) {
                 if (first + r + u < m) row[first + r + u] = a[r + u];
         }
     }
+}
+
+// The wave's four rows (one per 16 lanes, m <= kRegRow) by the longest of them.
+__device__ inline void sort_four_rows(const uint32_t* from, uint32_t* row, uint32_t m) {
+    if (__any(m > 128u)) sort_row<16>(from, row, m);
+    else if (__any(m > 64u)) sort_row<8>(from, row, m);
+    else if (__any(m > 32u)) sort_row<4>(from, row, m);
+    else if (__any(m > 0u)) sort_row<2>(from, row, m);
 }
 
 // The same sort over v[0, m) by the whole workgroup, for memory that its threads share
@@ -155,53 +165,6 @@ __device__ inline void block_sort(uint32_t* v, uint32_t m) {
             }
             __syncthreads();
         }
-}
-
-// Sixteen lanes take a row of up to 256 entries into registers (the wave's four rows by
-// the longest of them), sort it with lane exchanges that need no LDS, and store it; a
-// longer row is sorted by the whole workgroup in LDS, or, above 4096 entries, where it
-// lies.  Bound by the list's bytes, read and written once: 500,009 rows of 72 entries (36M,
-// 290 MB moved) in 108 us, 2.7 TB/s.  As one thread's insertion sort in global memory, at
-// the end of the kernel that lists the partners, that kernel took 7172 us, and 479 us
-// without it.
-__global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long long* __restrict__ rows, uint32_t n,
-                                                            uint32_t* __restrict__ cols) {
-    __shared__ uint32_t stage[kLdsRow];
-    const uint32_t first = blockIdx.x * kBlockRows;
-    const uint32_t i = first + threadIdx.x / kRowLanes;
-    unsigned long long r0 = 0, len = 0;
-    if (i < n) {
-        r0 = rows[i];
-        len = rows[i + 1] - r0;
-    }
-    const bool fits = len <= kRegRow;
-    const uint32_t m = fits ? (uint32_t)len : 0u;
-    uint32_t* const row = cols + r0;
-    if (__any(m > 128u)) sort_row<16>(row, m);
-    else if (__any(m > 64u)) sort_row<8>(row, m);
-    else if (__any(m > 32u)) sort_row<4>(row, m);
-    else if (__any(m > 1u)) sort_row<2>(row, m);
-    if (!__syncthreads_or(!fits)) return;
-    for (uint32_t q = first; q < first + kBlockRows && q < n; ++q) {
-        const unsigned long long s0 = rows[q], sl = rows[q + 1] - s0;
-        if (sl <= kRegRow) continue;  // the same for every thread of the workgroup
-        if (sl <= kLdsRow) {
-            for (uint32_t t = threadIdx.x; t < sl; t += kSortThreads) stage[t] = cols[s0 + t];
-            __syncthreads();
-            block_sort(stage, (uint32_t)sl);
-            for (uint32_t t = threadIdx.x; t < sl; t += kSortThreads) cols[s0 + t] = stage[t];
-            __syncthreads();
-        } else {
-            // in place: __syncthreads orders the workgroup's own global accesses
-            block_sort(cols + s0, (uint32_t)sl);
-        }
-    }
-}
-
-}  // namespace
-
-void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_sort_rows, dim3(div_up(n, kBlockRows)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols);
 }
 
 }  // namespace lj
