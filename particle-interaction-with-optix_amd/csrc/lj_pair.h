@@ -23,6 +23,8 @@ struct Acc<LJ_PREC_MIXED> {
     __device__ inline void add(double v) { s += v; }
     __device__ inline void fma(double a, double b) { s = __builtin_fma(a, b, s); }
     __device__ inline double value() const { return s; }
+    // adds the sum of the lane `d` away (both lanes then hold the two lanes' sum)
+    __device__ inline void merge_xor(int d) { s += __shfl_xor(s, d, kWaveSize); }
 };
 
 template <>
@@ -31,6 +33,7 @@ struct Acc<LJ_PREC_FP32> {
     __device__ inline void add(float v) { s += v; }
     __device__ inline void fma(float a, float b) { s = __builtin_fmaf(a, b, s); }
     __device__ inline float value() const { return s; }
+    __device__ inline void merge_xor(int d) { s += __shfl_xor(s, d, kWaveSize); }
 };
 
 template <>
@@ -44,6 +47,11 @@ struct Acc<LJ_PREC_FP32_COMP> {
     }
     __device__ inline void fma(float a, float b) { add(a * b); }
     __device__ inline float value() const { return s + c; }
+    __device__ inline void merge_xor(int d) {
+        const float os = __shfl_xor(s, d, kWaveSize), oc = __shfl_xor(c, d, kWaveSize);
+        add(os);
+        c += oc;
+    }
 };
 
 // FP64 reciprocal: hardware estimate plus one Newton-Raphson step.  Measured on
@@ -72,6 +80,16 @@ struct PairSums {
         px = pi.x;
         py = pi.y;
         pz = pi.z;
+    }
+    // Sums over groups of `lanes` neighbouring lanes (a power of two), left in each of them.
+    __device__ inline void merge(int lanes) {
+        for (int d = 1; d < lanes; d <<= 1) {
+            ax.merge_xor(d);
+            ay.merge_xor(d);
+            az.merge_xor(d);
+            ae.merge_xor(d);
+            if constexpr (VIR) av.merge_xor(d);
+        }
     }
     // Accepted partners of a cutoff predicate lie within rc of p_i on every axis.  If
     // |p_i| >= 2 rc on every axis (so p_j has the sign of p_i and lies in [p_i/2, 2 p_i]),

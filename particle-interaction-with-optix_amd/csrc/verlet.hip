@@ -14,48 +14,86 @@ namespace lj {
 
 namespace {
 
-// One thread per particle (row i of the CSR list, caller order).  Entries j >= n are
-// ignored.  Per-block FP64 energy/virial partials; the listed and accepted pair counts
-// go to res.
+// The positions as one 16-byte record each: the list's partners lie at random indices,
+// and one load then brings a partner's position where three arrays took three.
+__global__ __launch_bounds__(256) void k_pack_positions(const float* __restrict__ x, const float* __restrict__ y,
+                                                        const float* __restrict__ z, uint32_t n,
+                                                        float4* __restrict__ pos) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n) pos[i] = make_float4(x[i], y[i], z[i], 0.f);
+}
+
+// kListLanes lanes per particle (row i of the CSR list, caller order), each taking every
+// kListLanes-th entry, kListUnroll of them loaded at once; a workgroup takes `turns` times
+// kListRows rows, one set after the other.  Entries j >= n are ignored.  Per-block FP64
+// energy/virial partials; the listed and accepted pair counts go to res.
+// Bound by the partners' gathers, a line each: 500,009 particles at shuffled indices, 36M
+// entries, 366 us (12.6 TB/s of 128-byte lines from the caches).  One lane per row, whose
+// loads of the list touched 64 lines and whose three gathers per entry waited for each
+// other, took 1144 us.
+constexpr int kListLanes = 8;
+constexpr int kListUnroll = 4;
+constexpr int kListRows = 256 / kListLanes;
+
 template <int PRED, int PREC, bool VIR>
-__global__ __launch_bounds__(256) void k_list_force(const float* __restrict__ x, const float* __restrict__ y,
-                                                    const float* __restrict__ z, uint32_t n,
+__global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ pos, uint32_t n,
                                                     const unsigned long long* __restrict__ rows,
-                                                    const uint32_t* __restrict__ cols, PairConst c,
+                                                    const uint32_t* __restrict__ cols, PairConst c, uint32_t turns,
                                                     float* __restrict__ fx, float* __restrict__ fy,
                                                     float* __restrict__ fz, float* __restrict__ e,
                                                     double* __restrict__ partials, lj_result* __restrict__ res) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    PairSums<PREC, PRED == LJ_PRED_CUDALJ, VIR> acc;
+    const uint32_t sub = threadIdx.x % kListLanes;
     unsigned long long np = 0, listed = 0;
     double esum = 0.0, vsum = 0.0;
-    if (i < n) {
-        const float4 pi = make_float4(x[i], y[i], z[i], 0.f);
+    for (uint32_t turn = 0; turn < turns; ++turn) {
+        const uint32_t i = (blockIdx.x * turns + turn) * kListRows + threadIdx.x / kListLanes;
+        PairSums<PREC, PRED == LJ_PRED_CUDALJ, VIR> acc;
+        const bool active = i < n;
+        const float4 pi = active ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
         acc.set_i(pi);
-        acc.allow_exact_diff(c, pi, true);  // over the lanes with a particle
-        const unsigned long long r0 = rows[i], r1 = rows[i + 1];
-        for (unsigned long long q = r0; q < r1; ++q) {
-            const uint32_t j = cols[q];
-            if (j >= n) continue;
-            ++listed;
-            const float4 pj = make_float4(x[j], y[j], z[j], 0.f);
-            const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-            const float d2 = dist2(dx, dy, dz);
-            if constexpr (PRED == LJ_PRED_CUDALJ) {
-                if (j == i) continue;
-            }
-            const int mult = pair_mult<PRED>(c, pi, pj, d2);
-            if (!mult) continue;
-            np += (unsigned long long)mult;
-            acc.add(c, pj, dx, dy, dz, d2, mult);
+        acc.allow_exact_diff(c, pi, active);
+        unsigned long long q = 0, r1 = 0;
+        if (active) {
+            q = rows[i] + sub;
+            r1 = rows[i + 1];
         }
-        fx[i] = (float)(-c.e24 * (double)acc.ax.value());
-        fy[i] = (float)(-c.e24 * (double)acc.ay.value());
-        fz[i] = (float)(-c.e24 * (double)acc.az.value());
-        const double ei = c.e4 * (double)acc.ae.value();
-        if (e) e[i] = (float)ei;
-        esum = ei;
-        vsum = c.e24 * (double)acc.av.value();
+        for (; q < r1; q += kListLanes * kListUnroll) {
+            uint32_t j[kListUnroll];
+            float4 pj[kListUnroll];
+            // every load issued before any is used; a place past the row's end reads the
+            // lane's first entry again and is not counted
+#pragma unroll
+            for (int u = 0; u < kListUnroll; ++u) {
+                const unsigned long long at = q + u * kListLanes;
+                j[u] = cols[at < r1 ? at : q];
+            }
+#pragma unroll
+            for (int u = 0; u < kListUnroll; ++u) pj[u] = pos[j[u] < n ? j[u] : i];
+#pragma unroll
+            for (int u = 0; u < kListUnroll; ++u) {
+                if (q + u * kListLanes >= r1 || j[u] >= n) continue;
+                ++listed;
+                const float dx = pj[u].x - pi.x, dy = pj[u].y - pi.y, dz = pj[u].z - pi.z;
+                const float d2 = dist2(dx, dy, dz);
+                if constexpr (PRED == LJ_PRED_CUDALJ) {
+                    if (j[u] == i) continue;
+                }
+                const int mult = pair_mult<PRED>(c, pi, pj[u], d2);
+                if (!mult) continue;
+                np += (unsigned long long)mult;
+                acc.add(c, pj[u], dx, dy, dz, d2, mult);
+            }
+        }
+        acc.merge(kListLanes);
+        if (active && sub == 0) {
+            fx[i] = (float)(-c.e24 * (double)acc.ax.value());
+            fy[i] = (float)(-c.e24 * (double)acc.ay.value());
+            fz[i] = (float)(-c.e24 * (double)acc.az.value());
+            const double ei = c.e4 * (double)acc.ae.value();
+            if (e) e[i] = (float)ei;
+            esum += ei;
+            vsum += c.e24 * (double)acc.av.value();
+        }
     }
     block_sum2(esum, vsum);
     const unsigned long long bp = block_sum_u64(np);
@@ -68,21 +106,30 @@ __global__ __launch_bounds__(256) void k_list_force(const float* __restrict__ x,
     }
 }
 
-// Largest |p - p0|^2 (FP32, a non-negative float: its bits order like the value).
+// Largest |p - p0|^2 (FP32, a non-negative float: its bits order like the value).  At
+// most kDispBlocks workgroups, one atomic each: with one per wave, 500,009 particles sent
+// 7,800 atomics to the one counter and took 91 us.
+constexpr unsigned kDispBlocks = 512;
+
 __global__ __launch_bounds__(256) void k_max_disp(const float* __restrict__ x, const float* __restrict__ y,
                                                   const float* __restrict__ z, const float* __restrict__ x0,
                                                   const float* __restrict__ y0, const float* __restrict__ z0, uint32_t n,
                                                   unsigned int* __restrict__ max2) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ float wmax[256 / kWaveSize];
     float m = 0.f;
-    if (i < n) {
+    for (uint64_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) {
         const float dx = x[i] - x0[i], dy = y[i] - y0[i], dz = z[i] - z0[i];
-        m = dist2(dx, dy, dz);
-        if (!(m >= 0.f)) m = INFINITY;  // a NaN displacement forces a rebuild
+        const float d2 = dist2(dx, dy, dz);
+        m = fmaxf(m, d2 >= 0.f ? d2 : INFINITY);  // a NaN displacement forces a rebuild
     }
 #pragma unroll
     for (int d = kWaveSize / 2; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, kWaveSize));
-    if (__lane_id() == 0 && m > 0.f) atomicMax(max2, __float_as_uint(m));
+    if (__lane_id() == 0) wmax[threadIdx.x / kWaveSize] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 256 / kWaveSize; ++w) m = fmaxf(m, wmax[w]);
+        if (m > 0.f) atomicMax(max2, __float_as_uint(m));
+    }
 }
 
 __global__ void k_zero_u32(unsigned int* p) { *p = 0u; }
@@ -113,14 +160,20 @@ int lj_compute_list(lj_context* ctx, const float* x, const float* y, const float
     }
     PhaseTimer tf(ctx, LJ_PHASE_FORCE, s);
     fill_u64(&res->n_candidates, 2, 0ull, s);
-    const unsigned nb = div_up(n > 0 ? n : 1, 256);
+    // up to 8 sets of rows per workgroup once there are workgroups for every CU
+    const int64_t sets = div_up(n > 0 ? n : 1, kListRows);
+    const uint32_t turns = (uint32_t)(sets < 2048 ? 1 : sets < 16384 ? sets / 2048 : 8);
+    const unsigned nb = div_up(sets, turns);
+    LJ_HIP(ctx, ctx->bin.pos.grow(((size_t)(n > 0 ? n : 1) + kPosSpare) * sizeof(float4)));
+    float4* pos = ctx->bin.pos.as<float4>();
+    if (n > 0) hipLaunchKernelGGL(k_pack_positions, dim3(div_up(n, 256)), dim3(256), 0, s, x, y, z, (uint32_t)n, pos);
     LJ_HIP(ctx, ctx->bin.partials.grow(((size_t)nb + nb / 1024 + 1) * 2 * sizeof(double)));
     double* partials = ctx->bin.partials.as<double>();
     const bool vir = !(p->flags & LJ_FLAG_NO_VIRIAL);
     const uint32_t nn = (uint32_t)n;
 #define LJ_LF(PRED, PREC, VIR)                                                                                    \
-    hipLaunchKernelGGL((k_list_force<PRED, PREC, VIR>), dim3(nb), dim3(256), 0, s, x, y, z, nn, row_offsets, cols, c, \
-                       fx, fy, fz, e, partials, res)
+    hipLaunchKernelGGL((k_list_force<PRED, PREC, VIR>), dim3(nb), dim3(256), 0, s, (const float4*)pos, nn, row_offsets, \
+                       cols, c, turns, fx, fy, fz, e, partials, res)
 #define LJ_LF_V(PRED, PREC)            \
     do {                               \
         if (vir) LJ_LF(PRED, PREC, true); \
@@ -159,7 +212,8 @@ int lj_max_displacement(lj_context* ctx, const float* x, const float* y, const f
     // a fill kernel, not hipMemsetAsync: the call may be captured in a graph
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, m);
     if (n > 0)
-        hipLaunchKernelGGL(k_max_disp, dim3(div_up(n, 256)), dim3(256), 0, s, x, y, z, x0, y0, z0, (uint32_t)n, m);
+        hipLaunchKernelGGL(k_max_disp, dim3(n > (int64_t)kDispBlocks * 256 ? kDispBlocks : div_up(n, 256)), dim3(256), 0, s,
+                           x, y, z, x0, y0, z0, (uint32_t)n, m);
     LJ_HIP(ctx, hipGetLastError());
     return LJ_OK;
 }

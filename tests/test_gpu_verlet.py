@@ -134,3 +134,61 @@ def test_velocity_verlet_with_list_reuse(engine):
     # over the first steps, before the relaxing crystal brings pairs across rc, the
     # integrator conserves the energy
     assert np.max(np.abs(e_list[:5] - e_list[0])) <= 1e-7 * abs(e_list[0])
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp32", "fp32_comp"])
+@pytest.mark.parametrize("n,m", [(1, 0), (33, 1), (64, 7), (65, 8), (257, 9), (1000, 31), (1001, 32), (4097, 33), (70001, 5)])
+def test_list_rows_of_every_length(engine, n, m, prec):
+    """Rows of m entries on both sides of the eight lanes and the four entries a lane loads
+    at once, workgroups of one and of several sets of rows, entries past n ignored: the
+    sums over the list in 64 bits.  In 32 bits s^6 is within 15 roundings (five each in r^2
+    and in sigma^2 / r^2, cubed) of its value, so a term s^6 (2 s^6 - 1), a difference of
+    two parts, is within 32 of 2^-24 of their sum, and 33 terms add as much at most again:
+    2^-18 of the parts' sum."""
+    rng = np.random.default_rng(n + m)
+    x, y, z = (rng.uniform(0, 1, n).astype(np.float32) for _ in range(3))
+    cols = rng.integers(0, n, (n, m)).astype(np.int64)
+    if m > 1:
+        cols[:, m // 2] = n + 5  # out of range: ignored
+    rows = np.arange(n + 1, dtype=np.int64) * m
+    p = ljamd.make_params(0.6, sigma=0.05, precision=prec)
+    d = engine.to_device(x, y, z)
+    pad = np.append(cols.reshape(-1), 0).astype(np.int32)
+    out = engine.compute_list(*d, p, *engine.to_device(rows, pad))
+    res = ljamd.read_results(out["result"])[0]
+    ok = cols < n
+    j = np.where(ok, cols, 0)
+    pos = np.stack([x, y, z], 1)
+    d32 = pos[j] - pos[:, None, :]
+    fma = lambda a, s: (a.astype(np.float64) ** 2 + s.astype(np.float64)).astype(np.float32)  # noqa: E731
+    d2 = fma(d32[..., 2], fma(d32[..., 1], d32[..., 0] * d32[..., 0]))
+    hit = ok & (d2 <= np.float32(0.6) * np.float32(0.6)) & (d2 >= 1e-16)
+    dd = pos[j].astype(np.float64) - pos[:, None, :].astype(np.float64)
+    r2 = np.where(hit, (dd**2).sum(-1), 1.0)
+    s6 = np.where(hit, (float(np.float32(0.05)) ** 2 / r2) ** 3, 0.0)
+    w = -24.0 * s6 * (2 * s6 - 1) / r2
+    parts = 24.0 * s6 * (2 * s6 + 1) / r2
+    f, terms = (w[..., None] * dd).sum(1), (parts[..., None] * np.abs(dd)).sum(1)
+    tol = 2.0**-23 * np.abs(f) + (2.0**-18 if prec != "mixed" else 2.0**-45) * terms
+    got = np.stack([out[k][:n].cpu().numpy() for k in ("fx", "fy", "fz")], 1).astype(np.float64)
+    assert int(res["n_candidates"]) == int(ok.sum()) and int(res["n_pairs"]) == int(hit.sum())
+    assert np.all(np.abs(got - f) <= tol)
+    e_tol = (2.0**-45 if prec == "mixed" else 2.0**-18) * 2.0 * (s6 * (s6 + 1)).sum()
+    assert abs(float(res["e_total"]) - 2.0 * (s6 * (s6 - 1)).sum()) <= e_tol
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 512 * 256 - 1, 512 * 256 + 1, 400_003])
+def test_max_displacement_sizes(engine, n):
+    """The largest displacement wherever it lies, across the grid's stride; a NaN one is
+    infinite."""
+    rng = np.random.default_rng(n)
+    x = rng.uniform(0, 1, n).astype(np.float32)
+    d = engine.to_device(x, x, x)
+    for at in {0, n // 2, n - 1}:
+        moved = d[0].clone()
+        moved[at] += 0.5
+        want = float((moved[at] - d[0][at]).cpu()) ** 2
+        got = float(engine.max_displacement2(moved, d[1], d[2], *d).cpu()[0])
+        assert got == pytest.approx(want, rel=1e-6)
+        moved[at] = float("nan")
+        assert float(engine.max_displacement2(moved, d[1], d[2], *d).cpu()[0]) == float("inf")
