@@ -410,10 +410,11 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     uint32_t* off;
     {
         PhaseTimer tb(ctx, LJ_PHASE_BIN, s);
-        fill_u64(reinterpret_cast<unsigned long long*>(results), (uint32_t)(4 * nsys), 0ull, s);
         int bits = 0;
         while (bits < 32 && ((uint64_t)1 << bits) < (uint64_t)ncells) ++bits;
-        LJ_TRY(sort_particles(ctx, x, y, z, n, BatchKeyOp{dsys, dfirst, hfirst, (uint32_t)nsys}, bits, s));
+        uint32_t* ngaps = nullptr;
+        LJ_TRY(gap_list(ctx, ncells, &ngaps));
+        LJ_TRY(sort_particles(ctx, x, y, z, n, BatchKeyOp{dsys, dfirst, hfirst, (uint32_t)nsys}, bits, s, ngaps));
         LJ_TRY(cell_offsets_from_sorted(ctx, n, ncells, s));
         off = B.offsets.as<uint32_t>();
     }

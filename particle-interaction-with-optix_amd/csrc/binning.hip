@@ -19,6 +19,7 @@
 //    once, with no per-cell count array or scan (the reference counts with atomics
 //    and prefix-sums the counts, cudaLJ.cu:345-383 and prefixsum.hpp);
 //  - the candidate count is a closed form over cells, not a pass over particles.
+#include "lj_candidates.h"
 #include "lj_internal.h"
 #include "lj_sort.h"
 
@@ -148,6 +149,10 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_down(const TI* in, TS* ou
 constexpr uint32_t kGapLane = 8;
 constexpr uint32_t kGapInline = 256;
 constexpr uint32_t kGapPiece = 4096;
+// Grids of up to this many cells need no list: the longest possible range is 1024 stores
+// of one wave (about 7 us, once), and the list costs two launches (its clearing and
+// k_fill_gaps, 4-6 us together).
+constexpr uint32_t kGapNoList = 65536;
 constexpr unsigned kGapBlocks = 1024;
 
 struct GapPiece {
@@ -157,11 +162,13 @@ struct GapPiece {
 // off[a .. b) = v for each lane's range: short ranges by the lane itself, medium ones
 // by the whole wave one range at a time, longer ones cut into pieces appended to the
 // list (one atomic per wave: lanes take consecutive entries from a wave-wide prefix
-// sum).  Every lane of the wave calls this.
+// sum).  Without LIST the wave writes a range of any length itself.  Every lane of the
+// wave calls this.
+template <bool LIST>
 __device__ inline void fill_cells(uint32_t a, uint32_t b, uint32_t v, uint32_t* __restrict__ off,
                                   GapPiece* __restrict__ gaps, uint32_t* __restrict__ ngaps) {
     const uint32_t len = b - a;
-    const bool piecewise = len > kGapInline;
+    const bool piecewise = LIST && len > kGapInline;
     if (len <= kGapLane)
         for (uint32_t c = a; c < b; ++c) off[c] = v;
     for (uint64_t m = __ballot(len > kGapLane && !piecewise); m; m &= m - 1) {
@@ -170,7 +177,7 @@ __device__ inline void fill_cells(uint32_t a, uint32_t b, uint32_t v, uint32_t* 
         const uint32_t lv = __builtin_amdgcn_readlane(v, l);
         for (uint32_t c = la + lane_id(); c < lb; c += kWave) off[c] = lv;
     }
-    if (!__any(piecewise)) return;
+    if (!LIST || !__any(piecewise)) return;
     const uint32_t pieces = piecewise ? (len + kGapPiece - 1) / kGapPiece : 0u;
     const uint32_t incl = wave_incl_scan_t(pieces);
     uint32_t at = 0;
@@ -198,7 +205,7 @@ constexpr uint32_t kStage = 1024;
 constexpr uint32_t kStageMin = kWave;
 constexpr int kOffChunks = 4;
 
-template <bool STAGE>
+template <bool STAGE, bool LIST>
 __global__ __launch_bounds__(256) void k_offsets(const uint32_t* __restrict__ skeys, uint32_t n, uint32_t ncells,
                                                  uint32_t* __restrict__ off, GapPiece* __restrict__ gaps,
                                                  uint32_t* __restrict__ ngaps) {
@@ -246,12 +253,12 @@ __global__ __launch_bounds__(256) void k_offsets(const uint32_t* __restrict__ sk
             }
             for (uint32_t c = lane_id(); c < E - A; c += kWave) off[A + c] = st[c];
         } else {
-            fill_cells(a, b, v, off, gaps, ngaps);
+            fill_cells<LIST>(a, b, v, off, gaps, ngaps);
         }
         // the cells above the last key take n (the wave holding slot n - 1)
         if (__any(k == n - 1)) {
             const bool last = k == n - 1;
-            fill_cells(last ? key + 1u : 0u, last ? ncells + 1u : 0u, n, off, gaps, ngaps);
+            fill_cells<LIST>(last ? key + 1u : 0u, last ? ncells + 1u : 0u, n, off, gaps, ngaps);
         }
     }
 }
@@ -280,49 +287,20 @@ __global__ __launch_bounds__(256) void k_fill_u64(unsigned long long* p, uint32_
     if (i < n) p[i] = v;
 }
 
-// sum over cells of n_c * (S_c - 1), S_c = the clipped 27-cell count including c;
-// equals the per-particle count of ComputeNbInteractions (cudaLJ.cu:278-292).  One
-// wave per (y,z) row of cells at a time, lanes along x: the row's neighbour rows are
-// wave-uniform, so a cell's 27-cell count is nine x-range differences of the offsets
-// (coalesced across the lanes) and no per-cell index arithmetic.  Each workgroup
-// writes its sum to part[blockIdx.x] and k_sum_parts adds them up: on sparse grids
-// (millions of mostly empty cells) the walk is a chain of dependent loads, so it needs
-// many waves in flight, and atomics of that many workgroups to one counter would
-// serialise.
+// Each workgroup writes its sum to part[blockIdx.x]: on sparse grids (millions of mostly
+// empty cells) the walk is a chain of dependent loads, so it needs many waves in flight,
+// and atomics of that many workgroups to one counter would serialise.
 constexpr unsigned kCandBlocks = 8192;
 
 __global__ __launch_bounds__(256) void k_candidates(const uint32_t* __restrict__ off, GridGeom g,
                                                     unsigned long long* __restrict__ part) {
     constexpr unsigned kWaves = 256 / kWave;
     __shared__ unsigned long long wsum[kWaves];
-    const int32_t gx = g.g[0], gy = g.g[1], gz = g.g[2];
-    const uint32_t nrows = (uint32_t)gy * (uint32_t)gz;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int32_t lane = (int32_t)lane_id();
-    unsigned long long v = 0;
-    for (uint32_t r = blockIdx.x * kWaves + wave; r < nrows; r += gridDim.x * kWaves) {
-        const int32_t cy = (int32_t)(r % (uint32_t)gy), cz = (int32_t)(r / (uint32_t)gy);
-        const int32_t z0 = cz > 0 ? cz - 1 : 0, z1 = cz < gz - 1 ? cz + 1 : gz - 1;
-        const int32_t y0 = cy > 0 ? cy - 1 : 0, y1 = cy < gy - 1 ? cy + 1 : gy - 1;
-        const uint32_t* home = off + (size_t)r * (size_t)gx;
-        for (int32_t cx = lane; cx < gx; cx += kWave) {
-            const uint32_t nh = home[cx + 1] - home[cx];
-            if (!nh) continue;
-            // x-cells x0 .. xe - 1 of each neighbour row (the counts of at most n
-            // particles fit 32 bits)
-            const int32_t x0 = cx > 0 ? cx - 1 : 0, xe = cx < gx - 1 ? cx + 2 : gx;
-            uint32_t sum = 0;
-            for (int32_t zz = z0; zz <= z1; ++zz)
-                for (int32_t yy = y0; yy <= y1; ++yy) {
-                    const uint32_t* rw = off + ((size_t)zz * (size_t)gy + (size_t)yy) * (size_t)gx;
-                    sum += rw[xe] - rw[x0];
-                }
-            v += (unsigned long long)nh * (sum - 1);
-        }
-    }
+    unsigned long long v = candidate_rows(off, g, blockIdx.x * kWaves + wave, gridDim.x * kWaves);
 #pragma unroll
     for (int d = kWave / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, kWave);
-    if (lane == 0) wsum[wave] = v;
+    if (lane_id() == 0) wsum[wave] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long t = 0;
@@ -421,6 +399,21 @@ int scan_u32_to_u64(lj_context* ctx, const uint32_t* in, unsigned long long* out
     return scan_any<uint32_t, unsigned long long>(ctx, in, out, n, out + (n > 0 ? n : 0), s);
 }
 
+// gaps are disjoint and each piece list entry covers kGapPiece cells, or ends a gap of
+// more than kGapInline cells
+static size_t gap_capacity(uint32_t ncells) {
+    const size_t cells = (size_t)ncells + 1;
+    return cells / kGapPiece + cells / kGapInline + 2;
+}
+
+int gap_list(lj_context* ctx, uint32_t ncells, uint32_t** counter) {
+    *counter = nullptr;
+    if (ncells <= kGapNoList) return LJ_OK;
+    LJ_HIP(ctx, ctx->bin.gaps.grow(sizeof(uint32_t) * 4 + gap_capacity(ncells) * sizeof(GapPiece)));
+    *counter = ctx->bin.gaps.as<uint32_t>();
+    return LJ_OK;
+}
+
 int cell_offsets_from_sorted(lj_context* ctx, int64_t n, uint32_t ncells, hipStream_t s) {
     BinWork& w = ctx->bin;
     LJ_HIP(ctx, w.offsets.grow(((size_t)ncells + 1) * 4));
@@ -430,29 +423,33 @@ int cell_offsets_from_sorted(lj_context* ctx, int64_t n, uint32_t ncells, hipStr
         LJ_HIP(ctx, hipGetLastError());
         return LJ_OK;
     }
-    // gaps are disjoint and each piece list entry covers kGapPiece cells, or ends a gap
-    // of more than kGapInline cells
-    const size_t cells = (size_t)ncells + 1;
-    const size_t cap = cells / kGapPiece + cells / kGapInline + 2;
-    LJ_HIP(ctx, w.gaps.grow(sizeof(uint32_t) * 4 + cap * sizeof(GapPiece)));
-    uint32_t* ngaps = w.gaps.as<uint32_t>();
-    GapPiece* gaps = reinterpret_cast<GapPiece*>(w.gaps.as<uint8_t>() + sizeof(uint32_t) * 4);
-    fill_u32(ngaps, 1, 0u, s);
-    if (2 * (uint64_t)ncells >= 3 * (uint64_t)n)
-        hipLaunchKernelGGL(k_offsets<true>, dim3(div_up(n, 256 * kOffChunks)), dim3(256), 0, s, w.sorted_keys(), (uint32_t)n, ncells, off,
-                       gaps, ngaps);
-    else
-        hipLaunchKernelGGL(k_offsets<false>, dim3(div_up(n, 256 * kOffChunks)), dim3(256), 0, s, w.sorted_keys(), (uint32_t)n, ncells, off,
-                       gaps, ngaps);
-    const unsigned nb = (unsigned)(cap < kGapBlocks ? cap : kGapBlocks);
-    hipLaunchKernelGGL(k_fill_gaps, dim3(nb), dim3(256), 0, s, (const GapPiece*)gaps, (const uint32_t*)ngaps, off);
+    uint32_t* ngaps = nullptr;
+    LJ_TRY(gap_list(ctx, ncells, &ngaps));
+    GapPiece* gaps = ngaps ? reinterpret_cast<GapPiece*>(ngaps + 4) : nullptr;
+    const bool stage = 2 * (uint64_t)ncells >= 3 * (uint64_t)n;
+#define LJ_OFFSETS(STAGE, LIST)                                                                                      \
+    hipLaunchKernelGGL((k_offsets<STAGE, LIST>), dim3(div_up(n, 256 * kOffChunks)), dim3(256), 0, s, w.sorted_keys(), \
+                       (uint32_t)n, ncells, off, gaps, ngaps)
+    if (ngaps) {
+        if (stage) LJ_OFFSETS(true, true);
+        else LJ_OFFSETS(false, true);
+        const size_t cap = gap_capacity(ncells);
+        const unsigned nb = (unsigned)(cap < kGapBlocks ? cap : kGapBlocks);
+        hipLaunchKernelGGL(k_fill_gaps, dim3(nb), dim3(256), 0, s, (const GapPiece*)gaps, (const uint32_t*)ngaps, off);
+    } else {
+        if (stage) LJ_OFFSETS(true, false);
+        else LJ_OFFSETS(false, false);
+    }
+#undef LJ_OFFSETS
     LJ_HIP(ctx, hipGetLastError());
     return LJ_OK;
 }
 
 int bin_particles(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n,
                   const GridGeom& g, hipStream_t s) {
-    LJ_TRY(sort_particles(ctx, x, y, z, n, CellKeyOp{g}, key_bits(g.ncells), s));
+    uint32_t* ngaps = nullptr;
+    LJ_TRY(gap_list(ctx, g.ncells, &ngaps));
+    LJ_TRY(sort_particles(ctx, x, y, z, n, CellKeyOp{g}, key_bits(g.ncells), s, ngaps));
     return cell_offsets_from_sorted(ctx, n, g.ncells, s);
 }
 
@@ -464,21 +461,28 @@ int extract_perm(lj_context* ctx, int64_t n, uint32_t* perm, hipStream_t s) {
     return LJ_OK;
 }
 
-int count_candidates_from(lj_context* ctx, const GridGeom& g, const uint32_t* offsets, unsigned long long* out,
-                          hipStream_t s) {
+unsigned candidate_blocks(const GridGeom& g) {
     const uint64_t nrows = (uint64_t)g.g[1] * (uint64_t)g.g[2];
     const uint64_t rb = (nrows + 3) / 4;  // four waves (rows) per workgroup
-    const unsigned nb = (unsigned)(rb < kCandBlocks ? (rb > 0 ? rb : 1) : kCandBlocks);
+    return (unsigned)(rb < kCandBlocks ? (rb > 0 ? rb : 1) : kCandBlocks);
+}
+
+int candidate_parts(lj_context* ctx, const GridGeom& g, const uint32_t* offsets, unsigned* nparts, hipStream_t s) {
+    const unsigned nb = candidate_blocks(g);
     LJ_HIP(ctx, ctx->bin.cand.grow((size_t)nb * sizeof(unsigned long long)));
-    unsigned long long* part = ctx->bin.cand.as<unsigned long long>();
-    hipLaunchKernelGGL(k_candidates, dim3(nb), dim3(256), 0, s, offsets, g, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kSumThreads), 0, s, (const unsigned long long*)part, nb, out);
+    hipLaunchKernelGGL(k_candidates, dim3(nb), dim3(256), 0, s, offsets, g, ctx->bin.cand.as<unsigned long long>());
     LJ_HIP(ctx, hipGetLastError());
+    *nparts = nb;
     return LJ_OK;
 }
 
 int count_candidates(lj_context* ctx, const GridGeom& g, unsigned long long* out, hipStream_t s) {
-    return count_candidates_from(ctx, g, ctx->bin.offsets.as<uint32_t>(), out, s);
+    unsigned nb = 0;
+    LJ_TRY(candidate_parts(ctx, g, ctx->bin.offsets.as<uint32_t>(), &nb, s));
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kSumThreads), 0, s,
+                       (const unsigned long long*)ctx->bin.cand.as<unsigned long long>(), nb, out);
+    LJ_HIP(ctx, hipGetLastError());
+    return LJ_OK;
 }
 
 void fill_u64(unsigned long long* p, uint32_t n, unsigned long long v, hipStream_t s) {

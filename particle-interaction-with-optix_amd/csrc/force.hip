@@ -13,6 +13,7 @@
 // itself is stencil_pairs in lj_stencil.h).
 #include <cmath>
 
+#include "lj_candidates.h"
 #include "lj_rows.h"
 #include "lj_sort.h"
 #include "lj_stencil.h"
@@ -25,8 +26,10 @@ namespace {
 // dynamic LDS (depth x block entries of 16 bytes, one block of rings per wave; none
 // without QUEUE).  Outputs go to the caller's order (pi.w holds the original index),
 // or, when `so` is set (lj_compute_sorted), to the sorted slot k together with the
-// particle's position and original index; per-block FP64 energy and virial partials are
-// reduced later in a fixed order.
+// particle's position and original index; each workgroup's totals go to sums and are
+// reduced later in a fixed order.  The workgroups past the first nforce count the 27-cell
+// candidates of the same grid instead (none when they are not wanted or belong to another
+// grid): they need only the offsets, and a launch of their own costs 4-5 us.
 // OUT: how the outputs are stored -- 0 ordinary stores, 1 non-temporal stores, 2 one
 // non-temporal staged record per particle at its caller index (large outputs at
 // shuffled indices; never with `so`).
@@ -35,11 +38,18 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force(const float4* __restrict
                                                      const uint32_t* __restrict__ off, uint32_t n, GridGeom g, int Rx,
                                                      int R, Trim tr, PairConst c, uint32_t depth, float* __restrict__ fx,
                                                      float* __restrict__ fy, float* __restrict__ fz,
-                                                     float* __restrict__ e, double* __restrict__ partials,
-                                                     unsigned long long* __restrict__ npairs, SortedOut so,
+                                                     float* __restrict__ e, uint32_t nforce,
+                                                     BlockSums* __restrict__ sums, SortedOut so,
                                                      float4* __restrict__ stage) {
     extern __shared__ QEntry queue[];
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    if (blockIdx.x >= nforce) {
+        const uint32_t waves = blockDim.x / kWaveSize;
+        const uint32_t wave = (blockIdx.x - nforce) * waves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+        const unsigned long long nc = candidate_rows(off, g, wave, (gridDim.x - nforce) * waves);
+        store_block_sums<false, true>(&sums[blockIdx.x], 0.0, 0.0, 0ull, nc);
+        return;
+    }
+    const uint32_t blk = xcd_block(blockIdx.x, nforce);
     const uint32_t k = blk * blockDim.x + threadIdx.x;
     // the slot rebuilt after the pair loop from wave-uniform values and the lane id, so
     // that no per-lane index stays live across it (64 VGPRs are the budget)
@@ -83,13 +93,7 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force(const float4* __restrict
         esum = ei;
         vsum = c.e24 * (double)acc.av.value();
     }
-    block_sum2(esum, vsum);
-    const unsigned long long bp = block_sum_u64(np);
-    if (threadIdx.x == 0) {
-        partials[2 * blk] = esum;
-        partials[2 * blk + 1] = vsum;
-        if (npairs && bp) atomicAdd(npairs, bp);
-    }
+    store_block_sums<true, false>(&sums[blk], esum, vsum, np, 0ull);
 }
 
 __global__ __launch_bounds__(256) void k_split_outputs(const float4* __restrict__ stage, uint32_t n,
@@ -111,27 +115,34 @@ __global__ __launch_bounds__(256) void k_coarse_counts(const uint32_t* __restric
     ccount[c] = coarse_count(foff, fg, cg, Kx, K, c);
 }
 
-// FP64 reduction of the per-block partials in a fixed order: stage 1 sums chunks of
-// 1024 pairs into out (one block per chunk), stage 2 (one block, res != NULL) sums
-// the chunk results into res.
-__global__ __launch_bounds__(256) void k_finalize(const double* __restrict__ partials, uint32_t nblocks,
-                                                  double* __restrict__ out, lj_result* __restrict__ res) {
+// The workgroups' sums in a fixed order: stage 1 (res NULL) sums chunks of kFinalChunk of
+// them into out (one workgroup per chunk), stage 2 (one workgroup) sums those, or up to
+// kFinalOne sums directly, and further candidate counts into *res.
+__global__ __launch_bounds__(1024) void k_finalize(const BlockSums* __restrict__ sums, uint32_t nblocks,
+                                                   const unsigned long long* __restrict__ cand, uint32_t ncand,
+                                                   const int* __restrict__ overflow, BlockSums* __restrict__ out,
+                                                   lj_result* __restrict__ res) {
+    __shared__ BlockSums total;
     double a = 0.0, b = 0.0;
-    const uint32_t lo = res ? 0 : blockIdx.x * 1024u;
-    const uint32_t hi = res ? nblocks : (lo + 1024u < nblocks ? lo + 1024u : nblocks);
-    for (uint32_t q = lo + threadIdx.x; q < hi; q += 256) {
-        a += partials[2 * q];
-        b += partials[2 * q + 1];
+    unsigned long long np = 0, nc = 0;
+    const uint32_t lo = res ? 0 : blockIdx.x * kFinalChunk;
+    const uint32_t hi = res ? nblocks : (lo + kFinalChunk < nblocks ? lo + kFinalChunk : nblocks);
+    for (uint32_t q = lo + threadIdx.x; q < hi; q += blockDim.x) {
+        a += sums[q].e;
+        b += sums[q].v;
+        np += sums[q].np;
+        nc += sums[q].nc;
     }
-    block_sum2(a, b);
-    if (threadIdx.x == 0) {
-        if (res) {
-            res->e_total = 0.5 * a;
-            res->virial = 0.5 * b;
-        } else {
-            out[2 * blockIdx.x] = a;
-            out[2 * blockIdx.x + 1] = b;
-        }
+    if (res)
+        for (uint32_t q = threadIdx.x; q < ncand; q += blockDim.x) nc += cand[q];
+    store_block_sums<true, true>(&total, a, b, np, nc);
+    if (threadIdx.x != 0) return;
+    if (!res) {
+        out[blockIdx.x] = total;
+    } else if (overflow && *overflow) {
+        *res = lj_result{__builtin_nan(""), __builtin_nan(""), total.nc, ~0ull};
+    } else {
+        *res = lj_result{0.5 * total.e, 0.5 * total.v, total.nc, total.np};
     }
 }
 
@@ -347,13 +358,13 @@ __global__ __launch_bounds__(256) void k_unpack(const float4* __restrict__ pos, 
 template <int PRED>
 void launch_force(int prec, bool vir, const Shape& sh, unsigned nb, hipStream_t s, const float4* pos,
                   const uint32_t* cell_of, const uint32_t* off, uint32_t n, const GridGeom& g, const Trim& tr,
-                  const PairConst& c, float* fx, float* fy, float* fz, float* e, double* partials,
-                  unsigned long long* npairs, const SortedOut& so, float4* stage) {
+                  const PairConst& c, float* fx, float* fy, float* fz, float* e, unsigned nforce, BlockSums* sums,
+                  const SortedOut& so, float4* stage) {
     const size_t lds = sh.lds_bytes();
     const int out = stage ? 2 : non_temporal_outputs(n) ? 1 : 0;
 #define LJ_LAUNCH_QN(PREC, VIR, Q, OUT)                                                                              \
     hipLaunchKernelGGL((k_force<PRED, PREC, VIR, Q, OUT>), dim3(nb), dim3(sh.block), lds, s, pos, cell_of, off, n, g, \
-                       sh.refine_x, sh.refine, tr, c, (uint32_t)sh.depth, fx, fy, fz, e, partials, npairs, so, stage)
+                       sh.refine_x, sh.refine, tr, c, (uint32_t)sh.depth, fx, fy, fz, e, nforce, sums, so, stage)
 #define LJ_LAUNCH_Q(PREC, VIR, Q)                      \
     do {                                               \
         if (out == 2) LJ_LAUNCH_QN(PREC, VIR, Q, 2);   \
@@ -382,19 +393,28 @@ void split_outputs(const float4* stage, uint32_t n, float* fx, float* fy, float*
     hipLaunchKernelGGL(k_split_outputs, dim3(div_up(n, 256)), dim3(256), 0, s, stage, n, fx, fy, fz, e);
 }
 
-void finalize_energy(double* partials, unsigned nblocks, lj_result* res, hipStream_t s) {
-    if (nblocks > 1024) {
-        // stage 1 writes behind the nblocks input pairs (the partials buffer holds room)
-        const unsigned chunks = (nblocks + 1023) / 1024;
-        double* tmp = partials + 2 * (size_t)nblocks;
-        hipLaunchKernelGGL(k_finalize, dim3(chunks), dim3(256), 0, s, (const double*)partials, (uint32_t)nblocks, tmp,
-                           (lj_result*)nullptr);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, (const double*)tmp, (uint32_t)chunks, (double*)nullptr,
-                           res);
-    } else {
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s, (const double*)partials, (uint32_t)nblocks,
-                           (double*)nullptr, res);
+int grow_block_sums(lj_context* ctx, unsigned nblocks, BlockSums** out) {
+    LJ_HIP(ctx, ctx->bin.partials.grow(((size_t)nblocks + nblocks / kFinalChunk + 1) * sizeof(BlockSums)));
+    *out = ctx->bin.partials.as<BlockSums>();
+    return LJ_OK;
+}
+
+int finalize_totals(lj_context* ctx, unsigned nblocks, const unsigned long long* cand, unsigned ncand,
+                    const int* overflow, lj_result* res, hipStream_t s) {
+    BlockSums* sums = ctx->bin.partials.as<BlockSums>();
+    if (nblocks > kFinalOne) {
+        // stage 1 writes behind the nblocks input sums (grow_block_sums left room)
+        const unsigned chunks = (nblocks + kFinalChunk - 1) / kFinalChunk;
+        BlockSums* tmp = sums + nblocks;
+        hipLaunchKernelGGL(k_finalize, dim3(chunks), dim3(256), 0, s, (const BlockSums*)sums, (uint32_t)nblocks,
+                           (const unsigned long long*)nullptr, 0u, (const int*)nullptr, tmp, (lj_result*)nullptr);
+        sums = tmp;
+        nblocks = chunks;
     }
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, s, (const BlockSums*)sums, (uint32_t)nblocks, cand, ncand,
+                       overflow, (BlockSums*)nullptr, res);
+    LJ_HIP(ctx, hipGetLastError());
+    return LJ_OK;
 }
 
 // Scalar results live in the caller's lj_result or, when it is NULL, in a scratch one.
@@ -487,27 +507,27 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
     }
     lj_result* res;
     LJ_TRY(result_slot(ctx, result, &res));
-    {
+    // The candidate count, on the cell_edge grid (ComputeNbInteractions semantics), is
+    // only made for a caller that takes the results: by further workgroups of the force
+    // launch when that grid is the force grid, else from cell_edge offsets of its own.
+    const unsigned nforce = div_up(n > 0 ? n : 1, sh.block);
+    unsigned ncount = 0, nparts = 0;
+    if (result && !refined) ncount = candidate_blocks(g);
+    if (result && refined) {
         PhaseTimer t(ctx, LJ_PHASE_OTHER, s);
-        if (!refined) {
-            LJ_TRY(count_candidates(ctx, g, &res->n_candidates, s));
-        } else {
-            // candidate count on the cell_edge grid (ComputeNbInteractions semantics)
-            BinWork& w = ctx->bin;
-            LJ_HIP(ctx, w.ccounts.grow((size_t)g.ncells * 4));
-            LJ_HIP(ctx, w.coffsets.grow(((size_t)g.ncells + 1) * 4));
-            hipLaunchKernelGGL(k_coarse_counts, dim3(div_up(g.ncells, 256)), dim3(256), 0, s,
-                               (const uint32_t*)w.offsets.as<uint32_t>(), fg, g, sh.refine_x, sh.refine,
-                               w.ccounts.as<uint32_t>());
-            uint32_t* coff = w.coffsets.as<uint32_t>();
-            LJ_TRY(scan_u32(ctx, w.ccounts.as<uint32_t>(), coff, g.ncells, coff + g.ncells, s));
-            LJ_TRY(count_candidates_from(ctx, g, coff, &res->n_candidates, s));
-        }
-        fill_u64(&res->n_pairs, 1, 0ull, s);
+        BinWork& w = ctx->bin;
+        LJ_HIP(ctx, w.ccounts.grow((size_t)g.ncells * 4));
+        LJ_HIP(ctx, w.coffsets.grow(((size_t)g.ncells + 1) * 4));
+        hipLaunchKernelGGL(k_coarse_counts, dim3(div_up(g.ncells, 256)), dim3(256), 0, s,
+                           (const uint32_t*)w.offsets.as<uint32_t>(), fg, g, sh.refine_x, sh.refine,
+                           w.ccounts.as<uint32_t>());
+        uint32_t* coff = w.coffsets.as<uint32_t>();
+        LJ_TRY(scan_u32(ctx, w.ccounts.as<uint32_t>(), coff, g.ncells, coff + g.ncells, s));
+        LJ_TRY(candidate_parts(ctx, g, coff, &nparts, s));
     }
-    const unsigned nb = div_up(n > 0 ? n : 1, sh.block);
-    LJ_HIP(ctx, ctx->bin.partials.grow(((size_t)nb + nb / 1024 + 1) * 2 * sizeof(double)));
-    double* partials = ctx->bin.partials.as<double>();
+    const unsigned nb = nforce + ncount;
+    BlockSums* sums;
+    LJ_TRY(grow_block_sums(ctx, nb, &sums));
     const int prec = p->precision;
     const bool vir = !(p->flags & LJ_FLAG_NO_VIRIAL);
     const float4* pos = ctx->bin.pos.as<float4>();
@@ -524,8 +544,8 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
         PhaseTimer tf(ctx, LJ_PHASE_FORCE, s);
 #define LJ_PRED_CASE(P)                                                                                         \
     case P:                                                                                                     \
-        launch_force<P>(prec, vir, sh, nb, s, pos, cell_of, off, nn, fg, tr, c, fx, fy, fz, e, partials,      \
-                        &res->n_pairs, so, stage);                                                              \
+        launch_force<P>(prec, vir, sh, nb, s, pos, cell_of, off, nn, fg, tr, c, fx, fy, fz, e, nforce, sums, so, \
+                        stage);                                                                                 \
         break;
         switch (p->predicate) {
             LJ_PRED_CASE(LJ_PRED_AABB)
@@ -538,9 +558,7 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
     }
     PhaseTimer to(ctx, LJ_PHASE_OTHER, s);
     if (stage) split_outputs(stage, nn, fx, fy, fz, e, s);
-    finalize_energy(partials, nb, res, s);
-    LJ_HIP(ctx, hipGetLastError());
-    return LJ_OK;
+    return finalize_totals(ctx, nb, ctx->bin.cand.as<unsigned long long>(), nparts, nullptr, res, s);
 }
 
 static void sort_long_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {

@@ -417,8 +417,8 @@ __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_force(const float4* __restr
                                                     const int* __restrict__ rope_by_end, const float4* __restrict__ box, int n, float h, uint32_t limit, PairConst c,
                                                     float* __restrict__ fx, float* __restrict__ fy,
                                                     float* __restrict__ fz, float* __restrict__ e,
-                                                    double* __restrict__ partials, lj_result* __restrict__ res,
-                                                    int* __restrict__ overflow, float4* __restrict__ stage) {
+                                                    BlockSums* __restrict__ sums, int* __restrict__ overflow,
+                                                    float4* __restrict__ stage) {
     extern __shared__ int lds_list[];
     int* list = lds_list + threadIdx.x;
     // consecutive queries walk nearly the same nodes: keep them on one XCD (own L2)
@@ -456,15 +456,7 @@ __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_force(const float4* __restr
         esum = ei;
         vsum = c.e24 * (double)acc.av.value();
     }
-    block_sum2(esum, vsum);
-    const unsigned long long bp = block_sum_u64(np);
-    const unsigned long long bt = block_sum_u64(tests);
-    if (threadIdx.x == 0) {
-        partials[2 * blk] = esum;
-        partials[2 * blk + 1] = vsum;
-        if (bp) atomicAdd(&res->n_pairs, bp);
-        if (bt) atomicAdd(&res->n_candidates, bt);
-    }
+    store_block_sums<true, true>(&sums[blk], esum, vsum, np, tests);
 }
 
 template <int PRED>
@@ -504,17 +496,6 @@ __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_fill(const float4* __restri
             cols[w++] = __float_as_uint(pj.w);
     });
     if (!ok) atomicOr(overflow, 1);
-}
-
-// Marks the results of a force call whose walk tripped its step guard: n_pairs =
-// UINT64_MAX and NaN totals, so a caller that reads the results sees the failure
-// without the call synchronising.
-__global__ void k_poison_on_overflow(const int* __restrict__ overflow, lj_result* __restrict__ res) {
-    if (threadIdx.x == 0 && *overflow) {
-        res->n_pairs = ~0ull;
-        res->e_total = __builtin_nan("");
-        res->virial = __builtin_nan("");
-    }
 }
 
 }  // namespace
@@ -646,11 +627,10 @@ int lj_lbvh_compute(lj_context* ctx, const float* x, const float* y, const float
         LJ_HIP(ctx, ctx->bin.counters.grow(sizeof(lj_result)));
         res = ctx->bin.counters.as<lj_result>();
     }
-    fill_u64(&res->n_candidates, 2, 0ull, s);
     const unsigned nb = div_up(n > 0 ? n : 1, kLbvhBlock);
     const size_t lds = (size_t)kList * kLbvhBlock * sizeof(int);
-    LJ_HIP(ctx, ctx->bin.partials.grow(((size_t)nb + nb / 1024 + 1) * 2 * sizeof(double)));
-    double* partials = ctx->bin.partials.as<double>();
+    BlockSums* sums;
+    LJ_TRY(grow_block_sums(ctx, nb, &sums));
     int* ovf = overflow_flag(ctx, n);
     const float h = query_half_width(p);
     const uint32_t lim = walk_limit(p, n);
@@ -668,7 +648,7 @@ int lj_lbvh_compute(lj_context* ctx, const float* x, const float* y, const float
     }
 #define LJ_LBN(PRED, PREC, VIR, NT)                                                                                  \
     hipLaunchKernelGGL((k_lbvh_force<PRED, PREC, VIR, NT>), dim3(nb), dim3(kLbvhBlock), lds, s, leaf, range, rope, box, \
-                       (int)n, h, lim, c, fx, fy, fz, e, partials, res, ovf, stage)
+                       (int)n, h, lim, c, fx, fy, fz, e, sums, ovf, stage)
 #define LJ_LB(PRED, PREC, VIR)                  \
     do {                                        \
         if (nt) LJ_LBN(PRED, PREC, VIR, true);  \
@@ -691,7 +671,7 @@ int lj_lbvh_compute(lj_context* ctx, const float* x, const float* y, const float
             }
         } else {
             hipLaunchKernelGGL((k_lbvh_force<LJ_PRED_AABB, LJ_PREC_MIXED, true, false>), dim3(1), dim3(kLbvhBlock), lds,
-                               s, leaf, range, rope, box, 0, h, lim, c, fx, fy, fz, e, partials, res, ovf, stage);
+                               s, leaf, range, rope, box, 0, h, lim, c, fx, fy, fz, e, sums, ovf, stage);
         }
     }
 #undef LJ_LB_PREC
@@ -699,10 +679,9 @@ int lj_lbvh_compute(lj_context* ctx, const float* x, const float* y, const float
 #undef LJ_LBN
     PhaseTimer to(ctx, LJ_PHASE_OTHER, s);
     if (stage) split_outputs(stage, (uint32_t)n, fx, fy, fz, e, s);
-    finalize_energy(partials, nb, res, s);
-    hipLaunchKernelGGL(k_poison_on_overflow, dim3(1), dim3(64), 0, s, (const int*)ovf, res);
-    LJ_HIP(ctx, hipGetLastError());
-    return LJ_OK;
+    // a walk that tripped its step guard marks the results, so a caller that reads them
+    // sees the failure without the call synchronising
+    return finalize_totals(ctx, nb, nullptr, 0u, ovf, res, s);
 }
 
 int lj_lbvh_pairs(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n, const lj_params* p,

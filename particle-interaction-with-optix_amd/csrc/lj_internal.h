@@ -218,15 +218,24 @@ struct CellKeyOp {
     __device__ uint32_t operator()(float x, float y, float z, uint32_t) const { return cell_key(g, x, y, z); }
 };
 
-// Cell counts and offsets (ncells+1) of ctx->bin from the sorted keys of a sort_particles.
+// Cell offsets (ncells+1) of ctx->bin from the sorted keys of a sort_particles, whose
+// first kernel must have cleared the word that gap_list returns (NULL: none).
+int gap_list(lj_context* ctx, uint32_t ncells, uint32_t** counter);
 int cell_offsets_from_sorted(lj_context* ctx, int64_t n, uint32_t ncells, hipStream_t s);
 
 // perm[k] = original index of sorted slot k (from ctx->bin.pos after a sort).
 int extract_perm(lj_context* ctx, int64_t n, uint32_t* perm, hipStream_t s);
 
-// res->e_total / res->virial from per-block FP64 partials (pairs of doubles), fixed order.
-// partials must hold room for nblocks + nblocks/1024 + 1 pairs (stage-1 results).
-void finalize_energy(double* partials, unsigned nblocks, lj_result* res, hipStream_t s);
+// All of *res from the BlockSums of nblocks workgroups (fixed order), plus ncand further
+// candidate counts (cand nullable).  overflow (nullable): a flag that marks the results as
+// failed (n_pairs = UINT64_MAX, NaN totals).
+struct BlockSums;
+constexpr unsigned kFinalChunk = 1024;  // sums of one workgroup of the first stage
+constexpr unsigned kFinalOne = 4096;    // sums that one workgroup takes without a first stage
+int finalize_totals(lj_context* ctx, unsigned nblocks, const unsigned long long* cand, unsigned ncand,
+                    const int* overflow, lj_result* res, hipStream_t s);
+// Room for nblocks BlockSums and the first stage's results in ctx->bin.partials.
+int grow_block_sums(lj_context* ctx, unsigned nblocks, BlockSums** out);
 
 // Bins n particles: fills ctx->bin.offsets (ncells+1), ctx->bin.pos (sorted float4 with
 // the original index in w) and the sorted cell keys (ctx->bin.sorted_keys()).
@@ -236,9 +245,11 @@ int bin_particles(lj_context* ctx, const float* x, const float* y, const float* 
 // Candidate count of the 27-cell stencil from ctx->bin.offsets, into *out (device u64),
 // which is overwritten (not accumulated).
 int count_candidates(lj_context* ctx, const GridGeom& g, unsigned long long* out, hipStream_t s);
-// Same from explicit offsets of grid g.
-int count_candidates_from(lj_context* ctx, const GridGeom& g, const uint32_t* offsets, unsigned long long* out,
-                          hipStream_t s);
+// Partial counts (their sum is the candidate count) from explicit offsets of grid g, in
+// ctx->bin.cand; *nparts of them.
+int candidate_parts(lj_context* ctx, const GridGeom& g, const uint32_t* offsets, unsigned* nparts, hipStream_t s);
+// Workgroups that a candidate count over grid g is worth (four rows of cells each, capped).
+unsigned candidate_blocks(const GridGeom& g);
 
 void fill_u64(unsigned long long* p, uint32_t n, unsigned long long v, hipStream_t s);
 // fx, fy, fz, e[i] = stage[i] for i < n (e nullable): outputs staged as one float4 per

@@ -235,4 +235,37 @@ __device__ inline unsigned long long block_sum_u64(unsigned long long v) {
     return t;
 }
 
+// What one workgroup adds to a call's totals: energy, virial, accepted and candidate
+// pairs.  finalize_totals sums them in a fixed order.
+struct BlockSums {
+    double e, v;
+    unsigned long long np, nc;
+};
+
+// Sums of a workgroup of up to 1024 threads (a whole number of waves) into *out, in a fixed
+// order.  Every thread must call it.  SUMS, COUNT: whether e, v and np, and nc, are given
+// (else zero).
+template <bool SUMS, bool COUNT>
+__device__ inline void store_block_sums(BlockSums* out, double e, double v, unsigned long long np, unsigned long long nc) {
+    __shared__ BlockSums sh[1024 / kWaveSize];
+    if constexpr (SUMS) {
+        e = wave_sum(e);
+        v = wave_sum(v);
+        np = wave_sum(np);
+    }
+    if constexpr (COUNT) nc = wave_sum(nc);
+    if (__lane_id() == 0) sh[threadIdx.x / kWaveSize] = BlockSums{e, v, np, nc};
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        BlockSums t{0.0, 0.0, 0ull, 0ull};
+        for (unsigned q = 0; q < blockDim.x / kWaveSize; ++q) {
+            t.e += sh[q].e;
+            t.v += sh[q].v;
+            t.np += sh[q].np;
+            t.nc += sh[q].nc;
+        }
+        *out = t;
+    }
+}
+
 }  // namespace lj

@@ -67,9 +67,10 @@ template <int RB, bool FIRST, class KeyOp>
 __global__ __launch_bounds__(kThreads) void k_hist(const float* __restrict__ x, const float* __restrict__ y,
                                                    const float* __restrict__ z, const uint32_t* __restrict__ kin,
                                                    uint32_t n, KeyOp op, int shift, uint32_t* __restrict__ hist,
-                                                   uint32_t* __restrict__ kstore) {
+                                                   uint32_t* __restrict__ kstore, uint32_t* __restrict__ zero) {
     constexpr int kRadix = 1 << RB;
     __shared__ uint32_t h[kRadix];
+    if (FIRST && zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0u;  // a counter of a later kernel
     for (int d = threadIdx.x; d < kRadix; d += kThreads) h[d] = 0;
     __syncthreads();
     const uint32_t base = blockIdx.x * kTile;
@@ -190,6 +191,39 @@ __global__ __launch_bounds__(1 << RB) void k_dig_down(uint32_t* __restrict__ his
     }
 }
 
+// The same in one kernel for tables of up to 16 PER tiles: a workgroup takes 64 digits, one
+// per lane, its 16 waves PER consecutive tiles each, all loaded at once.  hist[t * R + d]
+// becomes digit d's keys in earlier tiles, dtot[d] its total; the scatter adds the keys of
+// smaller digits itself (BASE).  Three launches cost about 9 us however small the table;
+// at 1M keys (512 tiles) the one takes 4.8 us.
+template <int RB, int PER>
+__global__ __launch_bounds__(1024) void k_dig_columns(uint32_t* __restrict__ hist, uint32_t ntiles,
+                                                      uint32_t* __restrict__ dtot) {
+    constexpr int kRadix = 1 << RB, kW = 1024 / kWave;
+    __shared__ uint32_t wsum[kW][kWave];
+    const unsigned lane = __lane_id(), w = threadIdx.x / kWave;
+    const uint32_t d = blockIdx.x * kWave + lane;
+    uint32_t v[PER];
+    uint32_t sum = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const uint32_t t = w * PER + i;
+        v[i] = t < ntiles ? hist[(uint64_t)t * kRadix + d] : 0u;
+        sum += v[i];
+    }
+    wsum[w][lane] = sum;
+    __syncthreads();
+    uint32_t run = 0;
+    for (unsigned k = 0; k < w; ++k) run += wsum[k][lane];
+    if (w == kW - 1) dtot[d] = run + sum;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const uint32_t t = w * PER + i;
+        if (t < ntiles) hist[(uint64_t)t * kRadix + d] = run;
+        run += v[i];
+    }
+}
+
 // Tile t (logical, XCD-aware: neighbouring tiles write neighbouring output runs and
 // share an L2) sorts its keys stably by digit and writes each digit's run.  Element j
 // of the tile (input order) is handled by wave j / kWaveKeys, round
@@ -198,7 +232,8 @@ template <int RB, bool FIRST, class KeyOp>
 __global__ __launch_bounds__(kSThreads) void k_scatter(const float* __restrict__ x, const float* __restrict__ y,
                                                        const float* __restrict__ z, const uint32_t* __restrict__ kin,
                                                        const float4* __restrict__ pin, uint32_t n, KeyOp op, int shift,
-                                                       const uint32_t* __restrict__ hist, uint32_t* __restrict__ kout,
+                                                       const uint32_t* __restrict__ hist,
+                                                       const uint32_t* __restrict__ dtot, uint32_t* __restrict__ kout,
                                                        float4* __restrict__ pout) {
     constexpr int kRadix = 1 << RB;
     static_assert(kRadix <= kSThreads, "one thread per digit combines the waves' counts");
@@ -212,7 +247,7 @@ __global__ __launch_bounds__(kSThreads) void k_scatter(const float* __restrict__
     static_assert(kTile < 65536, "16-bit counters");
     __shared__ uint32_t dstart[kRadix];         // first staging slot of each digit in this tile
     __shared__ uint32_t gbase[kRadix];          // first output slot of each digit for this tile
-    __shared__ uint32_t wsum[kRadix / kWave];
+    __shared__ uint32_t wsum[kRadix / kWave], bsum[kRadix / kWave];
     const unsigned tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t base = tile * kTile;
@@ -242,7 +277,13 @@ __global__ __launch_bounds__(kSThreads) void k_scatter(const float* __restrict__
     }
 #pragma unroll
     for (int q = 0; q < kRadix / 2 / kWave; ++q) wcnt[wave][q * kWave + lane] = 0;
-    if (tid < (unsigned)kRadix) gbase[tid] = hist[(uint64_t)tile * kRadix + tid];
+    // with dtot the table holds a digit's keys in earlier tiles, and the keys of smaller
+    // digits come from an exclusive scan of the digits' totals, here and at gbase's store
+    uint32_t first_slot = 0, below = 0;
+    if (tid < (unsigned)kRadix) {
+        first_slot = hist[(uint64_t)tile * kRadix + tid];
+        if (dtot) below = dtot[tid];
+    }
     // Stable ranks inside the wave: the lowest lane of each digit group adds the group's
     // size to the wave's counter with an LDS atomic (the wave's own counters, so no
     // other wave touches them) and hands the old value to its group.
@@ -271,7 +312,7 @@ __global__ __launch_bounds__(kSThreads) void k_scatter(const float* __restrict__
     // threads 0..R-1, one per digit: staging start of the digit (exclusive scan over
     // digits of the tile's counts) and of each wave's part of it
     uint32_t c[kSWaves];
-    uint32_t tot = 0, incl = 0;
+    uint32_t tot = 0, incl = 0, bincl = below;
     if (tid < (unsigned)kRadix) {
 #pragma unroll
         for (int w = 0; w < kSWaves; ++w) {
@@ -284,12 +325,26 @@ __global__ __launch_bounds__(kSThreads) void k_scatter(const float* __restrict__
             const uint32_t o = __shfl_up(incl, k, kWave);
             if (lane >= (unsigned)k) incl += o;
         }
-        if (lane == kWave - 1) wsum[wave] = incl;
+        if (dtot) {  // uniform
+#pragma unroll
+            for (int k = 1; k < kWave; k <<= 1) {
+                const uint32_t o = __shfl_up(bincl, k, kWave);
+                if (lane >= (unsigned)k) bincl += o;
+            }
+        }
+        if (lane == kWave - 1) {
+            wsum[wave] = incl;
+            bsum[wave] = bincl;
+        }
     }
     __syncthreads();
     if (tid < (unsigned)kRadix) {
-        uint32_t run = incl - tot;
-        for (unsigned q = 0; q < wave; ++q) run += wsum[q];
+        uint32_t run = incl - tot, base_d = first_slot + bincl - below;
+        for (unsigned q = 0; q < wave; ++q) {
+            run += wsum[q];
+            base_d += bsum[q];
+        }
+        gbase[tid] = base_d;
         dstart[tid] = run;
 #pragma unroll
         for (int w = 0; w < kSWaves; ++w) {
@@ -326,8 +381,10 @@ __global__ __launch_bounds__(kSThreads) void k_scatter(const float* __restrict__
 template <class KeyOp>
 __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ x, const float* __restrict__ y,
                                               const float* __restrict__ z, uint32_t n, KeyOp op,
-                                              uint32_t* __restrict__ kout, float4* __restrict__ pout) {
+                                              uint32_t* __restrict__ kout, float4* __restrict__ pout,
+                                              uint32_t* __restrict__ zero) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (zero && i == 0) *zero = 0u;
     if (i >= n) return;
     uint32_t k;
     float4 p;
@@ -346,7 +403,7 @@ namespace sortk {
 // (hist) has room for the largest radix.
 template <int RB, class KeyOp>
 void sort_pass(BinWork& w, uint32_t* hist, const float* x, const float* y, const float* z, int64_t n,
-               const KeyOp& op, int p, int passes, int shift, int& kcur, hipStream_t s) {
+               const KeyOp& op, int p, int passes, int shift, int& kcur, uint32_t* zero, hipStream_t s) {
     constexpr int kRadix = 1 << RB;
     const unsigned ntiles = div_up(n, kTile);
     const uint32_t chunk = div_up(ntiles, kMaxChunks);
@@ -360,27 +417,40 @@ void sort_pass(BinWork& w, uint32_t* hist, const float* x, const float* y, const
     if (p == 0) {
         // the keys in input order go to keys[0], which pass 0 does not otherwise use
         hipLaunchKernelGGL((k_hist<RB, true, KeyOp>), dim3(ntiles), dim3(kThreads), 0, s, x, y, z,
-                           (const uint32_t*)nullptr, (uint32_t)n, op, shift, hist, w.keys[0].as<uint32_t>());
+                           (const uint32_t*)nullptr, (uint32_t)n, op, shift, hist, w.keys[0].as<uint32_t>(), zero);
     } else {
         hipLaunchKernelGGL((k_hist<RB, false, KeyOp>), dim3(ntiles), dim3(kThreads), 0, s, x, y, z,
                            (const uint32_t*)w.keys[kcur].as<uint32_t>(), (uint32_t)n, op, shift, hist,
-                           (uint32_t*)nullptr);
+                           (uint32_t*)nullptr, (uint32_t*)nullptr);
     }
-    hipLaunchKernelGGL(k_dig_reduce<RB>, dim3(nchunks), dim3(kRadix), 0, s, (const uint32_t*)hist, ntiles, chunk,
-                       part);
-    hipLaunchKernelGGL(k_dig_scan<RB>, dim3(kRadix / kWave), dim3(1024), 0, s, part, nchunks, dtot);
-    hipLaunchKernelGGL(k_dig_down<RB>, dim3(nchunks), dim3(kRadix), 0, s, hist, ntiles, chunk, (const uint32_t*)part,
-                       (const uint32_t*)dtot);
+    const uint32_t* base = nullptr;  // digit totals for the scatter to scan, or none
+#define LJ_COLUMNS(PER)                                                                                   \
+    hipLaunchKernelGGL((k_dig_columns<RB, PER>), dim3(kRadix / kWave), dim3(1024), 0, s, hist, ntiles, dtot); \
+    base = dtot
+    if (ntiles <= 16 * 2) {
+        LJ_COLUMNS(2);
+    } else if (ntiles <= 16 * 8) {
+        LJ_COLUMNS(8);
+    } else if (ntiles <= 16 * 32) {
+        LJ_COLUMNS(32);
+    } else {
+        hipLaunchKernelGGL(k_dig_reduce<RB>, dim3(nchunks), dim3(kRadix), 0, s, (const uint32_t*)hist, ntiles, chunk,
+                           part);
+        hipLaunchKernelGGL(k_dig_scan<RB>, dim3(kRadix / kWave), dim3(1024), 0, s, part, nchunks, dtot);
+        hipLaunchKernelGGL(k_dig_down<RB>, dim3(nchunks), dim3(kRadix), 0, s, hist, ntiles, chunk,
+                           (const uint32_t*)part, (const uint32_t*)dtot);
+    }
+#undef LJ_COLUMNS
     if (p == 0) {
         // pass 0 reads positions and the stored keys; it writes keys[1]
         hipLaunchKernelGGL((k_scatter<RB, true, KeyOp>), dim3(ntiles), dim3(kSThreads), 0, s, x, y, z,
                            (const uint32_t*)w.keys[0].as<uint32_t>(), (const float4*)nullptr, (uint32_t)n, op,
-                           shift, (const uint32_t*)hist, w.keys[1].as<uint32_t>(), pdst);
+                           shift, (const uint32_t*)hist, base, w.keys[1].as<uint32_t>(), pdst);
         kcur = 1;
     } else {
         hipLaunchKernelGGL((k_scatter<RB, false, KeyOp>), dim3(ntiles), dim3(kSThreads), 0, s, x, y, z,
                            (const uint32_t*)w.keys[kcur].as<uint32_t>(), psrc, (uint32_t)n, op, shift,
-                           (const uint32_t*)hist, w.keys[kdst].as<uint32_t>(), pdst);
+                           (const uint32_t*)hist, base, w.keys[kdst].as<uint32_t>(), pdst);
         kcur = kdst;
     }
 }
@@ -390,7 +460,7 @@ void sort_pass(BinWork& w, uint32_t* hist, const float* x, const float* y, const
 // 9+9+9; the 9-bit digit scan takes 17 us on 16.7M keys where the 8-bit one takes 10).
 template <class KeyOp>
 int sort_passes(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n, const KeyOp& op,
-                int bits, hipStream_t s) {
+                int bits, uint32_t* zero, hipStream_t s) {
     BinWork& w = ctx->bin;
     const unsigned ntiles = div_up(n, kTile);
     int nine = 0, passes = (bits + 7) / 8;
@@ -403,10 +473,10 @@ int sort_passes(lj_context* ctx, const float* x, const float* y, const float* z,
     int kcur = 0, shift = 0;
     for (int p = 0; p < passes; ++p) {
         if (p >= passes - nine) {
-            sort_pass<9>(w, hist, x, y, z, n, op, p, passes, shift, kcur, s);
+            sort_pass<9>(w, hist, x, y, z, n, op, p, passes, shift, kcur, zero, s);
             shift += 9;
         } else {
-            sort_pass<8>(w, hist, x, y, z, n, op, p, passes, shift, kcur, s);
+            sort_pass<8>(w, hist, x, y, z, n, op, p, passes, shift, kcur, zero, s);
             shift += 8;
         }
     }
@@ -420,10 +490,11 @@ int sort_passes(lj_context* ctx, const float* x, const float* y, const float* z,
 // Sorts n particles by op's key (the low `bits` bits).  The sorted keys land in
 // ctx->bin.keys[ctx->bin.cur] and the payload (x, y, z, bits of the original index)
 // in ctx->bin.pos, which has room for n + kPosSpare entries (the spare ones are not
-// written).
+// written).  The first kernel clears *zero (nullable; not when n = 0), a counter that a
+// later kernel of the call adds to.
 template <class KeyOp>
 int sort_particles(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n, const KeyOp& op,
-                   int bits, hipStream_t s) {
+                   int bits, hipStream_t s, uint32_t* zero = nullptr) {
     using namespace sortk;
     BinWork& w = ctx->bin;
     const size_t nn = (size_t)(n > 0 ? n : 1);
@@ -437,11 +508,11 @@ int sort_particles(lj_context* ctx, const float* x, const float* y, const float*
     if (n <= 0) return LJ_OK;
     if (n == 1 || bits == 0) {
         hipLaunchKernelGGL((k_pack<KeyOp>), dim3(div_up(n, 256)), dim3(256), 0, s, x, y, z, (uint32_t)n, op,
-                           w.keys[0].as<uint32_t>(), w.pos.as<float4>());
+                           w.keys[0].as<uint32_t>(), w.pos.as<float4>(), zero);
         LJ_HIP(ctx, hipGetLastError());
         return LJ_OK;
     }
-    return sort_passes(ctx, x, y, z, n, op, bits, s);
+    return sort_passes(ctx, x, y, z, n, op, bits, zero, s);
 }
 
 }  // namespace lj

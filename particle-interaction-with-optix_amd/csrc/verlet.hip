@@ -25,8 +25,8 @@ __global__ __launch_bounds__(256) void k_pack_positions(const float* __restrict_
 
 // kListLanes lanes per particle (row i of the CSR list, caller order), each taking every
 // kListLanes-th entry, kListUnroll of them loaded at once; a workgroup takes `turns` times
-// kListRows rows, one set after the other.  Entries j >= n are ignored.  Per-block FP64
-// energy/virial partials; the listed and accepted pair counts go to res.
+// kListRows rows, one set after the other.  Entries j >= n are ignored.  The workgroup's
+// totals, listed and accepted pairs among them, go to sums.
 // Bound by the partners' gathers, a line each: 500,009 particles at shuffled indices, 36M
 // entries, 366 us (12.6 TB/s of 128-byte lines from the caches).  One lane per row, whose
 // loads of the list touched 64 lines and whose three gathers per entry waited for each
@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ p
                                                     const uint32_t* __restrict__ cols, PairConst c, uint32_t turns,
                                                     float* __restrict__ fx, float* __restrict__ fy,
                                                     float* __restrict__ fz, float* __restrict__ e,
-                                                    double* __restrict__ partials, lj_result* __restrict__ res) {
+                                                    BlockSums* __restrict__ sums) {
     const uint32_t sub = threadIdx.x % kListLanes;
     unsigned long long np = 0, listed = 0;
     double esum = 0.0, vsum = 0.0;
@@ -95,15 +95,7 @@ __global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ p
             vsum += c.e24 * (double)acc.av.value();
         }
     }
-    block_sum2(esum, vsum);
-    const unsigned long long bp = block_sum_u64(np);
-    const unsigned long long bl = block_sum_u64(listed);
-    if (threadIdx.x == 0) {
-        partials[2 * blockIdx.x] = esum;
-        partials[2 * blockIdx.x + 1] = vsum;
-        if (bp) atomicAdd(&res->n_pairs, bp);
-        if (bl) atomicAdd(&res->n_candidates, bl);
-    }
+    store_block_sums<true, true>(&sums[blockIdx.x], esum, vsum, np, listed);
 }
 
 // Largest |p - p0|^2 (FP32, a non-negative float: its bits order like the value).  At
@@ -159,7 +151,6 @@ int lj_compute_list(lj_context* ctx, const float* x, const float* y, const float
         res = ctx->bin.counters.as<lj_result>();
     }
     PhaseTimer tf(ctx, LJ_PHASE_FORCE, s);
-    fill_u64(&res->n_candidates, 2, 0ull, s);
     // up to 8 sets of rows per workgroup once there are workgroups for every CU
     const int64_t sets = div_up(n > 0 ? n : 1, kListRows);
     const uint32_t turns = (uint32_t)(sets < 2048 ? 1 : sets < 16384 ? sets / 2048 : 8);
@@ -167,13 +158,13 @@ int lj_compute_list(lj_context* ctx, const float* x, const float* y, const float
     LJ_HIP(ctx, ctx->bin.pos.grow(((size_t)(n > 0 ? n : 1) + kPosSpare) * sizeof(float4)));
     float4* pos = ctx->bin.pos.as<float4>();
     if (n > 0) hipLaunchKernelGGL(k_pack_positions, dim3(div_up(n, 256)), dim3(256), 0, s, x, y, z, (uint32_t)n, pos);
-    LJ_HIP(ctx, ctx->bin.partials.grow(((size_t)nb + nb / 1024 + 1) * 2 * sizeof(double)));
-    double* partials = ctx->bin.partials.as<double>();
+    BlockSums* sums;
+    LJ_TRY(grow_block_sums(ctx, nb, &sums));
     const bool vir = !(p->flags & LJ_FLAG_NO_VIRIAL);
     const uint32_t nn = (uint32_t)n;
 #define LJ_LF(PRED, PREC, VIR)                                                                                    \
     hipLaunchKernelGGL((k_list_force<PRED, PREC, VIR>), dim3(nb), dim3(256), 0, s, (const float4*)pos, nn, row_offsets, \
-                       cols, c, turns, fx, fy, fz, e, partials, res)
+                       cols, c, turns, fx, fy, fz, e, sums)
 #define LJ_LF_V(PRED, PREC)            \
     do {                               \
         if (vir) LJ_LF(PRED, PREC, true); \
@@ -195,9 +186,7 @@ int lj_compute_list(lj_context* ctx, const float* x, const float* y, const float
 #undef LJ_LF_P
 #undef LJ_LF_V
 #undef LJ_LF
-    finalize_energy(partials, nb, res, s);
-    LJ_HIP(ctx, hipGetLastError());
-    return LJ_OK;
+    return finalize_totals(ctx, nb, nullptr, 0u, nullptr, res, s);
 }
 
 int lj_max_displacement(lj_context* ctx, const float* x, const float* y, const float* z, const float* x0,

@@ -461,3 +461,19 @@ def test_pair_rows_of_every_length_class(engine, lbvh):
         row = cols[rows[i] : rows[i + 1]]
         want = members[group[i]]
         assert np.array_equal(row, want[want != i]), (i, ROW_LENGTHS[group[i]])
+
+
+@pytest.mark.parametrize("cells", [40, 41, 300])
+@pytest.mark.parametrize("n", [2048 * 32, 2048 * 32 + 1, 2048 * 128, 2048 * 128 + 1, 2048 * 512, 2048 * 512 + 1])
+def test_bin_at_the_digit_scan_sizes(engine, n, cells):
+    """Tile counts on both sides of each form of the digit scan (one kernel of 2, 8 and 32
+    tiles a wave, three kernels beyond), with 8-bit digits (40^3 = 64,000 cells, offsets
+    without a list of gaps, and 41^3 = 68,921 with one) and 9-bit ones (300^3 cells)."""
+    x, y, z = ljamd.generate("clusters", n % 1000 + cells, n, [3, 0.1, 0.2, 0.8])
+    p = ljamd.make_params(1.0 / cells)
+    q = po.from_lj(p)
+    off_ref, perm_ref, _ = po.bin(q, x, y, z)
+    off, perm, cand = engine.bin(*engine.to_device(x, y, z), p)
+    assert np.array_equal(off.cpu().numpy().view(np.uint32), off_ref)
+    assert np.array_equal(perm.cpu().numpy().view(np.uint32), perm_ref)
+    assert int(cand.cpu()[0]) == po.candidates(q, off_ref)
