@@ -12,7 +12,7 @@
 #include <vector>
 
 #include "lj_sort.h"
-#include "lj_stencil.h"
+#include "lj_stencil27.h"
 
 namespace lj {
 
@@ -85,10 +85,40 @@ __global__ __launch_bounds__(256) void k_batch_coarse_counts(const uint32_t* __r
     ccount[c] = coarse_count(foff + d.cell_base, d.g, d.cg, Kx, K, c - d.ccell_base);
 }
 
-// 27-cell candidates per system on the cell_edge grids (offsets coff over the
-// concatenated cell_edge cells), ComputeNbInteractions semantics (cudaLJ.cu:255-297),
-// added into cand[system].  A wave's cells usually belong to one system: it then adds
-// its sum with one atomic.
+// 27-cell candidates of the particles in global cell c of system d's cell_edge grid, from
+// the offsets coff over the concatenated cell_edge cells (ComputeNbInteractions
+// semantics, cudaLJ.cu:255-297).
+__device__ inline unsigned long long cell_candidates(const uint32_t* __restrict__ coff, const SysDesc& d, uint32_t c) {
+    const GridGeom& g = d.cg;
+    const uint32_t base = d.ccell_base;
+    const uint32_t c0 = coff[c], c1 = coff[c + 1];
+    int32_t cx, cy, cz;
+    cell_coords(g, c - base, cx, cy, cz);
+    const int32_t gx = g.g[0], gy = g.g[1], gz = g.g[2];
+    const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx < gx - 1 ? cx + 1 : gx - 1;
+    // The nine rows' ranges loaded at once, with no branch between the loads: a row
+    // outside the grid reads the cell's own row and counts zero.  (Loaded row by row
+    // under the bounds tests, the loads went out one row at a time.)
+    uint32_t lo[9], hi[9];
+    bool in[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+        const int32_t zz = cz + q / 3 - 1, yy = cy + q % 3 - 1;
+        in[q] = zz >= 0 && zz < gz && yy >= 0 && yy < gy;
+        const uint32_t row = base + (uint32_t)(((in[q] ? zz : cz) * gy + (in[q] ? yy : cy)) * gx);
+        lo[q] = coff[row + x0];
+        hi[q] = coff[row + x1 + 1];
+    }
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+        if (in[q]) sum += hi[q] - lo[q];
+    const uint32_t nh = c1 - c0;
+    return nh ? (unsigned long long)nh * (sum - 1) : 0ull;
+}
+
+// The candidates of every system, added into cand[system].  A wave's cells usually belong
+// to one system: it then adds its sum with one atomic.
 __global__ __launch_bounds__(256) void k_batch_candidates(const uint32_t* __restrict__ coff, uint32_t nccells,
                                                           const SysDesc* __restrict__ sys,
                                                           const uint32_t* __restrict__ ccbase,
@@ -98,33 +128,8 @@ __global__ __launch_bounds__(256) void k_batch_candidates(const uint32_t* __rest
     uint32_t s = 0xffffffffu;
     unsigned long long v = 0;
     if (c < nccells) {
-        const uint32_t c0 = coff[c], c1 = coff[c + 1];
         s = find_sys(ccbase, cchint, nsys, c);
-        const GridGeom& g = sys[s].cg;
-        const uint32_t base = sys[s].ccell_base;
-        int32_t cx, cy, cz;
-        cell_coords(g, c - base, cx, cy, cz);
-        const int32_t gx = g.g[0], gy = g.g[1], gz = g.g[2];
-        const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx < gx - 1 ? cx + 1 : gx - 1;
-        // The nine rows' ranges loaded at once, with no branch between the loads: a row
-        // outside the grid reads the cell's own row and counts zero.  (Loaded row by row
-        // under the bounds tests, the loads went out one row at a time.)
-        uint32_t lo[9], hi[9];
-        bool in[9];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const int32_t zz = cz + q / 3 - 1, yy = cy + q % 3 - 1;
-            in[q] = zz >= 0 && zz < gz && yy >= 0 && yy < gy;
-            const uint32_t row = base + (uint32_t)(((in[q] ? zz : cz) * gy + (in[q] ? yy : cy)) * gx);
-            lo[q] = coff[row + x0];
-            hi[q] = coff[row + x1 + 1];
-        }
-        unsigned long long sum = 0;
-#pragma unroll
-        for (int q = 0; q < 9; ++q)
-            if (in[q]) sum += hi[q] - lo[q];
-        const uint32_t nh = c1 - c0;
-        if (nh) v = (unsigned long long)nh * (sum - 1);
+        v = cell_candidates(coff, sys[s], c);
     }
     const uint32_t s0 = __shfl(s, 0, kWaveSize);
     if (__all(s == s0 || s == 0xffffffffu)) {
@@ -183,15 +188,16 @@ __device__ inline void batch_pairs(const float4* __restrict__ pos, const uint32_
 // counts (fixed butterfly order) into one WaveTotals.  A wave shared by several
 // systems returns at once; k_batch_force_shared serves it.  A system's sorted slots are
 // the caller's index range [first, first + n) of that system (the key space orders
-// the systems).
+// the systems).  Systems of at most `skip` particles are left out (k_batch_force27 takes
+// them).
 template <int PRED, int PREC, bool QUEUE>
 __global__ __launch_bounds__(kMaxBlock) void k_batch_force(const float4* __restrict__ pos,
                                                            const uint32_t* __restrict__ cell_of,
                                                            const uint32_t* __restrict__ off, uint32_t n,
                                                            const SysDesc* __restrict__ sys,
                                                            const uint32_t* __restrict__ cbase,
-                                                           const uint32_t* __restrict__ chint, uint32_t nsys, int Rx,
-                                                           int R, uint32_t depth, float* __restrict__ fx,
+                                                           const uint32_t* __restrict__ chint, uint32_t nsys, uint32_t skip,
+                                                           int Rx, int R, uint32_t depth, float* __restrict__ fx,
                                                            float* __restrict__ fy, float* __restrict__ fz,
                                                            float* __restrict__ e, WaveTotals* __restrict__ wrec) {
     extern __shared__ QEntry queue[];
@@ -201,7 +207,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_batch_force(const float4* __restr
     const uint32_t si = find_sys(cbase, chint, nsys, key);
     // lane 0 holds the wave's lowest slot: idle only when the whole wave is
     const uint32_t s0 = __builtin_amdgcn_readfirstlane(active ? si : kSharedWave);
-    if (s0 == kSharedWave || !__all(!active || si == s0)) return;
+    if (s0 == kSharedWave || !__all(!active || si == s0) || (skip && sys[s0].n <= skip)) return;
     double ei, vi;
     uint32_t np;
     batch_pairs<PRED, PREC, QUEUE>(pos, off, k, active, key, sys[s0], Rx, R, depth,
@@ -219,17 +225,19 @@ template <int PRED, int PREC, bool QUEUE>
 __global__ __launch_bounds__(kWaveSize) void k_batch_force_shared(
     const float4* __restrict__ pos, const uint32_t* __restrict__ cell_of, const uint32_t* __restrict__ off, uint32_t n,
     const SysDesc* __restrict__ sys, const uint32_t* __restrict__ cbase, const uint32_t* __restrict__ chint,
-    uint32_t nsys, const uint32_t* __restrict__ shared_waves, int Rx, int R, uint32_t depth, float* __restrict__ fx,
+    uint32_t nsys, uint32_t skip, const uint32_t* __restrict__ shared_waves, int Rx, int R, uint32_t depth,
+    float* __restrict__ fx,
     float* __restrict__ fy, float* __restrict__ fz, float* __restrict__ e, double2* __restrict__ ev,
     uint32_t* __restrict__ npair, WaveTotals* __restrict__ wrec) {
     extern __shared__ QEntry queue[];
     const uint32_t w = shared_waves[blockIdx.x];
     const uint32_t k = w * kWaveSize + threadIdx.x;
-    const bool active = k < n;
-    const uint32_t key = active ? cell_of[k] : 0u;
+    const uint32_t key = k < n ? cell_of[k] : 0u;
+    const SysDesc& d = sys[find_sys(cbase, chint, nsys, key)];
+    const bool active = k < n && d.n > skip;
     double ei, vi;
     uint32_t np;
-    batch_pairs<PRED, PREC, QUEUE>(pos, off, k, active, key, sys[find_sys(cbase, chint, nsys, key)], Rx, R, depth,
+    batch_pairs<PRED, PREC, QUEUE>(pos, off, k, active, key, d, Rx, R, depth,
                                    queue + (threadIdx.x / kWaveSize) * depth * kWaveSize + __lane_id(), fx, fy, fz, e,
                                    ei, vi, np);
     if (active) {
@@ -239,20 +247,93 @@ __global__ __launch_bounds__(kWaveSize) void k_batch_force_shared(
     if (threadIdx.x == 0) wrec[w] = WaveTotals{0.0, 0.0, 0ull, kSharedWave, 0u};
 }
 
+// The systems that two_lanes takes (at most `most` particles): two lanes per particle, 32
+// sorted slots per wave.  A wave that holds slots of several systems takes them one after
+// the other, each with its constants in scalar registers, and keeps their values per slot,
+// as the waves of k_batch_force_shared do.
+// Up to this many cells of a batch are counted in the final reduction, one workgroup a
+// system; beyond, on the second stream beside the force pass (4,096 systems of 12.8M
+// cells: 138 us that the force pass's tail hides).
+constexpr uint64_t kReduceCells = 1u << 20;
+constexpr uint32_t kWaveSlots27 = kWaveSize / kPairLanes;
+
+template <int PRED, int PREC>
+__global__ __launch_bounds__(kMaxBlock, 8) void k_batch_force27(
+    const float4* __restrict__ pos, const uint32_t* __restrict__ cell_of, const uint32_t* __restrict__ off, uint32_t n,
+    const SysDesc* __restrict__ sys, const uint32_t* __restrict__ cbase, const uint32_t* __restrict__ chint,
+    uint32_t nsys, uint32_t most, float* __restrict__ fx, float* __restrict__ fy, float* __restrict__ fz,
+    float* __restrict__ e, double2* __restrict__ ev, uint32_t* __restrict__ npair, WaveTotals* __restrict__ wrec) {
+    const uint32_t k = (xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) / kPairLanes;
+    const bool live = k < n;
+    const uint32_t gkey = live ? cell_of[k] : 0xffffffffu;
+    const uint64_t all = __ballot(live);
+    // The keys ascend, so the slots of one system are consecutive lanes: the search for a
+    // system is wave-uniform (scalar loads), and its end tells which lanes it holds.
+    // Nothing per lane but k and the key is live across a turn (64 VGPRs are the budget).
+    for (uint64_t left = all; left;) {
+        const uint32_t s0 = find_sys(cbase, chint, nsys, __builtin_amdgcn_readlane(gkey, __builtin_ctzll(left)));
+        const uint32_t last = s0 + 1u < nsys ? cbase[s0 + 1u] : 0xffffffffu;
+        const uint64_t m = __ballot(gkey < last) & left;
+        const bool mine = (m >> __lane_id()) & 1u;
+        left &= ~m;
+        const SysDesc& d = sys[s0];
+        if (d.n > most) continue;
+        const float4 pi = mine ? pos[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const uint32_t key = mine ? gkey - d.cell_base : 0u;
+        const PairConst c = d.c;
+        PairSums<PREC, PRED == LJ_PRED_CUDALJ, true> acc;
+        acc.set_i(pi);
+        acc.allow_exact_diff(c, pi, mine);
+        const uint32_t np = stencil27<PRED>(pos, off, k, mine, pi, d.g, d.cell_base, key, d.tr, c, acc);
+        acc.template merge<kPairLanes>();
+        const bool first = mine && (__lane_id() & 1u) == 0u;
+        double ei = 0.0, vi = 0.0;
+        if (first) {
+            const uint32_t i = __float_as_uint(pos[k].w);
+            fx[i] = (float)(-c.e24 * (double)acc.ax.value());
+            fy[i] = (float)(-c.e24 * (double)acc.ay.value());
+            fz[i] = (float)(-c.e24 * (double)acc.az.value());
+            ei = c.e4 * (double)acc.ae.value();
+            if (e) e[i] = (float)ei;
+            vi = c.e24 * (double)acc.av.value();
+        }
+        if (m == all) {  // the wave's only system
+            // (a system of at most 2^20 particles: 64 lanes' pairs fit 32 bits)
+            const double es = wave_sum(ei), vs = wave_sum(vi);
+            const uint32_t ns = wave_sum(np);
+            if (__lane_id() == 0) wrec[k / kWaveSlots27] = WaveTotals{es, vs, ns, s0, 0u};
+        } else {
+            const uint32_t both = np + dpp_of<1>(np);
+            if (first) {
+                ev[k] = make_double2(ei, vi);
+                npair[k] = both;
+                wrec[k / kWaveSlots27].sys = kSharedWave;
+            }
+        }
+    }
+}
+
 // One block per system: FP64 totals over its waves in slot order -- the WaveTotals of
 // the waves it fills alone, the per-slot values of its slots in the (at most two)
-// waves it shares with other systems -- and its candidate count from cand.
+// waves it shares with other systems -- and its candidate count, from cand or, when cand
+// is NULL, counted here from the offsets coff (small batches on the cell_edge grid: one
+// launch less, and no second stream to fork and join, which took 20 us).
+// wrec27: the records of the systems of at most `most` particles.
 __global__ __launch_bounds__(256) void k_batch_reduce(const SysDesc* __restrict__ sys,
-                                                      const WaveTotals* __restrict__ wrec,
+                                                      const WaveTotals* __restrict__ wrec1,
+                                                      const WaveTotals* __restrict__ wrec27, uint32_t most,
                                                       const double2* __restrict__ ev,
                                                       const uint32_t* __restrict__ npair,
                                                       const unsigned long long* __restrict__ cand,
-                                                      lj_result* __restrict__ res) {
+                                                      const uint32_t* __restrict__ coff, lj_result* __restrict__ res) {
     const SysDesc& d = sys[blockIdx.x];
+    const bool two = d.n <= most;
+    const uint32_t slots = two ? kWaveSlots27 : (uint32_t)kWaveSize;  // of a record
+    const WaveTotals* const wrec = two ? wrec27 : wrec1;
     double a = 0.0, b = 0.0;
-    unsigned long long np = 0;
+    unsigned long long np = 0, nc = 0;
     if (d.n) {
-        const uint32_t w0 = d.first / kWaveSize, w1 = (d.first + d.n - 1) / kWaveSize;
+        const uint32_t w0 = d.first / slots, w1 = (d.first + d.n - 1) / slots;
         for (uint32_t w = w0 + threadIdx.x; w <= w1; w += 256) {
             const WaveTotals r = wrec[w];
             if (r.sys != kSharedWave) {
@@ -260,8 +341,8 @@ __global__ __launch_bounds__(256) void k_batch_reduce(const SysDesc* __restrict_
                 b += r.v;
                 np += r.np;
             } else {
-                const uint32_t lo = d.first > w * kWaveSize ? d.first : w * kWaveSize;
-                const uint32_t hi = d.first + d.n < (w + 1) * kWaveSize ? d.first + d.n : (w + 1) * kWaveSize;
+                const uint32_t lo = d.first > w * slots ? d.first : w * slots;
+                const uint32_t hi = d.first + d.n < (w + 1) * slots ? d.first + d.n : (w + 1) * slots;
                 for (uint32_t q = lo; q < hi; ++q) {
                     const double2 t = ev[q];
                     a += t.x;
@@ -270,15 +351,13 @@ __global__ __launch_bounds__(256) void k_batch_reduce(const SysDesc* __restrict_
                 }
             }
         }
+        if (!cand)
+            for (uint32_t c = threadIdx.x; c < d.cg.ncells; c += 256) nc += cell_candidates(coff, d, d.ccell_base + c);
     }
-    block_sum2(a, b);
-    const unsigned long long t = block_sum_u64(np);
-    if (threadIdx.x == 0) {
-        res[blockIdx.x].e_total = 0.5 * a;
-        res[blockIdx.x].virial = 0.5 * b;
-        res[blockIdx.x].n_pairs = t;
-        res[blockIdx.x].n_candidates = cand[blockIdx.x];
-    }
+    __shared__ BlockSums total;
+    store_block_sums<true, true>(&total, a, b, np, nc);
+    if (threadIdx.x == 0)
+        res[blockIdx.x] = lj_result{0.5 * total.e, 0.5 * total.v, cand ? cand[blockIdx.x] : total.nc, total.np};
 }
 
 }  // namespace
@@ -406,7 +485,15 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     const size_t nn = (size_t)(n > 0 ? n : 1);
     LJ_HIP(ctx, W.ev.grow(nn * sizeof(double2)));
     LJ_HIP(ctx, W.npair.grow(nn * sizeof(uint32_t)));
-    LJ_HIP(ctx, W.wrec.grow(div_up(nn, (size_t)kWaveSize) * sizeof(WaveTotals)));
+    // which systems take two lanes a particle, and the records of each kind of wave
+    bool any_one = false, any_two = false;
+    for (int32_t q = 0; q < nsys; ++q) {
+        if (!sys[q].n) continue;
+        (two_lanes(sh, sys[q].n) ? any_two : any_one) = true;
+    }
+    const uint32_t most = two_lanes(sh, 0) ? (uint32_t)kTwoLaneMax : 0u;
+    const size_t nrec = div_up((int64_t)nn, kWaveSize);
+    LJ_HIP(ctx, W.wrec.grow((nrec + div_up((int64_t)nn, kWaveSlots27)) * sizeof(WaveTotals)));
     uint32_t* off;
     {
         PhaseTimer tb(ctx, LJ_PHASE_BIN, s);
@@ -421,9 +508,12 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     // The candidate counts need only the cell offsets: they run on the context's second
     // stream beside the force pass, into an array of their own that the final
     // reduction copies into the results after the join.
-    LJ_HIP(ctx, W.cand.grow((size_t)nsys * sizeof(unsigned long long)));
-    unsigned long long* cand = W.cand.as<unsigned long long>();
-    {
+    // Small batches whose cell_edge cells are the force grid's count in the reduction.
+    const bool fork = sh.refine > 1 || sh.refine_x > 1 || cctot > kReduceCells;
+    unsigned long long* cand = nullptr;
+    if (fork) {
+        LJ_HIP(ctx, W.cand.grow((size_t)nsys * sizeof(unsigned long long)));
+        cand = W.cand.as<unsigned long long>();
         const hipStream_t sc = ctx->aux;
         LJ_HIP(ctx, hipEventRecord(ctx->ev_fork, s));
         LJ_HIP(ctx, hipStreamWaitEvent(sc, ctx->ev_fork, 0));
@@ -446,29 +536,36 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     double2* ev = W.ev.as<double2>();
     uint32_t* npair = W.npair.as<uint32_t>();
     WaveTotals* wrec = W.wrec.as<WaveTotals>();
+    WaveTotals* wrec27 = wrec + nrec;
     const float4* pos = B.pos.as<float4>();
     const uint32_t* cell_of = B.sorted_keys();
     {
         PhaseTimer tf(ctx, LJ_PHASE_FORCE, s);
-        const unsigned nb = div_up(n, sh.block);
+        const unsigned nb = div_up(n, sh.block), nb27 = div_up(n * kPairLanes, sh.block);
         const size_t lds = sh.lds_bytes();
         const size_t lds_shared = sh.queued() ? (size_t)sh.depth * kWaveSize * sizeof(QEntry) : 0;
         if (n > 0) {
 #define LJ_BFQ(PRED, PREC, Q)                                                                                     \
     do {                                                                                                          \
         hipLaunchKernelGGL((k_batch_force<PRED, PREC, Q>), dim3(nb), dim3(sh.block), lds, s, pos, cell_of,        \
-                           (const uint32_t*)off, (uint32_t)n, dsys, dcbase, hcbase, (uint32_t)nsys, sh.refine_x,    \
+                           (const uint32_t*)off, (uint32_t)n, dsys, dcbase, hcbase, (uint32_t)nsys, most, sh.refine_x, \
                            sh.refine, (uint32_t)sh.depth, fx, fy, fz, e, wrec);                                     \
         if (!shared.empty())                                                                                      \
             hipLaunchKernelGGL((k_batch_force_shared<PRED, PREC, Q>), dim3((unsigned)shared.size()),              \
                                dim3(kWaveSize), lds_shared, s, pos, cell_of, (const uint32_t*)off, (uint32_t)n,    \
-                               dsys, dcbase, hcbase, (uint32_t)nsys, dshared, sh.refine_x, sh.refine,              \
+                               dsys, dcbase, hcbase, (uint32_t)nsys, most, dshared, sh.refine_x, sh.refine,        \
                                (uint32_t)sh.depth, fx, fy, fz, e, ev, npair, wrec);                                 \
     } while (0)
-#define LJ_BF(PRED, PREC)                          \
-    do {                                           \
-        if (sh.queued()) LJ_BFQ(PRED, PREC, true); \
-        else LJ_BFQ(PRED, PREC, false);            \
+#define LJ_BF(PRED, PREC)                                                                                          \
+    do {                                                                                                           \
+        if (any_two)                                                                                               \
+            hipLaunchKernelGGL((k_batch_force27<PRED, PREC>), dim3(nb27), dim3(sh.block), 0, s, pos, cell_of,      \
+                               (const uint32_t*)off, (uint32_t)n, dsys, dcbase, hcbase, (uint32_t)nsys, most, fx, fy, \
+                               fz, e, ev, npair, wrec27);                                                          \
+        if (any_one) {                                                                                             \
+            if (sh.queued()) LJ_BFQ(PRED, PREC, true);                                                             \
+            else LJ_BFQ(PRED, PREC, false);                                                                        \
+        }                                                                                                          \
     } while (0)
 #define LJ_BF_PREC(PRED)                                   \
     switch (p0.precision) {                                \
@@ -490,9 +587,10 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     }
     {
         PhaseTimer to(ctx, LJ_PHASE_OTHER, s);
-        LJ_HIP(ctx, hipStreamWaitEvent(s, ctx->ev_join, 0));
+        if (fork) LJ_HIP(ctx, hipStreamWaitEvent(s, ctx->ev_join, 0));
         hipLaunchKernelGGL(k_batch_reduce, dim3((unsigned)nsys), dim3(256), 0, s, dsys, (const WaveTotals*)wrec,
-                           (const double2*)ev, (const uint32_t*)npair, (const unsigned long long*)cand, results);
+                           (const WaveTotals*)wrec27, most, (const double2*)ev, (const uint32_t*)npair,
+                           (const unsigned long long*)cand, (const uint32_t*)off, results);
     }
     LJ_HIP(ctx, hipGetLastError());
     return LJ_OK;

@@ -16,7 +16,7 @@
 #include "lj_candidates.h"
 #include "lj_rows.h"
 #include "lj_sort.h"
-#include "lj_stencil.h"
+#include "lj_stencil27.h"
 
 namespace lj {
 
@@ -27,9 +27,7 @@ namespace {
 // without QUEUE).  Outputs go to the caller's order (pi.w holds the original index),
 // or, when `so` is set (lj_compute_sorted), to the sorted slot k together with the
 // particle's position and original index; each workgroup's totals go to sums and are
-// reduced later in a fixed order.  The workgroups past the first nforce count the 27-cell
-// candidates of the same grid instead (none when they are not wanted or belong to another
-// grid): they need only the offsets, and a launch of their own costs 4-5 us.
+// reduced later in a fixed order.
 // OUT: how the outputs are stored -- 0 ordinary stores, 1 non-temporal stores, 2 one
 // non-temporal staged record per particle at its caller index (large outputs at
 // shuffled indices; never with `so`).
@@ -38,18 +36,10 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force(const float4* __restrict
                                                      const uint32_t* __restrict__ off, uint32_t n, GridGeom g, int Rx,
                                                      int R, Trim tr, PairConst c, uint32_t depth, float* __restrict__ fx,
                                                      float* __restrict__ fy, float* __restrict__ fz,
-                                                     float* __restrict__ e, uint32_t nforce,
-                                                     BlockSums* __restrict__ sums, SortedOut so,
+                                                     float* __restrict__ e, BlockSums* __restrict__ sums, SortedOut so,
                                                      float4* __restrict__ stage) {
     extern __shared__ QEntry queue[];
-    if (blockIdx.x >= nforce) {
-        const uint32_t waves = blockDim.x / kWaveSize;
-        const uint32_t wave = (blockIdx.x - nforce) * waves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
-        const unsigned long long nc = candidate_rows(off, g, wave, (gridDim.x - nforce) * waves);
-        store_block_sums<false, true>(&sums[blockIdx.x], 0.0, 0.0, 0ull, nc);
-        return;
-    }
-    const uint32_t blk = xcd_block(blockIdx.x, nforce);
+    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t k = blk * blockDim.x + threadIdx.x;
     // the slot rebuilt after the pair loop from wave-uniform values and the lane id, so
     // that no per-lane index stays live across it (64 VGPRs are the budget)
@@ -90,6 +80,57 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force(const float4* __restrict
             store_out<NT>(&fz[i], oz);
             if (e) store_out<NT>(&e[i], (float)ei);
         }
+        esum = ei;
+        vsum = c.e24 * (double)acc.av.value();
+    }
+    store_block_sums<true, false>(&sums[blk], esum, vsum, np, 0ull);
+}
+
+// The same for systems that two_lanes takes: two lanes per particle (stencil27), outputs
+// (which fit in the L2s) stored ordinarily.  The workgroups past the first nforce count the
+// 27-cell candidates of the same grid (none when no result is wanted): they need only the
+// offsets, and a launch of their own costs 4-5 us.
+template <int PRED, int PREC, bool VIR>
+__global__ __launch_bounds__(kMaxBlock, 8) void k_force27(const float4* __restrict__ pos,
+                                                      const uint32_t* __restrict__ cell_of,
+                                                      const uint32_t* __restrict__ off, uint32_t n, GridGeom g, Trim tr,
+                                                      PairConst c, float* __restrict__ fx, float* __restrict__ fy,
+                                                      float* __restrict__ fz, float* __restrict__ e, uint32_t nforce,
+                                                      BlockSums* __restrict__ sums, SortedOut so) {
+    if (blockIdx.x >= nforce) {
+        const uint32_t waves = blockDim.x / kWaveSize;
+        const uint32_t wave = (blockIdx.x - nforce) * waves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+        const unsigned long long nc = candidate_rows(off, g, wave, (gridDim.x - nforce) * waves);
+        store_block_sums<false, true>(&sums[blockIdx.x], 0.0, 0.0, 0ull, nc);
+        return;
+    }
+    const uint32_t blk = xcd_block(blockIdx.x, nforce);
+    const uint32_t k = (blk * blockDim.x + threadIdx.x) / kPairLanes;
+    const uint32_t wbase = (blk * blockDim.x + (__builtin_amdgcn_readfirstlane(threadIdx.x) & ~(kWaveSize - 1u))) / kPairLanes;
+    const bool active = k < n;
+    PairSums<PREC, PRED == LJ_PRED_CUDALJ, VIR> acc;
+    const float4 pi = active ? pos[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+    acc.set_i(pi);
+    acc.allow_exact_diff(c, pi, active);
+    const uint32_t np = stencil27<PRED>(pos, off, k, active, pi, g, 0u, active ? cell_of[k] : 0u, tr, c, acc);
+    acc.template merge<kPairLanes>();
+    double esum = 0.0, vsum = 0.0;
+    const uint32_t ks = wbase + __lane_id() / kPairLanes;  // = k
+    if (ks < n && (__lane_id() & 1u) == 0u) {
+        const float4 ps = pos[ks];
+        const double ei = c.e4 * (double)acc.ae.value();
+        const bool sorted = so.x != nullptr;  // uniform
+        const uint32_t i = sorted ? ks : __float_as_uint(ps.w);
+        if (sorted) {
+            so.x[ks] = ps.x;
+            so.y[ks] = ps.y;
+            so.z[ks] = ps.z;
+            if (so.perm) so.perm[ks] = __float_as_uint(ps.w);
+        }
+        fx[i] = (float)(-c.e24 * (double)acc.ax.value());
+        fy[i] = (float)(-c.e24 * (double)acc.ay.value());
+        fz[i] = (float)(-c.e24 * (double)acc.az.value());
+        if (e) e[i] = (float)ei;
         esum = ei;
         vsum = c.e24 * (double)acc.av.value();
     }
@@ -362,9 +403,22 @@ void launch_force(int prec, bool vir, const Shape& sh, unsigned nb, hipStream_t 
                   const SortedOut& so, float4* stage) {
     const size_t lds = sh.lds_bytes();
     const int out = stage ? 2 : non_temporal_outputs(n) ? 1 : 0;
+    if (two_lanes(sh, n)) {
+        // (`depth` has no effect: there is no queue)
+#define LJ_L27(PREC, VIR)                                                                                                  \
+    hipLaunchKernelGGL((k_force27<PRED, PREC, VIR>), dim3(nb), dim3(sh.block), 0, s, pos, cell_of, off, n, g, tr, c, fx, fy, \
+                       fz, e, nforce, sums, so)
+        switch (prec) {
+        case LJ_PREC_MIXED: if (vir) LJ_L27(LJ_PREC_MIXED, true); else LJ_L27(LJ_PREC_MIXED, false); break;
+        case LJ_PREC_FP32: if (vir) LJ_L27(LJ_PREC_FP32, true); else LJ_L27(LJ_PREC_FP32, false); break;
+        default: if (vir) LJ_L27(LJ_PREC_FP32_COMP, true); else LJ_L27(LJ_PREC_FP32_COMP, false); break;
+        }
+#undef LJ_L27
+        return;
+    }
 #define LJ_LAUNCH_QN(PREC, VIR, Q, OUT)                                                                              \
     hipLaunchKernelGGL((k_force<PRED, PREC, VIR, Q, OUT>), dim3(nb), dim3(sh.block), lds, s, pos, cell_of, off, n, g, \
-                       sh.refine_x, sh.refine, tr, c, (uint32_t)sh.depth, fx, fy, fz, e, nforce, sums, so, stage)
+                       sh.refine_x, sh.refine, tr, c, (uint32_t)sh.depth, fx, fy, fz, e, sums, so, stage)
 #define LJ_LAUNCH_Q(PREC, VIR, Q)                      \
     do {                                               \
         if (out == 2) LJ_LAUNCH_QN(PREC, VIR, Q, 2);   \
@@ -509,11 +563,16 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
     LJ_TRY(result_slot(ctx, result, &res));
     // The candidate count, on the cell_edge grid (ComputeNbInteractions semantics), is
     // only made for a caller that takes the results: by further workgroups of the force
-    // launch when that grid is the force grid, else from cell_edge offsets of its own.
-    const unsigned nforce = div_up(n > 0 ? n : 1, sh.block);
+    // launch (two lanes a particle), else before it, on a refined grid from cell_edge
+    // offsets of its own.
+    const unsigned nforce = div_up((n > 0 ? n : 1) * (two_lanes(sh, n) ? kPairLanes : 1), sh.block);
     unsigned ncount = 0, nparts = 0;
-    if (result && !refined) ncount = candidate_blocks(g);
-    if (result && refined) {
+    if (result && two_lanes(sh, n)) {
+        ncount = candidate_blocks(g);
+    } else if (result && !refined) {
+        PhaseTimer t(ctx, LJ_PHASE_OTHER, s);
+        LJ_TRY(candidate_parts(ctx, g, ctx->bin.offsets.as<uint32_t>(), &nparts, s));
+    } else if (result) {
         PhaseTimer t(ctx, LJ_PHASE_OTHER, s);
         BinWork& w = ctx->bin;
         LJ_HIP(ctx, w.ccounts.grow((size_t)g.ncells * 4));

@@ -86,7 +86,7 @@ struct Status {
 
 // Workspace of one binned system (or of a concatenated batch).
 // Entries past the last sorted particle in BinWork::pos (never written, read but unused).
-constexpr int kPosSpare = 3;
+constexpr int kPosSpare = 8;
 
 struct BinWork {
     DevBuf keys[2];      // u32 radix keys (ping-pong)

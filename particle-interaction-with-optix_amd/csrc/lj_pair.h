@@ -9,6 +9,25 @@ namespace lj {
 
 constexpr int kWaveSize = 64;
 
+// The value of the lane that lane ^ d is (d = 1, 2: quad_perm) or of its mirror image in 8
+// (d = 7) or 16 lanes (d = 15), by data-parallel moves: no LDS access and no wait.
+template <int D>
+__device__ inline uint32_t dpp_xor(uint32_t v) {
+    constexpr int kCtrl = D == 1 ? 0xB1 : D == 2 ? 0x4E : D == 7 ? 0x141 : 0x140;
+    static_assert(D == 1 || D == 2 || D == 7 || D == 15, "lane exchanges that DPP has");
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, true);
+}
+template <int D, class T>
+__device__ inline T dpp_of(T v) {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two registers");
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, dpp_xor<D>(__builtin_bit_cast(uint32_t, v)));
+    } else {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        return __builtin_bit_cast(T, (uint64_t)dpp_xor<D>((uint32_t)(u >> 32)) << 32 | dpp_xor<D>((uint32_t)u));
+    }
+}
+
 // Per-particle accumulators of one precision mode (LJ_PREC_*).
 //   MIXED      FP64 sums of FP64 pair terms
 //   FP32       plain FP32 sums
@@ -23,8 +42,9 @@ struct Acc<LJ_PREC_MIXED> {
     __device__ inline void add(double v) { s += v; }
     __device__ inline void fma(double a, double b) { s = __builtin_fma(a, b, s); }
     __device__ inline double value() const { return s; }
-    // adds the sum of the lane `d` away (both lanes then hold the two lanes' sum)
-    __device__ inline void merge_xor(int d) { s += __shfl_xor(s, d, kWaveSize); }
+    // adds the sum of the lane that dpp_xor<D> names (both then hold the two lanes' sum)
+    template <int D>
+    __device__ inline void merge_dpp() { s += dpp_of<D>(s); }
 };
 
 template <>
@@ -33,7 +53,8 @@ struct Acc<LJ_PREC_FP32> {
     __device__ inline void add(float v) { s += v; }
     __device__ inline void fma(float a, float b) { s = __builtin_fmaf(a, b, s); }
     __device__ inline float value() const { return s; }
-    __device__ inline void merge_xor(int d) { s += __shfl_xor(s, d, kWaveSize); }
+    template <int D>
+    __device__ inline void merge_dpp() { s += dpp_of<D>(s); }
 };
 
 template <>
@@ -47,8 +68,9 @@ struct Acc<LJ_PREC_FP32_COMP> {
     }
     __device__ inline void fma(float a, float b) { add(a * b); }
     __device__ inline float value() const { return s + c; }
-    __device__ inline void merge_xor(int d) {
-        const float os = __shfl_xor(s, d, kWaveSize), oc = __shfl_xor(c, d, kWaveSize);
+    template <int D>
+    __device__ inline void merge_dpp() {
+        const float os = dpp_of<D>(s), oc = dpp_of<D>(c);
         add(os);
         c += oc;
     }
@@ -81,15 +103,21 @@ struct PairSums {
         py = pi.y;
         pz = pi.z;
     }
-    // Sums over groups of `lanes` neighbouring lanes (a power of two), left in each of them.
-    __device__ inline void merge(int lanes) {
-        for (int d = 1; d < lanes; d <<= 1) {
-            ax.merge_xor(d);
-            ay.merge_xor(d);
-            az.merge_xor(d);
-            ae.merge_xor(d);
-            if constexpr (VIR) av.merge_xor(d);
-        }
+    // Sums over groups of LANES (2, 4 or 8) neighbouring lanes, left in each of them.
+    template <int D>
+    __device__ inline void merge_step() {
+        ax.template merge_dpp<D>();
+        ay.template merge_dpp<D>();
+        az.template merge_dpp<D>();
+        ae.template merge_dpp<D>();
+        if constexpr (VIR) av.template merge_dpp<D>();
+    }
+    template <int LANES>
+    __device__ inline void merge() {
+        static_assert(LANES == 2 || LANES == 4 || LANES == 8, "lanes of a particle");
+        merge_step<1>();
+        if constexpr (LANES > 2) merge_step<2>();
+        if constexpr (LANES > 4) merge_step<7>();
     }
     // Accepted partners of a cutoff predicate lie within rc of p_i on every axis.  If
     // |p_i| >= 2 rc on every axis (so p_j has the sign of p_i and lies in [p_i/2, 2 p_i]),
@@ -191,48 +219,16 @@ __device__ inline void store_staged(float4* p, float a, float b, float c, float 
     __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
 }
 
+// The wave's sum, in every lane: inside 16 lanes by DPP, then across.
 template <class T>
 __device__ inline T wave_sum(T v) {
-#pragma unroll
-    for (int d = kWaveSize / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, kWaveSize);
+    v += dpp_of<1>(v);
+    v += dpp_of<2>(v);
+    v += dpp_of<7>(v);
+    v += dpp_of<15>(v);
+    v += __shfl_xor(v, 16, kWaveSize);
+    v += __shfl_xor(v, 32, kWaveSize);
     return v;
-}
-
-// Blocks of up to 256 threads (a whole number of waves): deterministic tree sum of two
-// doubles; thread 0 holds the result.  Every thread must call it; the closing barrier
-// lets a block call it again (its LDS slots are reused).
-__device__ inline void block_sum2(double& a, double& b) {
-    __shared__ double sh[2][256 / kWaveSize];
-    a = wave_sum(a);
-    b = wave_sum(b);
-    const unsigned w = threadIdx.x / kWaveSize;
-    if (__lane_id() == 0) {
-        sh[0][w] = a;
-        sh[1][w] = b;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        a = 0.0;
-        b = 0.0;
-        for (unsigned q = 0; q < blockDim.x / kWaveSize; ++q) {
-            a += sh[0][q];
-            b += sh[1][q];
-        }
-    }
-    __syncthreads();
-}
-
-// Sum over the block (thread 0 holds it), callable repeatedly like block_sum2.
-__device__ inline unsigned long long block_sum_u64(unsigned long long v) {
-    __shared__ unsigned long long sh[256 / kWaveSize];
-    v = wave_sum(v);
-    if (__lane_id() == 0) sh[threadIdx.x / kWaveSize] = v;
-    __syncthreads();
-    unsigned long long t = 0;
-    if (threadIdx.x == 0)
-        for (unsigned q = 0; q < blockDim.x / kWaveSize; ++q) t += sh[q];
-    __syncthreads();
-    return t;
 }
 
 // What one workgroup adds to a call's totals: energy, virial, accepted and candidate

@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ p
                 acc.add(c, pj[u], dx, dy, dz, d2, mult);
             }
         }
-        acc.merge(kListLanes);
+        acc.template merge<kListLanes>();
         if (active && sub == 0) {
             fx[i] = (float)(-c.e24 * (double)acc.ax.value());
             fy[i] = (float)(-c.e24 * (double)acc.ay.value());

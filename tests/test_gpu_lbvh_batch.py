@@ -331,3 +331,55 @@ def test_batched_rejects_unpacked_systems(engine):
     dx, dy, dz = engine.to_device(X, Y, Z)
     with pytest.raises(ljamd.LJError):
         engine.compute_batched(systems, dx, dy, dz)
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp32", "fp32_comp"])
+@pytest.mark.parametrize("pred", ["aabb", "custom", "cudalj", "sphere", "triangle"])
+def test_batch_of_small_systems_equals_single_calls(engine, pred, prec):
+    """Two lanes a particle, 32 slots a wave: systems that end on, before and after a wave's
+    edge, several in one wave, empty ones, and one above them all; every predicate and
+    precision.  Each system's outputs are those of its own call, bit for bit, and its
+    counts; the totals agree to the order of the sums."""
+    sizes = [1, 31, 32, 33, 0, 2, 3, 64, 1, 1, 0, 127, 128, 130, 4000, 5]
+    systems, parts, first = [], [], 0
+    for s, n in enumerate(sizes):
+        parts.append(ljamd.generate("uniform", 900 + s, n) if n else (np.zeros(0, np.float32),) * 3)
+        p = ljamd.make_params(0.3 if n < 1000 else 0.1, predicate=pred, precision=prec, softening2=1e-5 if pred == "cudalj" else 0.0)
+        systems.append(ljamd.LJSystem(first, n, p))
+        first += n
+    d = engine.to_device(*(np.concatenate([q[i] for q in parts]).astype(np.float32) for i in range(3)))
+    out = engine.compute_batched(systems, *d)
+    res = ljamd.read_results(out["result"], len(systems))
+    for s, sy in enumerate(systems):
+        a, b = sy.first, sy.first + sy.n
+        one = engine.compute(*(v[a:b] for v in d), sy.params)
+        r1 = ljamd.read_results(one["result"])[0]
+        for k in ("fx", "fy", "fz", "e"):
+            got, want = out[k][a:b].view(engine.torch.int32), one[k][: sy.n].view(engine.torch.int32)
+            assert engine.torch.equal(got, want), (s, k)
+        assert int(r1["n_pairs"]) == int(res[s]["n_pairs"]) and int(r1["n_candidates"]) == int(res[s]["n_candidates"]), s
+        for k in ("e_total", "virial"):
+            assert float(res[s][k]) == pytest.approx(float(r1[k]), rel=1e-12, abs=1e-300, nan_ok=True), (s, k)
+
+
+def test_batch_across_the_two_lane_limit(engine):
+    """A batch with a system of 2^20 + 1 particles (one lane a particle, 64 slots a wave)
+    between systems of two lanes: the waves that both kinds share keep each system's own
+    values, and every system equals its own call."""
+    sizes = [1000, (1 << 20) + 1, 333]
+    systems, parts, first = [], [], 0
+    for s, n in enumerate(sizes):
+        parts.append(ljamd.generate("uniform", 950 + s, n))
+        systems.append(ljamd.LJSystem(first, n, ljamd.make_params(0.2 if n < 2000 else 0.015, refine=1, refine_x=1)))
+        first += n
+    d = engine.to_device(*(np.concatenate([q[i] for q in parts]) for i in range(3)))
+    out = engine.compute_batched(systems, *d)
+    res = ljamd.read_results(out["result"], len(systems))
+    for s, sy in enumerate(systems):
+        a, b = sy.first, sy.first + sy.n
+        one = engine.compute(*(v[a:b] for v in d), sy.params)
+        r1 = ljamd.read_results(one["result"])[0]
+        for k in ("fx", "fy", "fz", "e"):
+            assert engine.torch.equal(out[k][a:b].view(engine.torch.int32), one[k][: sy.n].view(engine.torch.int32)), (s, k)
+        assert int(r1["n_pairs"]) == int(res[s]["n_pairs"]) and int(r1["n_candidates"]) == int(res[s]["n_candidates"]), s
+        assert float(res[s]["e_total"]) == pytest.approx(float(r1["e_total"]), rel=1e-12)
