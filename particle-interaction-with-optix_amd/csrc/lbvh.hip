@@ -43,34 +43,10 @@ struct Box {
     float lo[3], hi[3];
 };
 
-__device__ inline uint32_t spread10(uint32_t v) {
-    v &= 0x3ffu;
-    v = (v | (v << 16)) & 0x030000FFu;
-    v = (v | (v << 8)) & 0x0300F00Fu;
-    v = (v | (v << 4)) & 0x030C30C3u;
-    v = (v | (v << 2)) & 0x09249249u;
-    return v;
-}
-
 // Morton precision: 2^kMortonBits steps per axis of the box.  The codes only order the
 // leaves (node bounds come from the positions, equal codes are split by index), and
 // 27-bit codes sort in three 9-bit radix passes where 30-bit ones take four.
 constexpr int kMortonBits = 9;
-
-__device__ inline uint32_t quant(float x, float lo, float inv) {
-    float q = (x - lo) * inv;
-    q = fminf(fmaxf(q, 0.0f), (float)((1 << kMortonBits) - 1));
-    return (uint32_t)q;
-}
-
-// 3 kMortonBits-bit Morton code of a position.
-struct MortonKeyOp {
-    float lo[3], inv[3];
-    __device__ uint32_t operator()(float x, float y, float z, uint32_t) const {
-        return (spread10(quant(x, lo[0], inv[0])) << 2) | (spread10(quant(y, lo[1], inv[1])) << 1) |
-               spread10(quant(z, lo[2], inv[2]));
-    }
-};
 
 // Common-prefix length of sorted keys i and j (Karras' delta); equal codes fall back
 // to the indices, which makes every key distinct.
@@ -533,11 +509,7 @@ static int lbvh_build(lj_context* ctx, const float* x, const float* y, const flo
         }
     }
     LJ_HIP(ctx, L.chunks.grow((size_t)pairs * 2 * sizeof(float4)));
-    MortonKeyOp op;
-    for (int d = 0; d < 3; ++d) {
-        op.lo[d] = p->box_lo[d];
-        op.inv[d] = (float)(1 << kMortonBits) / (p->box_hi[d] - p->box_lo[d]);
-    }
+    const MortonKeyOp<kMortonBits> op(p->box_lo, p->box_hi);
     // the sorted payload is the leaf array: positions in Morton order, w = original index
     LJ_TRY(sort_particles(ctx, x, y, z, n, op, 3 * kMortonBits, s));
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, overflow_flag(ctx, n), 1u, 0);

@@ -150,6 +150,36 @@ __device__ inline int pair_mult(const PairConst& c, const float4& pi, const floa
     }
 }
 
+__device__ inline uint32_t spread10(uint32_t v) {
+    v &= 0x3ffu;
+    v = (v | (v << 16)) & 0x030000FFu;
+    v = (v | (v << 8)) & 0x0300F00Fu;
+    v = (v | (v << 4)) & 0x030C30C3u;
+    v = (v | (v << 2)) & 0x09249249u;
+    return v;
+}
+
+// 3 BITS-bit Morton code of a position (BITS <= 10): 2^BITS steps per axis of the box.
+template <int BITS>
+struct MortonKeyOp {
+    float lo[3], inv[3];
+    MortonKeyOp(const float* box_lo, const float* box_hi) {
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = box_lo[d];
+            inv[d] = (float)(1 << BITS) / (box_hi[d] - box_lo[d]);
+        }
+    }
+    __device__ static uint32_t quant(float x, float lo, float inv) {
+        float q = (x - lo) * inv;
+        q = fminf(fmaxf(q, 0.0f), (float)((1 << BITS) - 1));
+        return (uint32_t)q;
+    }
+    __device__ uint32_t operator()(float x, float y, float z, uint32_t) const {
+        return (spread10(quant(x, lo[0], inv[0])) << 2) | (spread10(quant(y, lo[1], inv[1])) << 1) |
+               spread10(quant(z, lo[2], inv[2]));
+    }
+};
+
 // Workgroups are dispatched to the 8 XCDs of an MI355X round-robin (workgroup b runs on
 // XCD b % 8), and each XCD has its own L2.  This bijection gives XCD x a contiguous
 // run of logical blocks, so neighbouring blocks, which read the same neighbour cells,

@@ -9,6 +9,7 @@
 // lj_compute's.
 #include "lj_internal.h"
 #include "lj_pair.h"
+#include "lj_sort.h"
 
 namespace lj {
 
@@ -27,28 +28,44 @@ __global__ __launch_bounds__(256) void k_pack_positions(const float* __restrict_
 // kListLanes-th entry, kListUnroll of them loaded at once; a workgroup takes `turns` times
 // kListRows rows, one set after the other.  Entries j >= n are ignored.  The workgroup's
 // totals, listed and accepted pairs among them, go to sums.
-// Bound by the partners' gathers, a line each: 500,009 particles at shuffled indices, 36M
-// entries, 366 us (12.6 TB/s of 128-byte lines from the caches).  One lane per row, whose
-// loads of the list touched 64 lines and whose three gathers per entry waited for each
-// other, took 1144 us.
+// Bound by the partners' gathers, a line each.  While the positions fit in an XCD's L2 the
+// rows are taken as they come; beyond (order set, see kOrderBytes) in a spatial order, row
+// order[k].w being the k-th, so that rows taken together share their partners' lines.
+// 500,009 particles at shuffled indices, 36M entries: 366 us as they come (12.6 TB/s of
+// 128-byte lines from the caches), 156 us in spatial order.  One lane per row, whose loads
+// of the list touched 64 lines and whose three gathers per entry waited for each other,
+// took 1144 us.
 constexpr int kListLanes = 8;
 constexpr int kListUnroll = 4;
 constexpr int kListRows = 256 / kListLanes;
 
+// Positions above this size are gathered in spatial order: the rows by the Morton code of
+// their particles, 2^kOrderBits steps per axis of the box, whose two radix passes take 45 us
+// at 500,000 particles.  The line lies at one and a half times an XCD's 4 MiB L2.  Measured
+// (the step with the displacement test, us, as they come -> in order): shuffled uniform
+// 200,000 97 -> 97, 300,000 161 -> 126, 500,000 356 -> 198, 1M 956 -> 466; clustered 300,000
+// 166 -> 187, 500,000 383 -> 324, 1M 983 -> 767; particles that already lie in cell order,
+// where the sort is for nothing, 300,000 65 -> 92, 1M 196 -> 255.
+constexpr uint64_t kOrderBytes = 6u << 20;
+constexpr int kOrderBits = 5;
+
 template <int PRED, int PREC, bool VIR>
 __global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ pos, uint32_t n,
+                                                    const float4* __restrict__ order,
                                                     const unsigned long long* __restrict__ rows,
                                                     const uint32_t* __restrict__ cols, PairConst c, uint32_t turns,
                                                     float* __restrict__ fx, float* __restrict__ fy,
                                                     float* __restrict__ fz, float* __restrict__ e,
                                                     BlockSums* __restrict__ sums) {
     const uint32_t sub = threadIdx.x % kListLanes;
+    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
     unsigned long long np = 0, listed = 0;
     double esum = 0.0, vsum = 0.0;
     for (uint32_t turn = 0; turn < turns; ++turn) {
-        const uint32_t i = (blockIdx.x * turns + turn) * kListRows + threadIdx.x / kListLanes;
+        const uint32_t k = (blk * turns + turn) * kListRows + threadIdx.x / kListLanes;
         PairSums<PREC, PRED == LJ_PRED_CUDALJ, VIR> acc;
-        const bool active = i < n;
+        const bool active = k < n;
+        const uint32_t i = order && active ? __float_as_uint(order[k].w) : k;
         const float4 pi = active ? pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
         acc.set_i(pi);
         acc.allow_exact_diff(c, pi, active);
@@ -95,7 +112,7 @@ __global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ p
             vsum += c.e24 * (double)acc.av.value();
         }
     }
-    store_block_sums<true, true>(&sums[blockIdx.x], esum, vsum, np, listed);
+    store_block_sums<true, true>(&sums[blk], esum, vsum, np, listed);
 }
 
 // Largest |p - p0|^2 (FP32, a non-negative float: its bits order like the value).  At
@@ -155,15 +172,20 @@ int lj_compute_list(lj_context* ctx, const float* x, const float* y, const float
     const int64_t sets = div_up(n > 0 ? n : 1, kListRows);
     const uint32_t turns = (uint32_t)(sets < 2048 ? 1 : sets < 16384 ? sets / 2048 : 8);
     const unsigned nb = div_up(sets, turns);
-    LJ_HIP(ctx, ctx->bin.pos.grow(((size_t)(n > 0 ? n : 1) + kPosSpare) * sizeof(float4)));
-    float4* pos = ctx->bin.pos.as<float4>();
+    LJ_HIP(ctx, ctx->bin.stage.grow((size_t)(n > 0 ? n : 1) * sizeof(float4)));
+    float4* pos = ctx->bin.stage.as<float4>();
+    const float4* order = nullptr;
+    if ((uint64_t)n * sizeof(float4) > kOrderBytes) {
+        LJ_TRY(sort_particles(ctx, x, y, z, n, MortonKeyOp<kOrderBits>(p->box_lo, p->box_hi), 3 * kOrderBits, s));
+        order = ctx->bin.pos.as<float4>();
+    }
     if (n > 0) hipLaunchKernelGGL(k_pack_positions, dim3(div_up(n, 256)), dim3(256), 0, s, x, y, z, (uint32_t)n, pos);
     BlockSums* sums;
     LJ_TRY(grow_block_sums(ctx, nb, &sums));
     const bool vir = !(p->flags & LJ_FLAG_NO_VIRIAL);
     const uint32_t nn = (uint32_t)n;
 #define LJ_LF(PRED, PREC, VIR)                                                                                    \
-    hipLaunchKernelGGL((k_list_force<PRED, PREC, VIR>), dim3(nb), dim3(256), 0, s, (const float4*)pos, nn, row_offsets, \
+    hipLaunchKernelGGL((k_list_force<PRED, PREC, VIR>), dim3(nb), dim3(256), 0, s, (const float4*)pos, nn, order, row_offsets, \
                        cols, c, turns, fx, fy, fz, e, sums)
 #define LJ_LF_V(PRED, PREC)            \
     do {                               \
