@@ -198,7 +198,8 @@ __global__ __launch_bounds__(1024) void k_finalize(const BlockSums* __restrict__
 // at one row's length (with 16 lanes a row that took 15 us on those 500,009 rows).
 template <bool LONG>
 __global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long long* __restrict__ rows, uint32_t n,
-                                                            uint32_t* __restrict__ cols) {
+                                                            uint32_t* __restrict__ cols,
+                                                            const uint32_t* __restrict__ draft) {
     constexpr uint32_t kBlock = LONG ? kSortThreads : kBlockRows;  // rows of a workgroup
     __shared__ uint32_t stage[kLdsRow];
     const uint32_t first = blockIdx.x * kBlock;
@@ -209,7 +210,10 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long 
         len = rows[i + 1] - r0;
     }
     const bool fits = len <= kRegRow;
-    if constexpr (!LONG) sort_four_rows(cols + r0, cols + r0, fits ? (uint32_t)len : 0u);
+    if constexpr (!LONG) {
+        const uint32_t* const from = draft && len <= kDraftRow ? draft + (size_t)i * kDraftRow : cols + r0;
+        sort_four_rows(from, cols + r0, fits ? (uint32_t)len : 0u);
+    }
     if (!__syncthreads_or(!fits)) return;
     for (uint32_t q = first; q < first + kBlock && q < n; ++q) {
         const unsigned long long s0 = rows[q], sl = rows[q + 1] - s0;
@@ -622,12 +626,14 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
 
 static void sort_long_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {
     if (n > 0)
-        hipLaunchKernelGGL(k_sort_rows<true>, dim3(div_up(n, kSortThreads)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols);
+        hipLaunchKernelGGL(k_sort_rows<true>, dim3(div_up(n, kSortThreads)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols,
+                           (const uint32_t*)nullptr);
 }
 
-void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {
+void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, const uint32_t* draft, hipStream_t s) {
     if (n > 0)
-        hipLaunchKernelGGL(k_sort_rows<false>, dim3(div_up(n, kBlockRows)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols);
+        hipLaunchKernelGGL(k_sort_rows<false>, dim3(div_up(n, kBlockRows)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols,
+                           draft);
 }
 
 static int pairs_cellgrid(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n,

@@ -435,19 +435,29 @@ __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_force(const float4* __restr
     store_block_sums<true, true>(&sums[blk], esum, vsum, np, tests);
 }
 
-template <int PRED>
+// Counts every query's partners (rowcnt, by original index) and, with DRAFT, keeps the
+// first kDraftRow of them in draft[i * kDraftRow ..], in walk order: rows that fit are then
+// sorted from there into the list, and only longer ones need k_lbvh_fill's second walk.
+// 250,007 clustered particles of 46 partners: count 279 us and fill 338 us before, one walk
+// of 350 us now (mostly the walk: the entries go to 64 lines per store).
+template <int PRED, bool DRAFT>
 __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_count(const float4* __restrict__ leaf, const int2* __restrict__ range,
                                                     const int* __restrict__ rope_by_end, const float4* __restrict__ box, int n, float h, uint32_t limit, PairConst c,
-                                                    uint32_t* __restrict__ rowcnt, int* __restrict__ overflow) {
+                                                    uint32_t* __restrict__ rowcnt, uint32_t* __restrict__ draft,
+                                                    int* __restrict__ overflow) {
     extern __shared__ int lds_list[];
     int* list = lds_list + threadIdx.x;
     const int k = (int)(xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x);
     if (k >= n) return;
     const float4 pi = leaf[k];
     uint32_t cnt = 0;
+    uint32_t* const row = DRAFT ? draft + (size_t)__float_as_uint(pi.w) * kDraftRow : nullptr;
     unsigned long long tests = 0;
     const bool ok = traverse(leaf, range, box, rope_by_end, n, k, pi, h, limit, tests, list, blockDim.x, [&](int, float4 pj) {
-        if (pair_mult<PRED>(c, pi, pj, dist2(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z)) > 0) ++cnt;
+        if (pair_mult<PRED>(c, pi, pj, dist2(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z)) > 0) {
+            if (DRAFT && cnt < kDraftRow) row[cnt] = __float_as_uint(pj.w);
+            ++cnt;
+        }
     });
     if (!ok) atomicOr(overflow, 1);
     rowcnt[__float_as_uint(pi.w)] = cnt;
@@ -457,7 +467,8 @@ template <int PRED>
 __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_fill(const float4* __restrict__ leaf, const int2* __restrict__ range,
                                                    const int* __restrict__ rope_by_end, const float4* __restrict__ box, int n, float h, uint32_t limit, PairConst c,
                                                    const unsigned long long* __restrict__ rows,
-                                                   uint32_t* __restrict__ cols, int* __restrict__ overflow) {
+                                                   uint32_t* __restrict__ cols, uint32_t drafted,
+                                                   int* __restrict__ overflow) {
     extern __shared__ int lds_list[];
     int* list = lds_list + threadIdx.x;
     const int k = (int)(xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x);
@@ -465,6 +476,7 @@ __global__ __launch_bounds__(kLbvhBlock) void k_lbvh_fill(const float4* __restri
     const float4 pi = leaf[k];
     const uint32_t i = __float_as_uint(pi.w);
     const unsigned long long r0 = rows[i], r1 = rows[i + 1];
+    if (r1 - r0 <= drafted) return;
     unsigned long long w = r0;
     unsigned long long tests = 0;
     const bool ok = traverse(leaf, range, box, rope_by_end, n, k, pi, h, limit, tests, list, blockDim.x, [&](int, float4 pj) {
@@ -564,6 +576,9 @@ static float query_half_width(const lj_params* p) {
     }
     return h;
 }
+
+// Particles of the largest call whose partners are drafted: 512 MiB of them.
+constexpr int64_t kDraftMax = ((int64_t)512 << 20) / (kDraftRow * sizeof(uint32_t));
 
 static int check_lbvh_params(lj_context* ctx, const lj_params* p, int64_t n) {
     if (p->predicate == LJ_PRED_CUDALJ)
@@ -680,9 +695,23 @@ int lj_lbvh_pairs(lj_context* ctx, const float* x, const float* y, const float* 
     const int2* range = ctx->lbvh.range.as<int2>();
     const int* rope = ctx->lbvh.rope.as<int>();
     const float4* box = ctx->lbvh.node_box.as<float4>();
+    // the partners of the counting walk are kept when a list is wanted and there is room
+    uint32_t* draft = nullptr;
+    if (capacity > 0 && n > 0 && n <= kDraftMax) {
+        if (ctx->lbvh.draft.grow((size_t)n * kDraftRow * sizeof(uint32_t)) == hipSuccess) draft = ctx->lbvh.draft.as<uint32_t>();
+        else (void)hipGetLastError();
+    }
     if (n > 0) {
         switch (p->predicate) {
-#define LJ_C(P) case P: hipLaunchKernelGGL(k_lbvh_count<P>, dim3(nb), dim3(kLbvhBlock), lds, s, leaf, range, rope, box, (int)n, h, lim, c, rowcnt, ovf); break;
+#define LJ_C(P)                                                                                                       \
+    case P:                                                                                                           \
+        if (draft)                                                                                                    \
+            hipLaunchKernelGGL((k_lbvh_count<P, true>), dim3(nb), dim3(kLbvhBlock), lds, s, leaf, range, rope, box, (int)n, \
+                               h, lim, c, rowcnt, draft, ovf);                                                        \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_lbvh_count<P, false>), dim3(nb), dim3(kLbvhBlock), lds, s, leaf, range, rope, box, (int)n, \
+                               h, lim, c, rowcnt, draft, ovf);                                                        \
+        break;
             LJ_C(LJ_PRED_AABB) LJ_C(LJ_PRED_CUSTOM) LJ_C(LJ_PRED_SPHERE) LJ_C(LJ_PRED_TRIANGLE)
 #undef LJ_C
         }
@@ -698,11 +727,11 @@ int lj_lbvh_pairs(lj_context* ctx, const float* x, const float* y, const float* 
     if (total > capacity) return fail(ctx, LJ_ERR_CAPACITY, "pair list needs %llu entries, capacity is %llu", total, capacity);
     if (total == 0) return LJ_OK;
     switch (p->predicate) {
-#define LJ_F(P) case P: hipLaunchKernelGGL(k_lbvh_fill<P>, dim3(nb), dim3(kLbvhBlock), lds, s, leaf, range, rope, box, (int)n, h, lim, c, (const unsigned long long*)row_offsets, cols, ovf); break;
+#define LJ_F(P) case P: hipLaunchKernelGGL(k_lbvh_fill<P>, dim3(nb), dim3(kLbvhBlock), lds, s, leaf, range, rope, box, (int)n, h, lim, c, (const unsigned long long*)row_offsets, cols, draft ? kDraftRow : 0u, ovf); break;
         LJ_F(LJ_PRED_AABB) LJ_F(LJ_PRED_CUSTOM) LJ_F(LJ_PRED_SPHERE) LJ_F(LJ_PRED_TRIANGLE)
 #undef LJ_F
     }
-    sort_rows(row_offsets, n, cols, s);
+    sort_rows(row_offsets, n, cols, draft, s);
     LJ_HIP(ctx, hipGetLastError());
     return LJ_OK;
 }

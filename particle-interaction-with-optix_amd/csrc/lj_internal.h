@@ -116,6 +116,7 @@ struct LbvhWork {
     DevBuf chunks;        // float4 x2 bounds of aligned leaf chunks (levels of 4, 16, ..., 2^24 leaves)
     DevBuf rope;          // int per leaf: the node after every subtree ending at that leaf
     DevBuf flags;         // the traversal overflow flag
+    DevBuf draft;         // u32 x kDraftRow per particle: partners found by the counting walk
     DevBuf bucket_root;   // uint8 per internal node: 1 when its parent scans it as a bucket
 };
 
@@ -195,8 +196,10 @@ int scan_u32(lj_context* ctx, const uint32_t* in, uint32_t* out, int64_t n, uint
 int scan_u32_to_u64(lj_context* ctx, const uint32_t* in, unsigned long long* out, int64_t n, hipStream_t s);
 
 // Sorts every row of a CSR list, cols[rows[i] .. rows[i + 1]) for i < n, ascending and
-// in place (force.hip).
-void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s);
+// in place (force.hip); with draft (nullable), rows of up to kDraftRow entries are read
+// from draft[i * kDraftRow ..] instead.
+constexpr uint32_t kDraftRow = 256;
+void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, const uint32_t* draft, hipStream_t s);
 
 // Cell-grid pipelines (force.hip).
 // Where a force launch also leaves the particles in cell order (lj_compute_sorted):
