@@ -90,8 +90,14 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force(const float4* __restrict
 // (which fit in the L2s) stored ordinarily.  The workgroups past the first nforce count the
 // 27-cell candidates of the same grid (none when no result is wanted): they need only the
 // offsets, and a launch of their own costs 4-5 us.
-template <int PRED, int PREC, bool VIR>
-__global__ __launch_bounds__(kMaxBlock, 8) void k_force27(const float4* __restrict__ pos,
+// LDS: every workgroup first copies all the particles to LDS and walks them there: a system
+// of up to kLdsParticles leaves a SIMD one wave at most, which waits out each load (1,000
+// particles of 64 partners: 39 us from the caches, 33 us from LDS, now bound by the issue of
+// that one wave's 60 steps of three candidates).
+constexpr uint32_t kLdsParticles = 2048;
+
+template <int PRED, int PREC, bool VIR, bool LDS>
+__global__ __launch_bounds__(kMaxBlock, LDS ? 4 : 8) void k_force27(const float4* __restrict__ pos,
                                                       const uint32_t* __restrict__ cell_of,
                                                       const uint32_t* __restrict__ off, uint32_t n, GridGeom g, Trim tr,
                                                       PairConst c, float* __restrict__ fx, float* __restrict__ fy,
@@ -112,7 +118,13 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force27(const float4* __restri
     const float4 pi = active ? pos[k] : make_float4(0.f, 0.f, 0.f, 0.f);
     acc.set_i(pi);
     acc.allow_exact_diff(c, pi, active);
-    const uint32_t np = stencil27<PRED>(pos, off, k, active, pi, g, 0u, active ? cell_of[k] : 0u, tr, c, acc);
+    __shared__ float4 all[LDS ? kLdsParticles + kPosSpare : 1];
+    if constexpr (LDS) {
+        for (uint32_t t = threadIdx.x; t < n; t += blockDim.x)
+            reinterpret_cast<f32x4*>(all)[t] = reinterpret_cast<const f32x4*>(pos)[t];
+        __syncthreads();
+    }
+    const uint32_t np = stencil27<PRED>(LDS ? all : pos, off, k, active, pi, g, 0u, active ? cell_of[k] : 0u, tr, c, acc);
     acc.template merge<kPairLanes>();
     double esum = 0.0, vsum = 0.0;
     const uint32_t ks = wbase + __lane_id() / kPairLanes;  // = k
@@ -409,15 +421,21 @@ void launch_force(int prec, bool vir, const Shape& sh, unsigned nb, hipStream_t 
     const int out = stage ? 2 : non_temporal_outputs(n) ? 1 : 0;
     if (two_lanes(sh, n)) {
         // (`depth` has no effect: there is no queue)
-#define LJ_L27(PREC, VIR)                                                                                                  \
-    hipLaunchKernelGGL((k_force27<PRED, PREC, VIR>), dim3(nb), dim3(sh.block), 0, s, pos, cell_of, off, n, g, tr, c, fx, fy, \
-                       fz, e, nforce, sums, so)
+#define LJ_L27N(PREC, VIR, LDS)                                                                                        \
+    hipLaunchKernelGGL((k_force27<PRED, PREC, VIR, LDS>), dim3(nb), dim3(sh.block), 0, s, pos, cell_of, off, n, g, tr, c, \
+                       fx, fy, fz, e, nforce, sums, so)
+#define LJ_L27(PREC, VIR)                                     \
+    do {                                                      \
+        if (n <= kLdsParticles) LJ_L27N(PREC, VIR, true);     \
+        else LJ_L27N(PREC, VIR, false);                       \
+    } while (0)
         switch (prec) {
         case LJ_PREC_MIXED: if (vir) LJ_L27(LJ_PREC_MIXED, true); else LJ_L27(LJ_PREC_MIXED, false); break;
         case LJ_PREC_FP32: if (vir) LJ_L27(LJ_PREC_FP32, true); else LJ_L27(LJ_PREC_FP32, false); break;
         default: if (vir) LJ_L27(LJ_PREC_FP32_COMP, true); else LJ_L27(LJ_PREC_FP32_COMP, false); break;
         }
 #undef LJ_L27
+#undef LJ_L27N
         return;
     }
 #define LJ_LAUNCH_QN(PREC, VIR, Q, OUT)                                                                              \

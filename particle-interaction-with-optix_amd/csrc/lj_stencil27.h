@@ -35,14 +35,15 @@ __device__ inline uint32_t of_odd(uint32_t v) {
 // and (-dz, -dy): the even lane finds the trimmed slot range (see stencil_pairs) of its
 // own row and of one row of each pair, the odd lane those of the mirror rows, all ten
 // loads at once; then the two take every second candidate of each pair of rows, walked as
-// one stream.  Every lane of the wave calls this (idle ones with active = false).
+// one stream.  Every lane of the wave calls this (idle ones with active = false).  pos may
+// be a copy in LDS.
 // One lane a particle (stencil_pairs) leaves most of the chip's lanes empty below 500,000
 // particles and walks for twice as long; two lanes there take (lj_compute, us, one -> two
 // lanes): 1,000 particles 87 -> 56, 100,000 of 27 partners 78 -> 66, of 70 127 -> 102,
 // 300,000 clustered 226 -> 192, 131,073 CUDALJ 138 -> 95.  Splitting the rows over the lanes
 // instead, or four and eight lanes, gained less at 100,000 and cost 10-50 % at a million.
 template <int PRED, class Sink>
-__device__ inline uint32_t stencil27(const float4* __restrict__ pos, const uint32_t* __restrict__ off, uint32_t k,
+__device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restrict__ off, uint32_t k,
                                      bool active, const float4& pi, const GridGeom& g, uint32_t cbase, uint32_t key,
                                      const Trim& tr, const PairConst& c, Sink& acc) {
     constexpr int kSets = 5;  // the own row and four mirror pairs

@@ -477,3 +477,26 @@ def test_bin_at_the_digit_scan_sizes(engine, n, cells):
     assert np.array_equal(off.cpu().numpy().view(np.uint32), off_ref)
     assert np.array_equal(perm.cpu().numpy().view(np.uint32), perm_ref)
     assert int(cand.cpu()[0]) == po.candidates(q, off_ref)
+
+
+@pytest.mark.parametrize("cells", [1, 2, 16, 40])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 257, 1024, 2047, 2048, 2049, 4095, 4096, 4097])
+def test_small_systems_on_both_sides_of_the_limits(engine, n, cells):
+    """Binning in one workgroup (up to 4,096 particles) and forces from LDS (up to 2,048),
+    keys of 0, 3, 12 and 16 bits, dense and mostly empty cells: offsets, permutation and
+    counts bit-exact, forces within 1e-5 of FP64."""
+    x, y, z = ljamd.generate("clusters", 7 * n + cells, n, [2, 0.15, 0.3, 0.7])
+    # (a sparse set stays sparse in pairs: the cutoff follows the cells)
+    p = ljamd.make_params(1.0 / cells if cells > 2 else 0.3, cell_edge=1.0 / cells)
+    q = po.from_lj(p)
+    off_ref, perm_ref, _ = po.bin(q, x, y, z)
+    d = engine.to_device(x, y, z)
+    off, perm, cand = engine.bin(*d, p)
+    assert np.array_equal(off.cpu().numpy().view(np.uint32), off_ref)
+    assert np.array_equal(perm.cpu().numpy().view(np.uint32), perm_ref)
+    assert int(cand.cpu()[0]) == po.candidates(q, off_ref)
+    f, e, res = _forces(engine, x, y, z, p)
+    ref = po.forces_f64(q, x, y, z)
+    assert int(res["n_pairs"]) == ref["n_pairs"] and int(res["n_candidates"]) == ref["n_candidates"]
+    err = po.rel_errors(f, (ref["fx"], ref["fy"], ref["fz"]))["rel"]
+    assert err.max() <= FORCE_TOL
