@@ -248,68 +248,73 @@ __global__ __launch_bounds__(kWaveSize) void k_batch_force_shared(
 }
 
 // The systems that two_lanes takes (at most `most` particles): two lanes per particle, 32
-// sorted slots per wave.  A wave that holds slots of several systems takes them one after
-// the other, each with its constants in scalar registers, and keeps their values per slot,
-// as the waves of k_batch_force_shared do.
+// sorted slots per wave.  A wave takes one system, its constants in scalar registers: the
+// first nmain workgroups' waves the system of their first slot, and further waves, listed
+// in the plan as (wave, system), the systems that begin inside a wave; those waves keep
+// their values per slot, as the waves of k_batch_force_shared do.  (One wave that took its
+// systems one after the other kept more alive across them than its 64 registers hold.)
 // Up to this many cells of a batch are counted in the final reduction, one workgroup a
 // system; beyond, on the second stream beside the force pass (4,096 systems of 12.8M
 // cells: 138 us that the force pass's tail hides).
 constexpr uint64_t kReduceCells = 1u << 20;
 constexpr uint32_t kWaveSlots27 = kWaveSize / kPairLanes;
 
-template <int PRED, int PREC>
-__global__ __launch_bounds__(kMaxBlock, 8) void k_batch_force27(
+template <int PRED, int PREC, bool AHEAD>
+__global__ __launch_bounds__(kMaxBlock, AHEAD ? 4 : 8) void k_batch_force27(
     const float4* __restrict__ pos, const uint32_t* __restrict__ cell_of, const uint32_t* __restrict__ off, uint32_t n,
     const SysDesc* __restrict__ sys, const uint32_t* __restrict__ cbase, const uint32_t* __restrict__ chint,
-    uint32_t nsys, uint32_t most, float* __restrict__ fx, float* __restrict__ fy, float* __restrict__ fz,
-    float* __restrict__ e, double2* __restrict__ ev, uint32_t* __restrict__ npair, WaveTotals* __restrict__ wrec) {
-    const uint32_t k = (xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) / kPairLanes;
-    const bool live = k < n;
-    const uint32_t gkey = live ? cell_of[k] : 0xffffffffu;
-    const uint64_t all = __ballot(live);
-    // The keys ascend, so the slots of one system are consecutive lanes: the search for a
-    // system is wave-uniform (scalar loads), and its end tells which lanes it holds.
-    // Nothing per lane but k and the key is live across a turn (64 VGPRs are the budget).
-    for (uint64_t left = all; left;) {
-        const uint32_t s0 = find_sys(cbase, chint, nsys, __builtin_amdgcn_readlane(gkey, __builtin_ctzll(left)));
-        const uint32_t last = s0 + 1u < nsys ? cbase[s0 + 1u] : 0xffffffffu;
-        const uint64_t m = __ballot(gkey < last) & left;
-        const bool mine = (m >> __lane_id()) & 1u;
-        left &= ~m;
-        const SysDesc& d = sys[s0];
-        if (d.n > most) continue;
-        const float4 pi = mine ? pos[k] : make_float4(0.f, 0.f, 0.f, 0.f);
-        const uint32_t key = mine ? gkey - d.cell_base : 0u;
-        const PairConst c = d.c;
-        PairSums<PREC, PRED == LJ_PRED_CUDALJ, true> acc;
-        acc.set_i(pi);
-        acc.allow_exact_diff(c, pi, mine);
-        const uint32_t np = stencil27<PRED>(pos, off, k, mine, pi, d.g, d.cell_base, key, d.tr, c, acc);
-        acc.template merge<kPairLanes>();
-        const bool first = mine && (__lane_id() & 1u) == 0u;
-        double ei = 0.0, vi = 0.0;
+    uint32_t nsys, uint32_t most, uint32_t nmain, const uint2* __restrict__ extra, uint32_t nextra,
+    float* __restrict__ fx, float* __restrict__ fy, float* __restrict__ fz, float* __restrict__ e,
+    double2* __restrict__ ev, uint32_t* __restrict__ npair, WaveTotals* __restrict__ wrec) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize), waves = blockDim.x / kWaveSize;
+    uint32_t w, s0;  // wave-uniform
+    if (blockIdx.x < nmain) {
+        w = xcd_block(blockIdx.x, nmain) * waves + wave;
+        if (w * kWaveSlots27 >= n) return;
+        s0 = find_sys(cbase, chint, nsys, cell_of[w * kWaveSlots27]);
+    } else {
+        const uint32_t q = (blockIdx.x - nmain) * waves + wave;
+        if (q >= nextra) return;
+        w = extra[q].x;
+        s0 = extra[q].y;
+    }
+    const SysDesc& d = sys[s0];
+    if (d.n > most) return;
+    const uint32_t k = w * kWaveSlots27 + __lane_id() / kPairLanes;
+    // a system's sorted slots are its caller range
+    const bool mine = k >= d.first && k - d.first < d.n;
+    const bool whole = __all(mine || k >= n);
+    const float4 pi = mine ? pos[k] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t key = mine ? cell_of[k] - d.cell_base : 0u;
+    const PairConst c = d.c;
+    PairSums<PREC, PRED == LJ_PRED_CUDALJ, true> acc;
+    acc.set_i(pi);
+    acc.allow_exact_diff(c, pi, mine);
+    const uint32_t np = stencil27<PRED, AHEAD>(pos, off, k, mine, pi, d.g, d.cell_base, key, d.tr, c, acc);
+    acc.template merge<kPairLanes>();
+    const bool first = mine && (__lane_id() & 1u) == 0u;
+    double ei = 0.0, vi = 0.0;
+    if (first) {
+        const uint32_t i = __float_as_uint(pos[k].w);
+        fx[i] = (float)(-c.e24 * (double)acc.ax.value());
+        fy[i] = (float)(-c.e24 * (double)acc.ay.value());
+        fz[i] = (float)(-c.e24 * (double)acc.az.value());
+        ei = c.e4 * (double)acc.ae.value();
+        if (e) e[i] = (float)ei;
+        vi = c.e24 * (double)acc.av.value();
+    }
+    if (whole) {
+        // (a system of at most 2^20 particles: 64 lanes' pairs fit 32 bits)
+        const double es = wave_sum(ei), vs = wave_sum(vi);
+        const uint32_t ns = wave_sum(np);
+        if (__lane_id() == 0) wrec[w] = WaveTotals{es, vs, ns, s0, 0u};
+    } else {
+        const uint32_t both = np + dpp_of<1>(np);
         if (first) {
-            const uint32_t i = __float_as_uint(pos[k].w);
-            fx[i] = (float)(-c.e24 * (double)acc.ax.value());
-            fy[i] = (float)(-c.e24 * (double)acc.ay.value());
-            fz[i] = (float)(-c.e24 * (double)acc.az.value());
-            ei = c.e4 * (double)acc.ae.value();
-            if (e) e[i] = (float)ei;
-            vi = c.e24 * (double)acc.av.value();
+            ev[k] = make_double2(ei, vi);
+            npair[k] = both;
         }
-        if (m == all) {  // the wave's only system
-            // (a system of at most 2^20 particles: 64 lanes' pairs fit 32 bits)
-            const double es = wave_sum(ei), vs = wave_sum(vi);
-            const uint32_t ns = wave_sum(np);
-            if (__lane_id() == 0) wrec[k / kWaveSlots27] = WaveTotals{es, vs, ns, s0, 0u};
-        } else {
-            const uint32_t both = np + dpp_of<1>(np);
-            if (first) {
-                ev[k] = make_double2(ei, vi);
-                npair[k] = both;
-                wrec[k / kWaveSlots27].sys = kSharedWave;
-            }
-        }
+        if (__lane_id() == 0) wrec[w].sys = kSharedWave;
     }
 }
 
@@ -431,6 +436,15 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
             seen = true;
         }
     }
+    // two lanes a particle: the systems that begin inside a wave of 32 slots, as (wave, system)
+    std::vector<uint32_t> extra;
+    for (int32_t q = 0; q < nsys; ++q) {
+        const SysDesc& d = desc[(size_t)q];
+        if (d.n && d.first % kWaveSlots27 && two_lanes(sh, d.n)) {
+            extra.push_back(d.first / kWaveSlots27);
+            extra.push_back((uint32_t)q);
+        }
+    }
     LJ_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t s = (hipStream_t)stream;
     BatchWork& W = ctx->batch;
@@ -439,24 +453,30 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     // Upload the plan only when it changed (a cached plan keeps replays free of
     // host-to-device copies).
     const size_t dbytes = desc.size() * sizeof(SysDesc), ubytes = (size_t)nsys * 4;
-    const size_t sbytes = shared.size() * 4;
-    std::vector<uint8_t> blob(dbytes + 3 * ubytes + sbytes);
+    // (the pairs of `extra` come right after the descriptors, 8-byte aligned)
+    const size_t sbytes = shared.size() * 4, xbytes = extra.size() * 4;
+    static_assert(sizeof(SysDesc) % 8 == 0, "the pairs after the descriptors are 8-byte aligned");
+    std::vector<uint8_t> blob(dbytes + xbytes + 3 * ubytes + sbytes);
     std::memcpy(blob.data(), desc.data(), dbytes);
-    std::memcpy(blob.data() + dbytes, first.data(), ubytes);
-    std::memcpy(blob.data() + dbytes + ubytes, cbase.data(), ubytes);
-    std::memcpy(blob.data() + dbytes + 2 * ubytes, ccbase.data(), ubytes);
-    if (sbytes) std::memcpy(blob.data() + dbytes + 3 * ubytes, shared.data(), sbytes);
+    if (xbytes) std::memcpy(blob.data() + dbytes, extra.data(), xbytes);
+    const size_t ubase = dbytes + xbytes;
+    std::memcpy(blob.data() + ubase, first.data(), ubytes);
+    std::memcpy(blob.data() + ubase + ubytes, cbase.data(), ubytes);
+    std::memcpy(blob.data() + ubase + 2 * ubytes, ccbase.data(), ubytes);
+    if (sbytes) std::memcpy(blob.data() + ubase + 3 * ubytes, shared.data(), sbytes);
     const SysDesc* dsys = nullptr;
+    const uint2* dextra = nullptr;
     const uint32_t *dfirst = nullptr, *dcbase = nullptr, *dccbase = nullptr, *dshared = nullptr;
     // search hints of the three base arrays (particles, force-grid cells, cell_edge cells)
     const size_t h1 = hint_entries(ntot), h2 = hint_entries(ctot), h3 = hint_entries(cctot);
     auto bind = [&]() {
         dsys = W.sys.as<SysDesc>();
         const uint8_t* dplan = W.sys.as<uint8_t>();
-        dfirst = reinterpret_cast<const uint32_t*>(dplan + dbytes);
-        dcbase = reinterpret_cast<const uint32_t*>(dplan + dbytes + ubytes);
-        dccbase = reinterpret_cast<const uint32_t*>(dplan + dbytes + 2 * ubytes);
-        dshared = reinterpret_cast<const uint32_t*>(dplan + dbytes + 3 * ubytes);
+        dextra = reinterpret_cast<const uint2*>(dplan + dbytes);
+        dfirst = reinterpret_cast<const uint32_t*>(dplan + ubase);
+        dcbase = reinterpret_cast<const uint32_t*>(dplan + ubase + ubytes);
+        dccbase = reinterpret_cast<const uint32_t*>(dplan + ubase + 2 * ubytes);
+        dshared = reinterpret_cast<const uint32_t*>(dplan + ubase + 3 * ubytes);
     };
     if (blob != W.plan) {
         LJ_HIP(ctx, W.sys.grow(blob.size()));
@@ -542,6 +562,7 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     {
         PhaseTimer tf(ctx, LJ_PHASE_FORCE, s);
         const unsigned nb = div_up(n, sh.block), nb27 = div_up(n * kPairLanes, sh.block);
+        const unsigned nextra = (unsigned)(extra.size() / 2), nx27 = div_up((int64_t)nextra * kWaveSize, sh.block);
         const size_t lds = sh.lds_bytes();
         const size_t lds_shared = sh.queued() ? (size_t)sh.depth * kWaveSize * sizeof(QEntry) : 0;
         if (n > 0) {
@@ -556,12 +577,14 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
                                dsys, dcbase, hcbase, (uint32_t)nsys, most, dshared, sh.refine_x, sh.refine,        \
                                (uint32_t)sh.depth, fx, fy, fz, e, ev, npair, wrec);                                 \
     } while (0)
+#define LJ_BF27(PRED, PREC, AHEAD)                                                                                  \
+    hipLaunchKernelGGL((k_batch_force27<PRED, PREC, AHEAD>), dim3(nb27 + nx27), dim3(sh.block), 0, s, pos, cell_of,  \
+                       (const uint32_t*)off, (uint32_t)n, dsys, dcbase, hcbase, (uint32_t)nsys, most, nb27, dextra,  \
+                       nextra, fx, fy, fz, e, ev, npair, wrec27)
 #define LJ_BF(PRED, PREC)                                                                                          \
     do {                                                                                                           \
-        if (any_two)                                                                                               \
-            hipLaunchKernelGGL((k_batch_force27<PRED, PREC>), dim3(nb27), dim3(sh.block), 0, s, pos, cell_of,      \
-                               (const uint32_t*)off, (uint32_t)n, dsys, dcbase, hcbase, (uint32_t)nsys, most, fx, fy, \
-                               fz, e, ev, npair, wrec27);                                                          \
+        if (any_two && n <= kAheadMax) LJ_BF27(PRED, PREC, true);                                                  \
+        else if (any_two) LJ_BF27(PRED, PREC, false);                                                              \
         if (any_one) {                                                                                             \
             if (sh.queued()) LJ_BFQ(PRED, PREC, true);                                                             \
             else LJ_BFQ(PRED, PREC, false);                                                                        \
@@ -582,6 +605,7 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
             }
 #undef LJ_BF_PREC
 #undef LJ_BF
+#undef LJ_BF27
 #undef LJ_BFQ
         }
     }

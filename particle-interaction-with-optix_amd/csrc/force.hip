@@ -96,8 +96,8 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force(const float4* __restrict
 // that one wave's 60 steps of three candidates).
 constexpr uint32_t kLdsParticles = 2048;
 
-template <int PRED, int PREC, bool VIR, bool LDS>
-__global__ __launch_bounds__(kMaxBlock, LDS ? 4 : 8) void k_force27(const float4* __restrict__ pos,
+template <int PRED, int PREC, bool VIR, bool LDS, bool AHEAD>
+__global__ __launch_bounds__(kMaxBlock, LDS || AHEAD ? 4 : 8) void k_force27(const float4* __restrict__ pos,
                                                       const uint32_t* __restrict__ cell_of,
                                                       const uint32_t* __restrict__ off, uint32_t n, GridGeom g, Trim tr,
                                                       PairConst c, float* __restrict__ fx, float* __restrict__ fy,
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kMaxBlock, LDS ? 4 : 8) void k_force27(const float4
             reinterpret_cast<f32x4*>(all)[t] = reinterpret_cast<const f32x4*>(pos)[t];
         __syncthreads();
     }
-    const uint32_t np = stencil27<PRED>(LDS ? all : pos, off, k, active, pi, g, 0u, active ? cell_of[k] : 0u, tr, c, acc);
+    const uint32_t np = stencil27<PRED, AHEAD>(LDS ? all : pos, off, k, active, pi, g, 0u, active ? cell_of[k] : 0u, tr, c, acc);
     acc.template merge<kPairLanes>();
     double esum = 0.0, vsum = 0.0;
     const uint32_t ks = wbase + __lane_id() / kPairLanes;  // = k
@@ -421,13 +421,14 @@ void launch_force(int prec, bool vir, const Shape& sh, unsigned nb, hipStream_t 
     const int out = stage ? 2 : non_temporal_outputs(n) ? 1 : 0;
     if (two_lanes(sh, n)) {
         // (`depth` has no effect: there is no queue)
-#define LJ_L27N(PREC, VIR, LDS)                                                                                        \
-    hipLaunchKernelGGL((k_force27<PRED, PREC, VIR, LDS>), dim3(nb), dim3(sh.block), 0, s, pos, cell_of, off, n, g, tr, c, \
+#define LJ_L27N(PREC, VIR, LDS, AHEAD)                                                                                     \
+    hipLaunchKernelGGL((k_force27<PRED, PREC, VIR, LDS, AHEAD>), dim3(nb), dim3(sh.block), 0, s, pos, cell_of, off, n, g, tr, c, \
                        fx, fy, fz, e, nforce, sums, so)
 #define LJ_L27(PREC, VIR)                                     \
     do {                                                      \
-        if (n <= kLdsParticles) LJ_L27N(PREC, VIR, true);     \
-        else LJ_L27N(PREC, VIR, false);                       \
+        if (n <= kLdsParticles) LJ_L27N(PREC, VIR, true, true); \
+        else if (n <= kAheadMax) LJ_L27N(PREC, VIR, false, true); \
+        else LJ_L27N(PREC, VIR, false, false);                \
     } while (0)
         switch (prec) {
         case LJ_PREC_MIXED: if (vir) LJ_L27(LJ_PREC_MIXED, true); else LJ_L27(LJ_PREC_MIXED, false); break;

@@ -17,6 +17,11 @@ constexpr int kPairLanes = 2;
 // 1,000,000 on a sphere the two are level (228 us), at 3,000,001 uniform ones one lane is
 // 2.5 % faster (858 against 879 us: half as many set-ups).
 constexpr int64_t kTwoLaneMax = (int64_t)1 << 20;
+// Calls of up to this many particles in all load a step ahead (about four waves a SIMD):
+// us without -> with, 30,000 particles of 70 partners 73 -> 67, 65,000 92 -> 84, clustered
+// 30,000 135 -> 127; level at 140,000 (114, 114); at 300,000 175 -> 183, since the registers
+// leave five waves a SIMD instead of eight.
+constexpr int64_t kAheadMax = 140000;
 inline bool two_lanes(const Shape& sh, int64_t n) { return sh.refine == 1 && sh.refine_x == 1 && n <= kTwoLaneMax; }
 static_assert((kCandidates - 1) * kPairLanes <= kPosSpare, "unclamped candidate loads need spare slots");
 
@@ -37,12 +42,14 @@ __device__ inline uint32_t of_odd(uint32_t v) {
 // loads at once; then the two take every second candidate of each pair of rows, walked as
 // one stream.  Every lane of the wave calls this (idle ones with active = false).  pos may
 // be a copy in LDS.
+// AHEAD: the next iteration's candidates are loaded before this one's are tested, for calls
+// that leave a SIMD a few waves to hide the loads behind (kAheadMax).
 // One lane a particle (stencil_pairs) leaves most of the chip's lanes empty below 500,000
 // particles and walks for twice as long; two lanes there take (lj_compute, us, one -> two
 // lanes): 1,000 particles 87 -> 56, 100,000 of 27 partners 78 -> 66, of 70 127 -> 102,
 // 300,000 clustered 226 -> 192, 131,073 CUDALJ 138 -> 95.  Splitting the rows over the lanes
 // instead, or four and eight lanes, gained less at 100,000 and cost 10-50 % at a million.
-template <int PRED, class Sink>
+template <int PRED, bool AHEAD, class Sink>
 __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restrict__ off, uint32_t k,
                                      bool active, const float4& pi, const GridGeom& g, uint32_t cbase, uint32_t key,
                                      const Trim& tr, const PairConst& c, Sink& acc) {
@@ -94,6 +101,25 @@ __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restri
     range(4, inz && inp, 1, 1, gz + gyp);
     uint32_t np = 0;
     const f32x4* const p4 = reinterpret_cast<const f32x4*>(pos);
+    auto visit = [&](uint32_t t, uint32_t e, const f32x4 (&v)[kCandidates]) {
+#pragma unroll
+        for (int q = 0; q < kCandidates; ++q) {
+            const uint32_t tq = t + q * kPairLanes;
+            if (q > 0 && tq >= e) continue;
+            const float4 pj = make_float4(v[q].x, v[q].y, v[q].z, v[q].w);
+            const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+            const float d2 = dist2(dx, dy, dz);
+            if (PRED == LJ_PRED_CUDALJ && tq == k) continue;
+            const int mult = pair_mult<PRED>(c, pi, pj, d2);
+            if (!mult) continue;
+            np += (uint32_t)mult;
+            acc.add(c, pj, dx, dy, dz, d2, mult);
+        }
+    };
+    auto load = [&](uint32_t t, f32x4 (&v)[kCandidates]) {
+#pragma unroll
+        for (int q = 0; q < kCandidates; ++q) v[q] = p4[t + q * kPairLanes];
+    };
 #pragma unroll
     for (int u = 0; u < kSets; ++u) {
         uint32_t t = of_even(b[u]) + sub, e = of_even(en[u]), t2 = of_odd(b[u]) + (sub ^ 1u), e2 = of_odd(en[u]);
@@ -102,28 +128,35 @@ __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restri
             e = e2;
             t2 = e2;
         }
-        while (t < e) {
+        if constexpr (AHEAD) {
             f32x4 v[kCandidates];
+            load(t, v);
+            while (t < e) {
+                uint32_t tn = t + kCandidates * kPairLanes, eN = e;
+                if (tn >= e) {  // on to the mirror row
+                    tn = t2;
+                    eN = e2;
+                    t2 = e2;
+                }
+                f32x4 vn[kCandidates];
+                load(tn < eN ? tn : t, vn);
+                visit(t, e, v);
+                t = tn;
+                e = eN;
 #pragma unroll
-            for (int q = 0; q < kCandidates; ++q) v[q] = p4[t + q * kPairLanes];
-#pragma unroll
-            for (int q = 0; q < kCandidates; ++q) {
-                const uint32_t tq = t + q * kPairLanes;
-                if (q > 0 && tq >= e) continue;
-                const float4 pj = make_float4(v[q].x, v[q].y, v[q].z, v[q].w);
-                const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-                const float d2 = dist2(dx, dy, dz);
-                if (PRED == LJ_PRED_CUDALJ && tq == k) continue;
-                const int mult = pair_mult<PRED>(c, pi, pj, d2);
-                if (!mult) continue;
-                np += (uint32_t)mult;
-                acc.add(c, pj, dx, dy, dz, d2, mult);
+                for (int q = 0; q < kCandidates; ++q) v[q] = vn[q];
             }
-            t += kCandidates * kPairLanes;
-            if (t >= e) {  // on to the mirror row
-                t = t2;
-                e = e2;
-                t2 = e2;
+        } else {
+            while (t < e) {
+                f32x4 v[kCandidates];
+                load(t, v);
+                visit(t, e, v);
+                t += kCandidates * kPairLanes;
+                if (t >= e) {  // on to the mirror row
+                    t = t2;
+                    e = e2;
+                    t2 = e2;
+                }
             }
         }
     }
