@@ -68,6 +68,7 @@ static int grid_of(lj_context* ctx, const lj_params* p, GridGeom* g) {
     if (nc > 0x7fffffffull) return fail(ctx, LJ_ERR_OVERFLOW, "cell count %llu exceeds 2^31-1", (unsigned long long)nc);
     g->cw[0] = g->cw[1] = g->cw[2] = cw;
     g->ncells = (uint32_t)nc;
+    set_divisors(g);
     return LJ_OK;
 }
 

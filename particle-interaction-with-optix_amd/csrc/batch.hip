@@ -85,13 +85,13 @@ __global__ __launch_bounds__(256) void k_batch_coarse_counts(const uint32_t* __r
     ccount[c] = coarse_count(foff + d.cell_base, d.g, d.cg, Kx, K, c - d.ccell_base);
 }
 
-// 27-cell candidates of the particles in global cell c of system d's cell_edge grid, from
-// the offsets coff over the concatenated cell_edge cells (ComputeNbInteractions
+// 27-cell candidates of the nh particles in global cell c of system d's cell_edge grid,
+// from the offsets coff over the concatenated cell_edge cells (ComputeNbInteractions
 // semantics, cudaLJ.cu:255-297).
-__device__ inline unsigned long long cell_candidates(const uint32_t* __restrict__ coff, const SysDesc& d, uint32_t c) {
+__device__ inline unsigned long long cell_candidates(const uint32_t* __restrict__ coff, const SysDesc& d, uint32_t c,
+                                                     uint32_t nh) {
     const GridGeom& g = d.cg;
     const uint32_t base = d.ccell_base;
-    const uint32_t c0 = coff[c], c1 = coff[c + 1];
     int32_t cx, cy, cz;
     cell_coords(g, c - base, cx, cy, cz);
     const int32_t gx = g.g[0], gy = g.g[1], gz = g.g[2];
@@ -113,7 +113,6 @@ __device__ inline unsigned long long cell_candidates(const uint32_t* __restrict_
 #pragma unroll
     for (int q = 0; q < 9; ++q)
         if (in[q]) sum += hi[q] - lo[q];
-    const uint32_t nh = c1 - c0;
     return nh ? (unsigned long long)nh * (sum - 1) : 0ull;
 }
 
@@ -128,8 +127,9 @@ __global__ __launch_bounds__(256) void k_batch_candidates(const uint32_t* __rest
     uint32_t s = 0xffffffffu;
     unsigned long long v = 0;
     if (c < nccells) {
+        const uint32_t c0 = coff[c], c1 = coff[c + 1];  // on their way during the search
         s = find_sys(ccbase, cchint, nsys, c);
-        v = cell_candidates(coff, sys[s], c);
+        v = cell_candidates(coff, sys[s], c, c1 - c0);
     }
     const uint32_t s0 = __shfl(s, 0, kWaveSize);
     if (__all(s == s0 || s == 0xffffffffu)) {
@@ -357,7 +357,8 @@ __global__ __launch_bounds__(256) void k_batch_reduce(const SysDesc* __restrict_
             }
         }
         if (!cand)
-            for (uint32_t c = threadIdx.x; c < d.cg.ncells; c += 256) nc += cell_candidates(coff, d, d.ccell_base + c);
+            for (uint32_t c = d.ccell_base + threadIdx.x; c < d.ccell_base + d.cg.ncells; c += 256)
+                nc += cell_candidates(coff, d, c, coff[c + 1] - coff[c]);
     }
     __shared__ BlockSums total;
     store_block_sums<true, true>(&total, a, b, np, nc);

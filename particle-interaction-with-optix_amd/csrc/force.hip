@@ -525,6 +525,7 @@ int refine_geom(lj_context* ctx, const GridGeom& g, const lj_params* p, int Kx, 
     }
     if (nc > 0x7fffffffull) return fail(ctx, LJ_ERR_OVERFLOW, "refined grid holds more than 2^31-1 cells");
     f->ncells = (uint32_t)nc;
+    set_divisors(f);
     return LJ_OK;
 }
 

@@ -19,7 +19,25 @@ struct GridGeom {
     int32_t g[3];      // cells per axis
     float gmax[3];     // (float)(g-1), the clamp of the cell coordinate
     uint32_t ncells;
+    // n / g[d] for d = 0, 1 and n < 2^31 as mulhi(n, mul) >> shift (mul = 0: g[d] is 1);
+    // two 32-bit divisions per particle took 56 issue slots of a wave, these take 20
+    uint32_t mul[2], shift[2];
 };
+
+// The divisors above for g[0] and g[1].  With 2^(L-1) < d <= 2^L and m = ceil(2^(31+L) / d),
+// n m / 2^(31+L) exceeds n / d by less than n / 2^31 / d < 1 / d, so its floor is that of n / d.
+inline void set_divisors(GridGeom* g) {
+    for (int d = 0; d < 2; ++d) {
+        const uint32_t v = (uint32_t)g->g[d];
+        uint32_t L = 0;
+        while (((uint64_t)1 << L) < v) ++L;
+        g->mul[d] = v > 1 ? (uint32_t)((((uint64_t)1 << (31 + L)) + v - 1) / v) : 0u;
+        g->shift[d] = L > 0 ? L - 1 : 0u;
+    }
+}
+__device__ inline uint32_t div_axis(const GridGeom& g, int d, uint32_t n) {
+    return g.mul[d] ? __umulhi(n, g.mul[d]) >> g.shift[d] : n;
+}
 
 struct PairConst {
     double sig2d;      // sigma*sigma, exact in FP64

@@ -48,10 +48,10 @@ static_assert(kCandidates - 1 <= kPosSpare, "unclamped candidate loads need spar
 constexpr int kMaxDepth = 32;
 
 __device__ inline void cell_coords(const GridGeom& g, uint32_t key, int32_t& cx, int32_t& cy, int32_t& cz) {
-    cx = (int32_t)(key % (uint32_t)g.g[0]);
-    const uint32_t r = key / (uint32_t)g.g[0];
-    cy = (int32_t)(r % (uint32_t)g.g[1]);
-    cz = (int32_t)(r / (uint32_t)g.g[1]);
+    const uint32_t r = div_axis(g, 0, key), z = div_axis(g, 1, r);
+    cx = (int32_t)(key - r * (uint32_t)g.g[0]);
+    cy = (int32_t)(r - z * (uint32_t)g.g[1]);
+    cz = (int32_t)z;
 }
 
 // Particles in cell c of the cell_edge grid cg, from the offsets foff of the refined
@@ -61,9 +61,8 @@ __device__ inline void cell_coords(const GridGeom& g, uint32_t key, int32_t& cx,
 // cells, which the coarse clamp also maps to the last X).
 __device__ inline uint32_t coarse_count(const uint32_t* __restrict__ foff, const GridGeom& fg, const GridGeom& cg, int Kx,
                                         int K, uint32_t c) {
-    const int32_t X = (int32_t)(c % (uint32_t)cg.g[0]);
-    const uint32_t rem = c / (uint32_t)cg.g[0];
-    const int32_t Y = (int32_t)(rem % (uint32_t)cg.g[1]), Z = (int32_t)(rem / (uint32_t)cg.g[1]);
+    int32_t X, Y, Z;
+    cell_coords(cg, c, X, Y, Z);
     const int32_t fx0 = Kx * X, fx1 = X == cg.g[0] - 1 ? fg.g[0] - 1 : Kx * X + Kx - 1;
     const int32_t fy0 = K * Y, fy1 = Y == cg.g[1] - 1 ? fg.g[1] - 1 : K * Y + K - 1;
     const int32_t fz0 = K * Z, fz1 = Z == cg.g[2] - 1 ? fg.g[2] - 1 : K * Z + K - 1;
