@@ -109,7 +109,8 @@ typedef struct lj_params {
     int16_t refine_x;  /* force-grid cells per cell_edge along x: 1, 2, 4, 8 or 16, not
                           below refine; 0 = refine when refine is set, else the default */
     int16_t block;     /* particles per workgroup: 0, 64, 128 or 256 */
-    int16_t depth;     /* LDS queue entries per particle: 0, 8, 16 or 32; 1 = no queue */
+    int16_t depth;     /* LDS queue entries per particle: 0, 8, 16 or 32; 1 = no queue (no
+                          effect on the cell_edge grid up to 2^20 particles: no queue there) */
 } lj_params;
 
 /* Scalar results, written to DEVICE memory by the compute calls. */
