@@ -268,12 +268,13 @@ __global__ __launch_bounds__(kMaxBlock, AHEAD ? 4 : 8) void k_batch_force27(
     double2* __restrict__ ev, uint32_t* __restrict__ npair, WaveTotals* __restrict__ wrec) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize), waves = blockDim.x / kWaveSize;
     uint32_t w, s0;  // wave-uniform
-    if (blockIdx.x < nmain) {
-        w = xcd_block(blockIdx.x, nmain) * waves + wave;
+    const uint32_t blk = block_index();
+    if (blk < nmain) {
+        w = xcd_block(blk, nmain) * waves + wave;
         if (w * kWaveSlots27 >= n) return;
         s0 = find_sys(cbase, chint, nsys, cell_of[w * kWaveSlots27]);
     } else {
-        const uint32_t q = (blockIdx.x - nmain) * waves + wave;
+        const uint32_t q = (blk - nmain) * waves + wave;
         if (q >= nextra) return;
         w = extra[q].x;
         s0 = extra[q].y;
@@ -579,7 +580,7 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
                                (uint32_t)sh.depth, fx, fy, fz, e, ev, npair, wrec);                                 \
     } while (0)
 #define LJ_BF27(PRED, PREC, AHEAD)                                                                                  \
-    hipLaunchKernelGGL((k_batch_force27<PRED, PREC, AHEAD>), dim3(nb27 + nx27), dim3(sh.block), 0, s, pos, cell_of,  \
+    hipLaunchKernelGGL((k_batch_force27<PRED, PREC, AHEAD>), grid_of_blocks(nb27 + nx27), dim3(sh.block), 0, s, pos, cell_of,  \
                        (const uint32_t*)off, (uint32_t)n, dsys, dcbase, hcbase, (uint32_t)nsys, most, nb27, dextra,  \
                        nextra, fx, fy, fz, e, ev, npair, wrec27)
 #define LJ_BF(PRED, PREC)                                                                                          \

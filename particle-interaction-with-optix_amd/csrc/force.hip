@@ -214,7 +214,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long 
                                                             const uint32_t* __restrict__ draft) {
     constexpr uint32_t kBlock = LONG ? kSortThreads : kBlockRows;  // rows of a workgroup
     __shared__ uint32_t stage[kLdsRow];
-    const uint32_t first = blockIdx.x * kBlock;
+    const uint32_t first = block_index() * kBlock;
     const uint32_t i = first + (LONG ? threadIdx.x : threadIdx.x / kRowLanes);
     unsigned long long r0 = 0, len = 0;
     if (i < n) {
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kPairThreads) void k_pairs(const float4* __restrict
     __shared__ uint32_t lists[FILL ? kWaves : 1][FILL ? 4 * kListStride : 1];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const unsigned lane = __lane_id();
-    const uint32_t first = (xcd_block(blockIdx.x, gridDim.x) * kWaves + wave) * kPairSlots;
+    const uint32_t first = (xcd_block(block_index(), block_count()) * kWaves + wave) * kPairSlots;
     if (first >= n) return;  // the whole wave (no workgroup barrier below)
     const uint32_t cnt = n - first < (uint32_t)kPairSlots ? n - first : (uint32_t)kPairSlots;
     const uint32_t key = cell_of[first + (lane < cnt ? lane : cnt - 1u)];
@@ -646,13 +646,13 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
 
 static void sort_long_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, hipStream_t s) {
     if (n > 0)
-        hipLaunchKernelGGL(k_sort_rows<true>, dim3(div_up(n, kSortThreads)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols,
+        hipLaunchKernelGGL(k_sort_rows<true>, grid_of_blocks(div_up(n, kSortThreads)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols,
                            (const uint32_t*)nullptr);
 }
 
 void sort_rows(const unsigned long long* rows, int64_t n, uint32_t* cols, const uint32_t* draft, hipStream_t s) {
     if (n > 0)
-        hipLaunchKernelGGL(k_sort_rows<false>, dim3(div_up(n, kBlockRows)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols,
+        hipLaunchKernelGGL(k_sort_rows<false>, grid_of_blocks(div_up(n, kBlockRows)), dim3(kSortThreads), 0, s, rows, (uint32_t)n, cols,
                            draft);
 }
 
@@ -670,7 +670,7 @@ static int pairs_cellgrid(lj_context* ctx, const float* x, const float* y, const
     uint32_t* rowcnt = ctx->bin.rows.as<uint32_t>();
 #define LJ_PAIRS(P, FILL)                                                                                          \
     case P:                                                                                                        \
-        hipLaunchKernelGGL((k_pairs<P, FILL>), dim3(nb), dim3(kPairThreads), 0, s, pos, cell_of, off, nn, g, c, rowcnt, \
+        hipLaunchKernelGGL((k_pairs<P, FILL>), grid_of_blocks(nb), dim3(kPairThreads), 0, s, pos, cell_of, off, nn, g, c, rowcnt, \
                            (const unsigned long long*)rows, cols);                                                 \
         break;
 #define LJ_PAIRS_ALL(FILL)                                                                             \

@@ -207,4 +207,8 @@ __device__ inline uint32_t xcd_block(uint32_t b, uint32_t nb) {
     return xcd < r ? xcd * (q + 1u) + idx : r * (q + 1u) + (xcd - r) * q + idx;
 }
 
+// Place of a workgroup in a launch over grid_of_blocks (lj_internal.h), and their number.
+__device__ inline uint32_t block_index() { return blockIdx.y * gridDim.x + blockIdx.x; }
+__device__ inline uint32_t block_count() { return gridDim.y * gridDim.x; }
+
 }  // namespace lj

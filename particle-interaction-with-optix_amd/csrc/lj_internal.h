@@ -276,4 +276,15 @@ class PhaseTimer {
 
 inline unsigned div_up(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
+// The grid of a launch of `blocks` workgroups (fewer than 2^32 - 2^16) that may hold more
+// threads than a dimension of a launch takes, which is 2^32 - 1: rows of up to kGridRow
+// workgroups, of one length, so that fewer places than rows are left over.  Kernels launched
+// so take their place from block_index and have nothing to do past the end.
+constexpr uint64_t kGridRow = 1u << 16;
+inline dim3 grid_of_blocks(uint64_t blocks) {
+    const uint64_t rows = (blocks + kGridRow - 1) / kGridRow;
+    if (rows <= 1) return dim3((unsigned)(blocks > 0 ? blocks : 1));
+    return dim3((unsigned)((blocks + rows - 1) / rows), (unsigned)rows);
+}
+
 }  // namespace lj

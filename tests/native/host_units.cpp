@@ -1,0 +1,51 @@
+// Checks of the engine's host arithmetic that no call on a CPU reaches (built by
+// tests/native/Makefile with AddressSanitizer and UndefinedBehaviorSanitizer, the host side
+// only): launch sizes at the largest counts that the interface takes.  Exit status 0 = all
+// checks passed.
+#include <cstdio>
+
+#include "lj_rows.h"
+#include "lj_stencil27.h"
+
+static int failures = 0;
+#define CHECK(c)                                                           \
+    do {                                                                   \
+        if (!(c)) {                                                        \
+            std::fprintf(stderr, "check failed: %s (line %d)\n", #c, __LINE__); \
+            ++failures;                                                    \
+        }                                                                  \
+    } while (0)
+
+// Every workgroup has a place, no dimension holds 2^32 threads, and less than one row's
+// number of places is left over.
+static void check_launch(uint64_t blocks, uint64_t threads) {
+    const dim3 g = lj::grid_of_blocks(blocks);
+    const uint64_t places = (uint64_t)g.x * g.y;
+    CHECK(g.z == 1 && places >= blocks && places < 0xffffffffull);
+    CHECK(g.x * threads < (1ull << 32) && g.y < 65536);
+    CHECK(places - blocks < g.y || blocks == 0);
+}
+
+int main() {
+    const uint64_t most = 0x7fffffffull;  // particles of a call
+    for (uint64_t n : {(uint64_t)0, (uint64_t)1, (uint64_t)1 << 20, ((uint64_t)1 << 28) - 1, (uint64_t)1 << 28,
+                       (uint64_t)1 << 30, most - 1, most}) {
+        // row sort, 16 lanes a row and a thread a row
+        check_launch((n + lj::kBlockRows - 1) / lj::kBlockRows, lj::kSortThreads);
+        check_launch((n + lj::kSortThreads - 1) / lj::kSortThreads, lj::kSortThreads);
+        // neighbour lists, 16 slots a wave of 64
+        check_launch((n + 63) / 64, 256);
+        // batched forces, two lanes a particle, with as many further waves as there can be
+        for (uint64_t block : {64, 128, 256}) {
+            const uint64_t extra = n;  // one for every system of a particle
+            check_launch((n * lj::kPairLanes + block - 1) / block + (extra * lj::kWaveSize + block - 1) / block, block);
+        }
+    }
+    for (uint64_t blocks = 1; blocks < (1u << 27); blocks += 1 + blocks / 3) check_launch(blocks, 256);
+    if (failures) {
+        std::fprintf(stderr, "%d checks failed\n", failures);
+        return 1;
+    }
+    std::printf("all checks passed\n");
+    return 0;
+}

@@ -1,6 +1,7 @@
 """Sanitizer runs on the CPU (no GPU needed): the oracle with the engine's host
-generator, and the engine library's host code, each built with AddressSanitizer and
-UndefinedBehaviorSanitizer by tests/native/Makefile and run with leak detection on.
+generator, the engine library's host code, and checks of its host arithmetic, each built
+with AddressSanitizer and UndefinedBehaviorSanitizer by tests/native/Makefile and run with
+leak detection on.
 The drivers cross-check their results, so a run must be both clean and correct."""
 import os
 import pathlib
@@ -21,7 +22,7 @@ def build_dir(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("prog", ["oracle_sanitize", "host_sanitize"])
+@pytest.mark.parametrize("prog", ["oracle_sanitize", "host_sanitize", "host_units"])
 def test_sanitized_run_is_clean(build_dir, prog):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0:halt_on_error=1",
                UBSAN_OPTIONS="halt_on_error=1:print_stacktrace=1", OMP_NUM_THREADS="4")

@@ -500,3 +500,27 @@ def test_small_systems_on_both_sides_of_the_limits(engine, n, cells):
     assert int(res["n_pairs"]) == ref["n_pairs"] and int(res["n_candidates"]) == ref["n_candidates"]
     err = po.rel_errors(f, (ref["fx"], ref["fy"], ref["fz"]))["rel"]
     assert err.max() <= FORCE_TOL
+
+
+@pytest.mark.parametrize("lbvh,n", [(False, (1 << 22) + 65), (True, (1 << 20) + 17)])
+def test_pair_lists_beyond_one_row_of_workgroups(engine, lbvh, n):
+    """More workgroups than one row of a launch's grid holds (64 particles each in the list
+    from the grid, 16 in the row sort): two particles a lattice site, in shuffled order, the
+    last one alone, so that a particle's row is the other one of its site."""
+    rng = np.random.default_rng(n)
+    g = 1
+    while 2 * g**3 < n:
+        g += 1
+    who = rng.permutation(n)  # who[2 s], who[2 s + 1]: the particles of site s
+    site = np.empty(n, np.int64)
+    site[who] = np.arange(n) // 2
+    at = np.stack([site % g, site // g % g, site // (g * g)], 1)
+    x, y, z = ((at + 0.5 + rng.uniform(-0.1, 0.1, (n, 3))) / g).astype(np.float32).T
+    p = ljamd.make_params(0.4 / g, cell_edge=1.0 / g)
+    rows, cols = engine.pairs(*engine.to_device(x, y, z), p, lbvh=lbvh)
+    want = np.full(n, -1, np.int64)
+    want[who[0 : n - 1 : 2]] = who[1:n:2]
+    want[who[1:n:2]] = who[0 : n - 1 : 2]
+    rows = rows.cpu().numpy()
+    assert np.array_equal(np.diff(rows), (want >= 0).astype(np.int64))
+    assert np.array_equal(cols.cpu().numpy(), want[want >= 0])

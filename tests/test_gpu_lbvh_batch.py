@@ -383,3 +383,24 @@ def test_batch_across_the_two_lane_limit(engine):
             assert engine.torch.equal(out[k][a:b].view(engine.torch.int32), one[k][: sy.n].view(engine.torch.int32)), (s, k)
         assert int(r1["n_pairs"]) == int(res[s]["n_pairs"]) and int(r1["n_candidates"]) == int(res[s]["n_candidates"]), s
         assert float(res[s]["e_total"]) == pytest.approx(float(r1["e_total"]), rel=1e-12)
+
+
+def test_batch_beyond_one_row_of_workgroups(engine):
+    """More workgroups than one row of a launch's grid holds (32 particles each): every
+    system, the ones that begin inside a wave among them, equals its own call."""
+    sizes = [700_001, 5, 700_007, 31, 700_010, 97]
+    systems, parts, first = [], [], 0
+    for s, n in enumerate(sizes):
+        parts.append(ljamd.generate("uniform", 970 + s, n))
+        systems.append(ljamd.LJSystem(first, n, ljamd.make_params(0.02 if n > 1000 else 0.3, refine=1, refine_x=1, block=64)))
+        first += n
+    d = engine.to_device(*(np.concatenate([q[i] for q in parts]) for i in range(3)))
+    out = engine.compute_batched(systems, *d)
+    res = ljamd.read_results(out["result"], len(systems))
+    for s, sy in enumerate(systems):
+        a, b = sy.first, sy.first + sy.n
+        one = engine.compute(*(v[a:b] for v in d), sy.params)
+        r1 = ljamd.read_results(one["result"])[0]
+        for k in ("fx", "fy", "fz", "e"):
+            assert engine.torch.equal(out[k][a:b].view(engine.torch.int32), one[k][: sy.n].view(engine.torch.int32)), (s, k)
+        assert int(r1["n_pairs"]) == int(res[s]["n_pairs"]) and int(r1["n_candidates"]) == int(res[s]["n_candidates"]), s
