@@ -11,6 +11,7 @@
 #include <cstring>
 #include <vector>
 
+#include "lj_candidates.h"
 #include "lj_sort.h"
 #include "lj_stencil27.h"
 
@@ -253,10 +254,6 @@ __global__ __launch_bounds__(kWaveSize) void k_batch_force_shared(
 // in the plan as (wave, system), the systems that begin inside a wave; those waves keep
 // their values per slot, as the waves of k_batch_force_shared do.  (One wave that took its
 // systems one after the other kept more alive across them than its 64 registers hold.)
-// Up to this many cells of a batch are counted in the final reduction, one workgroup a
-// system; beyond, on the second stream beside the force pass (4,096 systems of 12.8M
-// cells: 138 us that the force pass's tail hides).
-constexpr uint64_t kReduceCells = 1u << 20;
 constexpr uint32_t kWaveSlots27 = kWaveSize / kPairLanes;
 
 template <int PRED, int PREC, bool AHEAD>
@@ -322,7 +319,7 @@ __global__ __launch_bounds__(kMaxBlock, AHEAD ? 4 : 8) void k_batch_force27(
 // One block per system: FP64 totals over its waves in slot order -- the WaveTotals of
 // the waves it fills alone, the per-slot values of its slots in the (at most two)
 // waves it shares with other systems -- and its candidate count, from cand or, when cand
-// is NULL, counted here from the offsets coff (small batches on the cell_edge grid: one
+// is NULL, counted here from the offsets coff (count_in_reduction: one
 // launch less, and no second stream to fork and join, which took 20 us).
 // wrec27: the records of the systems of at most `most` particles.
 __global__ __launch_bounds__(256) void k_batch_reduce(const SysDesc* __restrict__ sys,
@@ -383,6 +380,7 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     std::vector<SysDesc> desc((size_t)nsys);
     std::vector<uint32_t> first((size_t)nsys), cbase((size_t)nsys), ccbase((size_t)nsys);
     uint64_t ntot = 0, ctot = 0, cctot = 0;
+    uint32_t most_cells = 0;  // of one system, on the cell_edge grid
     const lj_params& p0 = sys[0].params;
     for (int32_t s = 0; s < nsys; ++s) {
         const lj_params& ps = sys[s].params;
@@ -406,6 +404,7 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
         d.ccell_base = (uint32_t)cctot;
         ntot += (uint64_t)sys[s].n;
         cctot += g.ncells;
+        most_cells = g.ncells > most_cells ? g.ncells : most_cells;
         if (ntot > 0x7fffffffull) return fail(ctx, LJ_ERR_OVERFLOW, "batch holds more than 2^31-1 particles");
         if (cctot > 0x7fffffffull) return fail(ctx, LJ_ERR_OVERFLOW, "batch holds more than 2^31-1 cells");
     }
@@ -530,8 +529,8 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     // The candidate counts need only the cell offsets: they run on the context's second
     // stream beside the force pass, into an array of their own that the final
     // reduction copies into the results after the join.
-    // Small batches whose cell_edge cells are the force grid's count in the reduction.
-    const bool fork = sh.refine > 1 || sh.refine_x > 1 || cctot > kReduceCells;
+    // Small systems in small batches whose cell_edge cells are the force grid's count in the reduction.
+    const bool fork = sh.refine > 1 || sh.refine_x > 1 || !count_in_reduction(cctot, most_cells);
     unsigned long long* cand = nullptr;
     if (fork) {
         LJ_HIP(ctx, W.cand.grow((size_t)nsys * sizeof(unsigned long long)));

@@ -1,5 +1,6 @@
 // lj_candidates.h -- the 27-cell candidate count over rows of cells, a kernel of its own
-// (binning.hip) or further workgroups of a force launch (force.hip).
+// (binning.hip) or further workgroups of a force launch (force.hip), and where a batch
+// counts (batch.hip).
 //
 // Reference: ComputeNbInteractions (Cuda-version/cudaLJ.cu:255-297).
 #pragma once
@@ -42,5 +43,18 @@ __device__ inline unsigned long long candidate_rows(const uint32_t* __restrict__
     }
     return v;
 }
+
+// Whether a batch on the cell_edge grid, of `total` cells and at most `most` in one system,
+// counts its candidates in the final reduction, one workgroup a system, or on the second
+// stream beside the force pass.  The reduction walks a system's cells 256 at a time after
+// the force pass: it saves the fork and join (20-40 us) while its longest system takes no
+// longer.  us, reduction and second stream: one system of 36,864 particles in 4,096 cells 73
+// and 76, 72,000 in 8,000 94 and 85, 2,400 in 8,000 62 and 75, 140,625 in 15,625 139 and 105,
+// 48,039 on a sphere in 125,000 425 and 105; 8 systems of 36,864 125 and 133, 72,000 201 and
+// 198, 140,625 389 and 380; 64 of 4,687 in 15,625 cells 135 and 182.  In large batches the
+// force pass's tail hides the count (4,096 systems of 12.8M cells in all: 138 us).
+constexpr uint64_t kReduceCells = 1u << 20;
+constexpr uint32_t kReduceSystem = 8192;
+inline bool count_in_reduction(uint64_t total, uint32_t most) { return total <= kReduceCells && most <= kReduceSystem; }
 
 }  // namespace lj

@@ -1,9 +1,10 @@
 // Checks of the engine's host arithmetic that no call on a CPU reaches (built by
 // tests/native/Makefile with AddressSanitizer and UndefinedBehaviorSanitizer, the host side
-// only): launch sizes at the largest counts that the interface takes.  Exit status 0 = all
-// checks passed.
+// only): launch sizes at the largest counts that the interface takes, where a batch counts
+// its candidates.  Exit status 0 = all checks passed.
 #include <cstdio>
 
+#include "lj_candidates.h"
 #include "lj_rows.h"
 #include "lj_stencil27.h"
 
@@ -41,6 +42,11 @@ int main() {
             check_launch((n * lj::kPairLanes + block - 1) / block + (extra * lj::kWaveSize + block - 1) / block, block);
         }
     }
+    // one workgroup is not left with the cells of a large system, however few there are
+    CHECK(lj::count_in_reduction(96 * 650, 650));
+    CHECK(!lj::count_in_reduction(195112, 195112));
+    CHECK(!lj::count_in_reduction(1000375, 1000000));
+    CHECK(!lj::count_in_reduction(4096ull * 3125, 8000));
     for (uint64_t blocks = 1; blocks < (1u << 27); blocks += 1 + blocks / 3) check_launch(blocks, 256);
     if (failures) {
         std::fprintf(stderr, "%d checks failed\n", failures);

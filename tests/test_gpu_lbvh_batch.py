@@ -404,3 +404,23 @@ def test_batch_beyond_one_row_of_workgroups(engine):
         for k in ("fx", "fy", "fz", "e"):
             assert engine.torch.equal(out[k][a:b].view(engine.torch.int32), one[k][: sy.n].view(engine.torch.int32)), (s, k)
         assert int(r1["n_pairs"]) == int(res[s]["n_pairs"]) and int(r1["n_candidates"]) == int(res[s]["n_candidates"]), s
+
+
+@pytest.mark.parametrize("sides", [(20, 5), (21, 5), (20, 20, 21)])
+def test_batch_candidates_on_both_sides_of_the_reduction(engine, sides):
+    """Systems of 8,000 and 9,261 cells, below and above what the final reduction counts by
+    itself, alone and beside each other, a sparse one each: the oracle's counts."""
+    systems, parts, want, first = [], [], [], 0
+    for s, side in enumerate(sides):
+        n = 3 * side**3 if s % 2 else side**3 // 4
+        x, y, z = ljamd.generate("clusters", 980 + s + side, n, [3, 0.1, 0.2, 0.8])
+        p = ljamd.make_params(1.0 / (side + 0.01), refine=1, refine_x=1)
+        q = po.from_lj(p)
+        want.append(po.candidates(q, po.bin(q, x, y, z)[0]))
+        parts.append((x, y, z))
+        systems.append(ljamd.LJSystem(first, n, p))
+        first += n
+    d = engine.to_device(*(np.concatenate([q[i] for q in parts]) for i in range(3)))
+    out = engine.compute_batched(systems, *d)
+    res = ljamd.read_results(out["result"], len(systems))
+    assert [int(r["n_candidates"]) for r in res] == want
