@@ -13,14 +13,18 @@ constexpr int kPairLanes = 2;
 // The two lanes' sums are added at the end, so the two forms differ in the last bits of
 // the 64-bit sums: which one a system takes follows from the system alone (and the shape),
 // never from what else is in the call, and lj_compute, lj_compute_sorted,
-// lj_compute_noalloc and lj_compute_batched agree bit for bit.  Up to 2^20 particles; at
-// 1,000,000 on a sphere the two are level (228 us), at 3,000,001 uniform ones one lane is
-// 2.5 % faster (858 against 879 us: half as many set-ups).
+// lj_compute_noalloc and lj_compute_batched agree bit for bit.  Up to 2^20 particles
+// (lj_compute, us, one lane -> two): 100,000 of 27 neighbours 98 -> 66, 1,000,000 of 70 446 ->
+// 408, on a sphere 278 -> 241; at 3,000,001 uniform of 45 867 -> 851, on a sphere 670 -> 722.
+// In batches that fill the chip: 25.5M particles in systems of 2,000-60,000 of 40 and 70
+// neighbours 6,419 -> 6,270 and 9,401 -> 9,172, 28 systems of 450,000 of 40 level (3,290 and
+// 3,320); 13 of a million of 40 3,480 -> 3,670, where a wave's 32 particles share fewer of
+// the lines that its rows no longer find in the CU's cache.
 constexpr int64_t kTwoLaneMax = (int64_t)1 << 20;
 // Calls of up to this many particles in all load a step ahead (about four waves a SIMD):
-// us without -> with, 30,000 particles of 70 partners 73 -> 67, 65,000 92 -> 84, clustered
-// 30,000 135 -> 127; level at 140,000 (114, 114); at 300,000 175 -> 183, since the registers
-// leave five waves a SIMD instead of eight.
+// us without -> with, 30,000 particles of 70 partners 74 -> 66, 65,000 92 -> 83, clustered
+// 30,000 185 -> 171; level at 140,000 (112, 113); at 300,000 172 -> 177, since the registers
+// leave fewer waves a SIMD.
 constexpr int64_t kAheadMax = 140000;
 inline bool two_lanes(const Shape& sh, int64_t n) { return sh.refine == 1 && sh.refine_x == 1 && n <= kTwoLaneMax; }
 static_assert((kCandidates - 1) * kPairLanes <= kPosSpare, "unclamped candidate loads need spare slots");
@@ -46,8 +50,8 @@ __device__ inline uint32_t of_odd(uint32_t v) {
 // that leave a SIMD a few waves to hide the loads behind (kAheadMax).
 // One lane a particle (stencil_pairs) leaves most of the chip's lanes empty below 500,000
 // particles and walks for twice as long; two lanes there take (lj_compute, us, one -> two
-// lanes): 1,000 particles 87 -> 56, 100,000 of 27 partners 78 -> 66, of 70 127 -> 102,
-// 300,000 clustered 226 -> 192, 131,073 CUDALJ 138 -> 95.  Splitting the rows over the lanes
+// lanes): 1,000 particles 90 -> 42 (from a copy in LDS), 100,000 of 27 partners 98 -> 66, of 70 135 -> 98,
+// 300,000 clustered 248 -> 190, 131,073 CUDALJ 137 -> 87.  Splitting the rows over the lanes
 // instead, or four and eight lanes, gained less at 100,000 and cost 10-50 % at a million.
 template <int PRED, bool AHEAD, class Sink>
 __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restrict__ off, uint32_t k,
@@ -101,24 +105,33 @@ __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restri
     range(4, inz && inp, 1, 1, gz + gyp);
     uint32_t np = 0;
     const f32x4* const p4 = reinterpret_cast<const f32x4*>(pos);
-    auto visit = [&](uint32_t t, uint32_t e, const f32x4 (&v)[kCandidates]) {
+    // candidate t + q kPairLanes exists iff t < lim[q]
+    auto limits = [](uint32_t e, uint32_t (&lim)[kCandidates]) {
+#pragma unroll
+        for (int q = 1; q < kCandidates; ++q) lim[q] = e > (uint32_t)(q * kPairLanes) ? e - (uint32_t)(q * kPairLanes) : 0u;
+    };
+    auto visit = [&](uint32_t t, const uint32_t (&lim)[kCandidates], const f32x4 (&v)[kCandidates]) {
 #pragma unroll
         for (int q = 0; q < kCandidates; ++q) {
-            const uint32_t tq = t + q * kPairLanes;
-            if (q > 0 && tq >= e) continue;
+            if (q > 0 && t >= lim[q]) continue;
             const float4 pj = make_float4(v[q].x, v[q].y, v[q].z, v[q].w);
             const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
             const float d2 = dist2(dx, dy, dz);
-            if (PRED == LJ_PRED_CUDALJ && tq == k) continue;
+            if (PRED == LJ_PRED_CUDALJ && t + q * kPairLanes == k) continue;
             const int mult = pair_mult<PRED>(c, pi, pj, d2);
             if (!mult) continue;
             np += (uint32_t)mult;
             acc.add(c, pj, dx, dy, dz, d2, mult);
         }
     };
+    // One 64-bit base, the candidates at immediate offsets from it, and their limits kept
+    // from step to step (a batch of 25.5M particles in systems of 2,000-60,000 of 70
+    // neighbours: 9,675 us with both formed anew for each candidate, 9,472 with the one base,
+    // 9,182 with the limits too).
     auto load = [&](uint32_t t, f32x4 (&v)[kCandidates]) {
+        const f32x4* const pt = p4 + t;
 #pragma unroll
-        for (int q = 0; q < kCandidates; ++q) v[q] = p4[t + q * kPairLanes];
+        for (int q = 0; q < kCandidates; ++q) v[q] = pt[q * kPairLanes];
     };
 #pragma unroll
     for (int u = 0; u < kSets; ++u) {
@@ -130,8 +143,10 @@ __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restri
         }
         if constexpr (AHEAD) {
             f32x4 v[kCandidates];
+            uint32_t lim[kCandidates];
             load(t, v);
             while (t < e) {
+                limits(e, lim);
                 uint32_t tn = t + kCandidates * kPairLanes, eN = e;
                 if (tn >= e) {  // on to the mirror row
                     tn = t2;
@@ -140,22 +155,25 @@ __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restri
                 }
                 f32x4 vn[kCandidates];
                 load(tn < eN ? tn : t, vn);
-                visit(t, e, v);
+                visit(t, lim, v);
                 t = tn;
                 e = eN;
 #pragma unroll
                 for (int q = 0; q < kCandidates; ++q) v[q] = vn[q];
             }
         } else {
+            uint32_t lim[kCandidates];
+            limits(e, lim);
             while (t < e) {
                 f32x4 v[kCandidates];
                 load(t, v);
-                visit(t, e, v);
+                visit(t, lim, v);
                 t += kCandidates * kPairLanes;
                 if (t >= e) {  // on to the mirror row
                     t = t2;
                     e = e2;
                     t2 = e2;
+                    limits(e, lim);
                 }
             }
         }
