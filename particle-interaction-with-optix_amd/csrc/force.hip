@@ -248,12 +248,16 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long 
 // as one sequence: the lanes hold up to kPairBatches x 64 of them in registers and test
 // each of the run's particles, wave-uniform, against all of them, so that a partner is
 // loaded once per run, a ballot is the answer for 64 candidates, and no lane waits for
-// another's longer walk.  FILL = false counts (a partner with a multiplicity above one
+// another's longer walk.  Where cells hold few particles (kSparseRuns), the run of one or
+// two slots would wait alone for its ranges and then for its candidates: there each of the
+// workgroup's slots gets a lane in every wave, and a wave a quarter of the nine rows.
+// FILL = false counts (a partner with a multiplicity above one
 // is listed once): rowcnt[original index].  FILL = true lists: four particles at a time
 // collect their partners' indices in LDS, and 16 lanes each sort them in registers and
 // store them; rows above kRegRow entries are stored unsorted (sort_long_rows follows).
 // Bound by VALU issue: 500,009 particles, 465 candidates and 72 partners each: count 92 us,
-// list 287 us (one thread per particle: 159 and 479 us, and 108 us more for the sort).
+// list 287 us (one thread per particle: 159 and 479 us, and 108 us more for the sort).  Where
+// cells hold few particles, by the latency of the offsets' and the candidates' loads.
 constexpr int kPairThreads = 256;
 constexpr int kPairSlots = 16;
 constexpr int kPairBatches = 8;
@@ -262,6 +266,16 @@ constexpr uint32_t kPairChunk = kPairBatches * kWaveSize;
 // entries between the four lists of a wave: a row and 16 more, so that the four groups of
 // 16 lanes read different banks
 constexpr int kListStride = (int)kRegRow + kRowLanes;
+// Runs among a workgroup's 64 slots from which on it takes them as sparse: four slots a cell.
+// lj_pairs as a whole, us, runs only -> with the sparse form (one thread per particle, with
+// its sort in the list): 1,000,000 uniform particles of 0.5 neighbours 794 -> 231 (230), of 3
+// 714 -> 264 (304), of 6 610 -> 309 (456), of 12 547 -> 403 (864), of 20 512 -> 498 (1,635);
+// on a sphere of 3 1,122 -> 694 (790).  With the line at 20 runs 235, 267, 314, 429 and 520.
+// Still behind one thread per particle at 3,000,000 uniform particles of 0.5 neighbours, 549
+// against 487, where a cell in eight holds one.
+constexpr int kSparseRuns = 16;
+// A workgroup's sparse rows share its lists.
+constexpr uint32_t kSparseRow = 4 * kListStride / kPairSlots;
 
 __device__ inline void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -280,12 +294,82 @@ __global__ __launch_bounds__(kPairThreads) void k_pairs(const float4* __restrict
     // every predicate but the two distance ones can accept the particle itself
     constexpr bool kSelf = PRED != LJ_PRED_AABB && PRED != LJ_PRED_CUSTOM;
     __shared__ uint32_t lists[FILL ? kWaves : 1][FILL ? 4 * kListStride : 1];
+    __shared__ uint32_t partners[kWaveSize], lens[FILL ? kWaveSize : 1];
+    __shared__ unsigned long long starts[FILL ? kWaveSize : 1];
+    static_assert(kWaves * kPairSlots == kWaveSize, "a lane for each slot of the workgroup");
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const unsigned lane = __lane_id();
-    const uint32_t first = (xcd_block(block_index(), block_count()) * kWaves + wave) * kPairSlots;
+    const uint32_t base = xcd_block(block_index(), block_count()) * kWaves * kPairSlots;
+    if (base >= n) return;  // the whole workgroup
+    const uint32_t mine = base + lane;  // one of the workgroup's slots for each lane of every wave
+    const bool within = mine < n;
+    const uint32_t cell = cell_of[within ? mine : n - 1u];
+    const uint32_t first = base + wave * kPairSlots, last = lane < (unsigned)kPairSlots ? first + lane : first + kPairSlots - 1u;
+    const uint32_t key = cell_of[last < n ? last : n - 1u];  // of the wave's slots (loaded beside cell)
+    const uint32_t before = (uint32_t)__shfl_up((int)cell, 1, kWaveSize);
+    if (__popcll(__ballot(within && (lane == 0 || cell != before))) >= kSparseRuns) {
+        // few slots to a cell: a lane for each of the workgroup's slots, a quarter of the nine
+        // rows of cells for each wave, and a particle's partners in LDS in any order, since
+        // the row is sorted before it is stored
+        if (FILL && lane < (unsigned)kPairSlots) {
+            const uint32_t slot = wave * kPairSlots + lane, k = base + slot;
+            const uint32_t i = k < n ? __float_as_uint(pos[k].w) : 0u;
+            const unsigned long long r0 = k < n ? rows[i] : 0ull;
+            starts[slot] = r0;
+            lens[slot] = k < n ? (uint32_t)(rows[i + 1] - r0) : 0u;
+        }
+        if (wave == 0) partners[lane] = 0u;
+        __syncthreads();
+        const uint32_t len = FILL ? lens[lane] : 0u;
+        if (!FILL || !__any(len > kSparseRow)) {  // the same for every wave
+            const bool walk = FILL ? len > 0u : within;
+            const float4 pi = within ? pos[mine] : make_float4(0.f, 0.f, 0.f, 0.f);
+            uint32_t* const list = &lists[0][0];
+            int32_t cx, cy, cz;
+            cell_coords(g, cell, cx, cy, cz);
+            const int32_t x0 = cx > 0 ? cx - 1 : 0, x1 = cx < g.g[0] - 1 ? cx + 1 : g.g[0] - 1;
+            constexpr int kTurns = (9 + kWaves - 1) / kWaves;
+            uint32_t b[kTurns], e[kTurns];
+#pragma unroll
+            for (int u = 0; u < kTurns; ++u) {
+                const int32_t r = (int32_t)wave + u * kWaves, zz = cz + r / 3 - 1, yy = cy + r % 3 - 1;
+                b[u] = e[u] = 0;
+                if (walk && r < 9 && zz >= 0 && zz < g.g[2] && yy >= 0 && yy < g.g[1]) {
+                    const uint32_t row = (uint32_t)((zz * g.g[1] + yy) * g.g[0]);
+                    b[u] = off[row + x0];
+                    e[u] = off[row + x1 + 1];
+                }
+            }
+            uint32_t m = 0;
+#pragma unroll
+            for (int u = 0; u < kTurns; ++u)
+                for (uint32_t t = b[u]; t < e[u]; ++t) {
+                    const float4 pj = pos[t];
+                    const float d2 = dist2(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
+                    if (t == mine || pair_mult<PRED>(c, pi, pj, d2) <= 0) continue;
+                    if constexpr (FILL) list[lane * kSparseRow + atomicAdd(&partners[lane], 1u)] = __float_as_uint(pj.w);
+                    else ++m;
+                }
+            if (!FILL && m) atomicAdd(&partners[lane], m);
+            __syncthreads();
+            if constexpr (!FILL) {
+                if (wave == 0 && within) rowcnt[__float_as_uint(pi.w)] = partners[lane];
+            } else if (!__any(len > kShortRow)) {
+                // each wave a quarter of the rows
+                const uint32_t slot = wave * kPairSlots + lane / kShortLanes;
+                sort_short_rows(list + slot * kSparseRow, cols + starts[slot], lens[slot]);
+            } else {
+#pragma unroll
+                for (uint32_t q = 0; q < kPairSlots; q += kWaveSize / kRowLanes) {
+                    const uint32_t slot = wave * kPairSlots + q + lane / kRowLanes;
+                    sort_four_rows(list + slot * kSparseRow, cols + starts[slot], lens[slot]);
+                }
+            }
+            return;
+        }
+    }
     if (first >= n) return;  // the whole wave (no workgroup barrier below)
     const uint32_t cnt = n - first < (uint32_t)kPairSlots ? n - first : (uint32_t)kPairSlots;
-    const uint32_t key = cell_of[first + (lane < cnt ? lane : cnt - 1u)];
     uint32_t found = 0;  // lane q: partners of slot first + q
     for (uint32_t j0 = 0; j0 < cnt;) {
         // the run: slots j0 .. j1 - 1, one cell (the keys are sorted)

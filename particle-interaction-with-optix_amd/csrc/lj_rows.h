@@ -84,26 +84,29 @@ __device__ inline void lane_stages(uint32_t (&a)[K]) {
     }
 }
 
-// Sorts the 16 K elements of a row, element lane K + r in register r of its lane
-// (Batcher's bitonic sort, "Sorting networks and their applications", AFIPS 1968, in
-// the form whose merges start with a mirrored comparison).
-template <int K>
+// Sorts the LANES K elements of a row (LANES 4 or 16), element lane K + r in register r of
+// its lane (Batcher's bitonic sort, "Sorting networks and their applications", AFIPS 1968,
+// in the form whose merges start with a mirrored comparison).
+template <int K, int LANES>
 __device__ inline void sort_regs(uint32_t (&a)[K]) {
+    static_assert(LANES == 4 || LANES == 16, "lanes of a row");
     lane_stages<K, 2>(a);
     cross<K, kXor1, true>(a, 1u);  // blocks of 2 lanes
     within<K, K / 2>(a);
     cross<K, kMirror4, true>(a, 2u);  // of 4
     cross<K, kXor1, false>(a, 1u);
     within<K, K / 2>(a);
-    cross<K, kMirror8, true>(a, 4u);  // of 8
-    cross<K, kXor2, false>(a, 2u);
-    cross<K, kXor1, false>(a, 1u);
-    within<K, K / 2>(a);
-    cross<K, kMirror16, true>(a, 8u);  // of 16
-    cross4<K>(a);
-    cross<K, kXor2, false>(a, 2u);
-    cross<K, kXor1, false>(a, 1u);
-    within<K, K / 2>(a);
+    if constexpr (LANES == 16) {
+        cross<K, kMirror8, true>(a, 4u);  // of 8
+        cross<K, kXor2, false>(a, 2u);
+        cross<K, kXor1, false>(a, 1u);
+        within<K, K / 2>(a);
+        cross<K, kMirror16, true>(a, 8u);  // of 16
+        cross4<K>(a);
+        cross<K, kXor2, false>(a, 2u);
+        cross<K, kXor1, false>(a, 1u);
+        within<K, K / 2>(a);
+    }
 }
 
 // K consecutive entries at any 4-byte address as one store of up to 16 bytes each.
@@ -111,19 +114,19 @@ struct __attribute__((packed, aligned(4))) Four {
     uint32_t v[4];
 };
 
-// Sorts from[0, m) (the row itself or a copy in LDS) into row[0, m), m <= 16 K.
-template <int K>
+// Sorts from[0, m) (the row itself or a copy in LDS) into row[0, m), m <= LANES K.
+template <int K, int LANES = kRowLanes>
 __device__ inline void sort_row(const uint32_t* from, uint32_t* row, uint32_t m) {
-    const uint32_t lane = threadIdx.x % kRowLanes;
+    const uint32_t lane = threadIdx.x % LANES;
     uint32_t a[K];
     // striped loads (the order before the sort does not matter); places past the row's
     // end hold the largest value and stay behind every entry
 #pragma unroll
     for (int r = 0; r < K; ++r) {
-        const uint32_t at = r * kRowLanes + lane;
+        const uint32_t at = r * LANES + lane;
         a[r] = at < m ? from[at] : 0xffffffffu;
     }
-    sort_regs<K>(a);
+    sort_regs<K, LANES>(a);
     const uint32_t first = lane * K;
 #pragma unroll
     for (int r = 0; r < K; r += 4) {
@@ -143,6 +146,15 @@ __device__ inline void sort_four_rows(const uint32_t* from, uint32_t* row, uint3
     else if (__any(m > 64u)) sort_row<8>(from, row, m);
     else if (__any(m > 32u)) sort_row<4>(from, row, m);
     else if (__any(m > 0u)) sort_row<2>(from, row, m);
+}
+
+// The wave's sixteen rows (one per four lanes, m <= kShortRow) by the longest of them.
+constexpr int kShortLanes = 4;
+constexpr uint32_t kShortRow = 4 * kShortLanes;
+__device__ inline void sort_short_rows(const uint32_t* from, uint32_t* row, uint32_t m) {
+    if (__any(m > 8u)) sort_row<4, 4>(from, row, m);
+    else if (__any(m > 4u)) sort_row<2, 4>(from, row, m);
+    else if (__any(m > 0u)) sort_row<1, 4>(from, row, m);
 }
 
 // The same sort over v[0, m) by the whole workgroup, for memory that its threads share

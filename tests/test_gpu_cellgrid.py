@@ -524,3 +524,40 @@ def test_pair_lists_beyond_one_row_of_workgroups(engine, lbvh, n):
     rows = rows.cpu().numpy()
     assert np.array_equal(np.diff(rows), (want >= 0).astype(np.int64))
     assert np.array_equal(cols.cpu().numpy(), want[want >= 0])
+
+
+@pytest.mark.parametrize("pred", ["aabb", "cudalj", "triangle"])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129, 4001])
+@pytest.mark.parametrize("per_cell", [0.1, 1, 3, 4, 5, 8])
+def test_pair_lists_at_every_occupancy(engine, per_cell, n, pred):
+    """Cells of a tenth of a particle to eight on average, on both sides of where a workgroup
+    takes its slots one by one instead of cell by cell: the oracle's lists."""
+    x, y, z = ljamd.generate("uniform", int(10 * per_cell) + n, n)
+    g = max(1, round((n / per_cell) ** (1 / 3)))
+    p = ljamd.make_params(0.9 / g, cell_edge=1.0 / g, predicate=pred, softening2=1e-5 if pred == "cudalj" else 0.0)
+    rows, cols = engine.pairs(*engine.to_device(x, y, z), p)
+    want_rows, want_cols = po.pairs_cellgrid(po.from_lj(p), x, y, z)
+    assert np.array_equal(rows.cpu().numpy().astype(np.int64), want_rows.astype(np.int64))
+    assert np.array_equal(cols.cpu().numpy().astype(np.int64), want_cols.astype(np.int64))
+
+
+@pytest.mark.parametrize("crowd", [0, 1, 4, 5, 8, 9, 16, 17, 67, 68, 69, 256, 257])
+def test_pair_lists_of_lone_particles_beside_crowds(engine, crowd):
+    """A row of 128 cells with one particle each beside a row with `crowd` in each, a lone
+    particle's partners: lists of workgroups of lone particles on both sides of what four
+    lanes' registers (4, 8 and 16 entries) and a row's part of LDS (68) hold."""
+    rng = np.random.default_rng(crowd)
+    g = 128
+    lone = np.stack([(np.arange(g) + 0.5) / g, np.full(g, 0.9 / g), np.full(g, 0.5 / g)], 1)
+    cell = np.repeat(np.arange(g), crowd)
+    near = np.stack([(cell + 0.5) / g, np.full(cell.size, 1.1 / g), np.full(cell.size, 0.5 / g)], 1)
+    near = near + rng.uniform(-0.05, 0.05, near.shape) / g
+    at = np.concatenate([lone, near])
+    order = rng.permutation(at.shape[0])
+    x, y, z = at[order].astype(np.float32).T
+    p = ljamd.make_params(0.4 / g, cell_edge=1.0 / g)
+    rows, cols = engine.pairs(*engine.to_device(x, y, z), p)
+    want_rows, want_cols = po.pairs_cellgrid(po.from_lj(p), x, y, z)
+    assert np.all(np.diff(want_rows.astype(np.int64))[order < g] == crowd)
+    assert np.array_equal(rows.cpu().numpy().astype(np.int64), want_rows.astype(np.int64))
+    assert np.array_equal(cols.cpu().numpy().astype(np.int64), want_cols.astype(np.int64))
