@@ -72,6 +72,7 @@ struct BatchKeyOp {
         const SysDesc& d = sys[find_sys(first, hint, nsys, i)];
         return d.cell_base + cell_key(d.g, x, y, z);
     }
+    __device__ bool skip() const { return false; }
 };
 
 // Particle counts of the cell_edge grids from the force grids' offsets (refine > 1).

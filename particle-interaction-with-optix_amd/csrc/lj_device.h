@@ -196,6 +196,7 @@ struct MortonKeyOp {
         return (spread10(quant(x, lo[0], inv[0])) << 2) | (spread10(quant(y, lo[1], inv[1])) << 1) |
                spread10(quant(z, lo[2], inv[2]));
     }
+    __device__ bool skip() const { return false; }
 };
 
 // Workgroups are dispatched to the 8 XCDs of an MI355X round-robin (workgroup b runs on

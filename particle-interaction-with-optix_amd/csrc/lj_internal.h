@@ -219,6 +219,7 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
 struct CellKeyOp {
     GridGeom g;
     __device__ uint32_t operator()(float x, float y, float z, uint32_t) const { return cell_key(g, x, y, z); }
+    __device__ bool skip() const { return false; }
 };
 
 // Cell offsets (ncells+1) of ctx->bin from the sorted keys of a sort_particles, whose

@@ -70,6 +70,7 @@ __global__ __launch_bounds__(kThreads) void k_hist(const float* __restrict__ x, 
                                                    uint32_t* __restrict__ kstore, uint32_t* __restrict__ zero) {
     constexpr int kRadix = 1 << RB;
     __shared__ uint32_t h[kRadix];
+    if (op.skip()) return;
     if (FIRST && zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0u;  // a counter of a later kernel
     for (int d = threadIdx.x; d < kRadix; d += kThreads) h[d] = 0;
     __syncthreads();
@@ -248,6 +249,7 @@ __global__ __launch_bounds__(kSThreads) void k_scatter(const float* __restrict__
     __shared__ uint32_t dstart[kRadix];         // first staging slot of each digit in this tile
     __shared__ uint32_t gbase[kRadix];          // first output slot of each digit for this tile
     __shared__ uint32_t wsum[kRadix / kWave], bsum[kRadix / kWave];
+    if (op.skip()) return;
     const unsigned tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
     const uint32_t base = tile * kTile;
@@ -490,7 +492,8 @@ int sort_passes(lj_context* ctx, const float* x, const float* y, const float* z,
 // Sorts n particles by op's key (the low `bits` bits).  The sorted keys land in
 // ctx->bin.keys[ctx->bin.cur] and the payload (x, y, z, bits of the original index)
 // in ctx->bin.pos, which has room for n + kPosSpare entries (the spare ones are not
-// written).  The first kernel clears *zero (nullable; not when n = 0), a counter that a
+// written).  Where op.skip() holds, which may look at device memory, nothing is sorted.  The
+// first kernel clears *zero (nullable; not when n = 0), a counter that a
 // later kernel of the call adds to.
 template <class KeyOp>
 int sort_particles(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n, const KeyOp& op,

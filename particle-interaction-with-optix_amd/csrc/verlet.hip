@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void k_pack_positions(const float* __restrict_
 // kListRows rows, one set after the other.  Entries j >= n are ignored.  The workgroup's
 // totals, listed and accepted pairs among them, go to sums.
 // Bound by the partners' gathers, a line each.  While the positions fit in an XCD's L2 the
-// rows are taken as they come; beyond (order set, see kOrderBytes) in a spatial order, row
+// rows are taken as they come; beyond (order set, see kOrderBytes and OrderIf) in a spatial order, row
 // order[k].w being the k-th, so that rows taken together share their partners' lines.
 // 500,009 particles at shuffled indices, 36M entries: 366 us as they come (12.6 TB/s of
 // 128-byte lines from the caches), 156 us in spatial order.  One lane per row, whose loads
@@ -46,12 +46,30 @@ constexpr int kListRows = 256 / kListLanes;
 // 200,000 97 -> 97, 300,000 161 -> 126, 500,000 356 -> 198, 1M 956 -> 466; clustered 300,000
 // 166 -> 187, 500,000 383 -> 324, 1M 983 -> 767; particles that already lie in cell order,
 // where the sort is for nothing, 300,000 65 -> 92, 1M 196 -> 255.
+// Lists of fewer than kOrderEntries a row are taken as they come, which the sort and the
+// forces see from the list's own length on the device (shuffled uniform, lj_compute_list, as
+// they come -> in order; before either, one lane a row): 500,000 particles of 2 neighbours
+// 63 -> 99 (75), of 16 118 -> 118 (223), of 20 136 -> 124 (292); 3M of 2 206 -> 561 (416), of 16
+// 859 -> 858 (2,620), of 20 1,065 -> 905 (3,386).
 constexpr uint64_t kOrderBytes = 6u << 20;
 constexpr int kOrderBits = 5;
+constexpr uint64_t kOrderEntries = 16;
+
+// The list's entries, on the device, and how few of them are not worth the order.
+struct OrderIf {
+    const unsigned long long* entries;
+    unsigned long long least;
+    __device__ bool no() const { return *entries < least; }
+};
+struct ListOrderOp : MortonKeyOp<kOrderBits> {
+    OrderIf order;
+    ListOrderOp(const lj_params* p, OrderIf o) : MortonKeyOp<kOrderBits>(p->box_lo, p->box_hi), order(o) {}
+    __device__ bool skip() const { return order.no(); }
+};
 
 template <int PRED, int PREC, bool VIR>
 __global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ pos, uint32_t n,
-                                                    const float4* __restrict__ order,
+                                                    const float4* __restrict__ order, OrderIf want,
                                                     const unsigned long long* __restrict__ rows,
                                                     const uint32_t* __restrict__ cols, PairConst c, uint32_t turns,
                                                     float* __restrict__ fx, float* __restrict__ fy,
@@ -59,6 +77,7 @@ __global__ __launch_bounds__(256) void k_list_force(const float4* __restrict__ p
                                                     BlockSums* __restrict__ sums) {
     const uint32_t sub = threadIdx.x % kListLanes;
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    if (order && want.no()) order = nullptr;
     unsigned long long np = 0, listed = 0;
     double esum = 0.0, vsum = 0.0;
     for (uint32_t turn = 0; turn < turns; ++turn) {
@@ -175,8 +194,9 @@ int lj_compute_list(lj_context* ctx, const float* x, const float* y, const float
     LJ_HIP(ctx, ctx->bin.stage.grow((size_t)(n > 0 ? n : 1) * sizeof(float4)));
     float4* pos = ctx->bin.stage.as<float4>();
     const float4* order = nullptr;
+    const OrderIf want{row_offsets + n, (unsigned long long)n * kOrderEntries};
     if ((uint64_t)n * sizeof(float4) > kOrderBytes) {
-        LJ_TRY(sort_particles(ctx, x, y, z, n, MortonKeyOp<kOrderBits>(p->box_lo, p->box_hi), 3 * kOrderBits, s));
+        LJ_TRY(sort_particles(ctx, x, y, z, n, ListOrderOp(p, want), 3 * kOrderBits, s));
         order = ctx->bin.pos.as<float4>();
     }
     if (n > 0) hipLaunchKernelGGL(k_pack_positions, dim3(div_up(n, 256)), dim3(256), 0, s, x, y, z, (uint32_t)n, pos);
@@ -185,7 +205,7 @@ int lj_compute_list(lj_context* ctx, const float* x, const float* y, const float
     const bool vir = !(p->flags & LJ_FLAG_NO_VIRIAL);
     const uint32_t nn = (uint32_t)n;
 #define LJ_LF(PRED, PREC, VIR)                                                                                    \
-    hipLaunchKernelGGL((k_list_force<PRED, PREC, VIR>), dim3(nb), dim3(256), 0, s, (const float4*)pos, nn, order, row_offsets, \
+    hipLaunchKernelGGL((k_list_force<PRED, PREC, VIR>), dim3(nb), dim3(256), 0, s, (const float4*)pos, nn, order, want, row_offsets, \
                        cols, c, turns, fx, fy, fz, e, sums)
 #define LJ_LF_V(PRED, PREC)            \
     do {                               \

@@ -137,11 +137,11 @@ def test_velocity_verlet_with_list_reuse(engine):
 
 
 @pytest.mark.parametrize("prec", ["mixed", "fp32", "fp32_comp"])
-@pytest.mark.parametrize("n,m", [(1, 0), (33, 1), (64, 7), (65, 8), (257, 9), (1000, 31), (1001, 32), (4097, 33), (70001, 5), (393216, 2), (393217, 3)])
+@pytest.mark.parametrize("n,m", [(1, 0), (33, 1), (64, 7), (65, 8), (257, 9), (1000, 31), (1001, 32), (4097, 33), (70001, 5), (393216, 2), (393217, 3), (393217, 15), (393217, 16), (400003, 17)])
 def test_list_rows_of_every_length(engine, n, m, prec):
     """Rows of m entries on both sides of the eight lanes and the four entries a lane loads
     at once, workgroups of one and of several sets of rows, rows taken as they come and in spatial
-    order (from 393,217 particles), entries past n ignored: the
+    order (from 393,217 particles and 16 entries a row), entries past n ignored: the
     sums over the list in 64 bits.  In 32 bits s^6 is within 15 roundings (five each in r^2
     and in sigma^2 / r^2, cubed) of its value, so a term s^6 (2 s^6 - 1), a difference of
     two parts, is within 32 of 2^-24 of their sum, and 33 terms add as much at most again:
