@@ -206,7 +206,11 @@ __global__ __launch_bounds__(1024) void k_finalize(const BlockSums* __restrict__
 // lies.  Bound by the list's bytes, read and written once: 500,009 rows of 72 entries (36M,
 // 290 MB moved) in 108 us, 2.7 TB/s.  As one thread's insertion sort in global memory, at
 // the end of the kernel that lists the partners, that kernel took 7172 us, and 479 us
-// without it.  LONG: the rows of up to kRegRow entries are sorted already, so a thread looks
+// without it.  A wave takes 16 rows, 4 lanes each, while none of them has more than 16
+// entries, then in four turns of 16 lanes: lists of short rows are bound by the number of
+// waves and of lanes that look at a row's length (lj_lbvh_pairs as a whole, us, four rows a
+// wave -> 16: 3M uniform particles of 0.5 partners 1,461 -> 1,312, of 12 2,815 -> 2,755;
+// 250,007 in clusters of 46 553 -> 555).  LONG: the rows of up to kRegRow entries are sorted already, so a thread looks
 // at one row's length (with 16 lanes a row that took 15 us on those 500,009 rows).
 template <bool LONG>
 __global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long long* __restrict__ rows, uint32_t n,
@@ -215,7 +219,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long 
     constexpr uint32_t kBlock = LONG ? kSortThreads : kBlockRows;  // rows of a workgroup
     __shared__ uint32_t stage[kLdsRow];
     const uint32_t first = block_index() * kBlock;
-    const uint32_t i = first + (LONG ? threadIdx.x : threadIdx.x / kRowLanes);
+    const uint32_t i = first + (LONG ? threadIdx.x : threadIdx.x / kShortLanes);
     unsigned long long r0 = 0, len = 0;
     if (i < n) {
         r0 = rows[i];
@@ -223,8 +227,20 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_rows(const unsigned long 
     }
     const bool fits = len <= kRegRow;
     if constexpr (!LONG) {
-        const uint32_t* const from = draft && len <= kDraftRow ? draft + (size_t)i * kDraftRow : cols + r0;
-        sort_four_rows(from, cols + r0, fits ? (uint32_t)len : 0u);
+        // rows to move or to sort
+        const uint32_t m = fits && (draft || len > 1) ? (uint32_t)len : 0u;
+        auto from = [&](uint32_t row, unsigned long long at) { return draft ? draft + (size_t)row * kDraftRow : cols + at; };
+        if (!__any(m > kShortRow)) {
+            sort_short_rows(from(i, r0), cols + r0, m);
+        } else {
+            const uint32_t wrow = first + threadIdx.x / kWaveSize * (kWaveSize / kShortLanes);  // the wave's first
+            for (int q = 0; q < kWaveSize / kShortLanes; q += kWaveSize / kRowLanes) {
+                const int row = q + (int)__lane_id() / kRowLanes, lane = row * kShortLanes;
+                const unsigned long long at = (unsigned long long)__shfl((uint32_t)(r0 >> 32), lane, kWaveSize) << 32 |
+                                              __shfl((uint32_t)r0, lane, kWaveSize);
+                sort_four_rows(from(wrow + row, at), cols + at, __shfl(m, lane, kWaveSize));
+            }
+        }
     }
     if (!__syncthreads_or(!fits)) return;
     for (uint32_t q = first; q < first + kBlock && q < n; ++q) {

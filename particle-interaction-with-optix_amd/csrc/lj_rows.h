@@ -13,7 +13,9 @@ namespace lj {
 
 constexpr int kSortThreads = 256;
 constexpr int kRowLanes = 16;                                // lanes of a row: one DPP row
-constexpr int kBlockRows = kSortThreads / kRowLanes;         // rows of a workgroup
+constexpr int kShortLanes = 4;                               // lanes of a short row
+constexpr uint32_t kShortRow = 4 * kShortLanes;              // longest row that they sort
+constexpr int kBlockRows = kSortThreads / kShortLanes;       // rows of a workgroup
 constexpr uint32_t kRegRow = 16 * kRowLanes;                 // longest row sorted in registers
 constexpr uint32_t kLdsRow = 4096;                           // longest row sorted in LDS
 
@@ -149,8 +151,6 @@ __device__ inline void sort_four_rows(const uint32_t* from, uint32_t* row, uint3
 }
 
 // The wave's sixteen rows (one per four lanes, m <= kShortRow) by the longest of them.
-constexpr int kShortLanes = 4;
-constexpr uint32_t kShortRow = 4 * kShortLanes;
 __device__ inline void sort_short_rows(const uint32_t* from, uint32_t* row, uint32_t m) {
     if (__any(m > 8u)) sort_row<4, 4>(from, row, m);
     else if (__any(m > 4u)) sort_row<2, 4>(from, row, m);

@@ -31,7 +31,7 @@ int main() {
     const uint64_t most = 0x7fffffffull;  // particles of a call
     for (uint64_t n : {(uint64_t)0, (uint64_t)1, (uint64_t)1 << 20, ((uint64_t)1 << 28) - 1, (uint64_t)1 << 28,
                        (uint64_t)1 << 30, most - 1, most}) {
-        // row sort, 16 lanes a row and a thread a row
+        // row sort, 4 lanes a row and a thread a row
         check_launch((n + lj::kBlockRows - 1) / lj::kBlockRows, lj::kSortThreads);
         check_launch((n + lj::kSortThreads - 1) / lj::kSortThreads, lj::kSortThreads);
         // neighbour lists, 16 slots a wave of 64

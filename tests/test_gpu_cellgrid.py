@@ -436,7 +436,7 @@ def test_c3_precision_subsample(engine):
     assert int(res["n_pairs"]) == pytest.approx(70.3 * n, rel=0.02)
 
 
-ROW_LENGTHS = [0, 1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 4096, 4097]
+ROW_LENGTHS = [0, 1, 2, 4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 4096, 4097]
 
 
 @pytest.mark.parametrize("lbvh", [False, True])
@@ -502,10 +502,10 @@ def test_small_systems_on_both_sides_of_the_limits(engine, n, cells):
     assert err.max() <= FORCE_TOL
 
 
-@pytest.mark.parametrize("lbvh,n", [(False, (1 << 22) + 65), (True, (1 << 20) + 17)])
+@pytest.mark.parametrize("lbvh,n", [(False, (1 << 22) + 65), (True, (1 << 22) + 17)])
 def test_pair_lists_beyond_one_row_of_workgroups(engine, lbvh, n):
     """More workgroups than one row of a launch's grid holds (64 particles each in the list
-    from the grid, 16 in the row sort): two particles a lattice site, in shuffled order, the
+    from the grid and in the row sort): two particles a lattice site, in shuffled order, the
     last one alone, so that a particle's row is the other one of its site."""
     rng = np.random.default_rng(n)
     g = 1
@@ -561,3 +561,22 @@ def test_pair_lists_of_lone_particles_beside_crowds(engine, crowd):
     assert np.all(np.diff(want_rows.astype(np.int64))[order < g] == crowd)
     assert np.array_equal(rows.cpu().numpy().astype(np.int64), want_rows.astype(np.int64))
     assert np.array_equal(cols.cpu().numpy().astype(np.int64), want_cols.astype(np.int64))
+
+
+@pytest.mark.parametrize("lbvh", [False, True])
+@pytest.mark.parametrize("longest", [0, 1, 4, 5, 8, 9, 16, 17])
+def test_pair_rows_of_short_lists(engine, longest, lbvh):
+    """Lists whose longest row has `longest` partners, on both sides of what four lanes sort
+    in one, two and four registers: groups of up to longest + 1 particles."""
+    rng = np.random.default_rng(longest)
+    group = np.repeat(np.arange(100), rng.integers(1, longest + 2, 100))
+    group = np.append(group, np.full(longest + 1, 100))
+    rng.shuffle(group)
+    at = np.stack([group % 11, group // 11, np.zeros_like(group)], 1) * 0.08 + 0.02
+    x, y, z = ((at + rng.uniform(0, 0.005, (group.size, 3))).astype(np.float32)).T
+    rows, cols = engine.pairs(*engine.to_device(x, y, z), ljamd.make_params(0.01), lbvh=lbvh)
+    rows, cols = rows.cpu().numpy(), cols.cpu().numpy()
+    assert np.diff(rows).max() == longest
+    for i, g in enumerate(group):
+        want = np.flatnonzero(group == g)
+        assert np.array_equal(cols[rows[i] : rows[i + 1]], want[want != i]), i
