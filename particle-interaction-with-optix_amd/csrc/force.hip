@@ -687,11 +687,11 @@ int compute_cellgrid(lj_context* ctx, const float* x, const float* y, const floa
     LJ_TRY(result_slot(ctx, result, &res));
     // The candidate count, on the cell_edge grid (ComputeNbInteractions semantics), is
     // only made for a caller that takes the results: by further workgroups of the force
-    // launch (two lanes a particle), else before it, on a refined grid from cell_edge
-    // offsets of its own.
+    // launch (two lanes a particle, count_beside_forces), else before it, on a refined grid
+    // from cell_edge offsets of its own.
     const unsigned nforce = div_up((n > 0 ? n : 1) * (two_lanes(sh, n) ? kPairLanes : 1), sh.block);
     unsigned ncount = 0, nparts = 0;
-    if (result && two_lanes(sh, n)) {
+    if (result && two_lanes(sh, n) && count_beside_forces(n, g.ncells)) {
         ncount = candidate_blocks(g);
     } else if (result && !refined) {
         PhaseTimer t(ctx, LJ_PHASE_OTHER, s);

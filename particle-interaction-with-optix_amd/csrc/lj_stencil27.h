@@ -27,6 +27,15 @@ constexpr int64_t kTwoLaneMax = (int64_t)1 << 20;
 // leave fewer waves a SIMD.
 constexpr int64_t kAheadMax = 140000;
 inline bool two_lanes(const Shape& sh, int64_t n) { return sh.refine == 1 && sh.refine_x == 1 && n <= kTwoLaneMax; }
+// Whether the candidate count of a call with two lanes a particle goes into further
+// workgroups of the force launch, which saves a launch (4-7 us), or into a kernel of its own.
+// Where the force kernel's registers leave four waves a SIMD, those workgroups walk a large
+// grid at that occupancy too: lj_compute of 1,000 and 100,000 particles, us, in the force
+// launch and by itself, in 160^3 cells 68 and 67, 114 and 119, in 256^3 97 and 86, 169 and
+// 168, in 640^3 878 and 646, 791 and 744; 500,000 particles, eight waves a SIMD, 1,156 and
+// 1,174 there.
+constexpr uint32_t kCountCells = 1u << 23;
+inline bool count_beside_forces(int64_t n, uint32_t ncells) { return n > kAheadMax || ncells <= kCountCells; }
 static_assert((kCandidates - 1) * kPairLanes <= kPosSpare, "unclamped candidate loads need spare slots");
 
 // The value of the even (or odd) lane of each pair of neighbouring lanes.

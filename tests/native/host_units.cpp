@@ -1,6 +1,6 @@
 // Checks of the engine's host arithmetic that no call on a CPU reaches (built by
 // tests/native/Makefile with AddressSanitizer and UndefinedBehaviorSanitizer, the host side
-// only): launch sizes at the largest counts that the interface takes, where a batch counts
+// only): launch sizes at the largest counts that the interface takes, where a call counts
 // its candidates.  Exit status 0 = all checks passed.
 #include <cstdio>
 
@@ -47,6 +47,9 @@ int main() {
     CHECK(!lj::count_in_reduction(195112, 195112));
     CHECK(!lj::count_in_reduction(1000375, 1000000));
     CHECK(!lj::count_in_reduction(4096ull * 3125, 8000));
+    // nor a large grid with the few waves of a small system's force launch
+    CHECK(lj::count_beside_forces(1000, 4096) && lj::count_beside_forces(500000, 640u * 640 * 640));
+    CHECK(!lj::count_beside_forces(1000, 640u * 640 * 640) && !lj::count_beside_forces(100000, 400u * 400 * 400));
     for (uint64_t blocks = 1; blocks < (1u << 27); blocks += 1 + blocks / 3) check_launch(blocks, 256);
     if (failures) {
         std::fprintf(stderr, "%d checks failed\n", failures);

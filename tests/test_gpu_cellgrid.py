@@ -580,3 +580,20 @@ def test_pair_rows_of_short_lists(engine, longest, lbvh):
     for i, g in enumerate(group):
         want = np.flatnonzero(group == g)
         assert np.array_equal(cols[rows[i] : rows[i + 1]], want[want != i]), i
+
+
+@pytest.mark.parametrize("side", [203, 204])
+@pytest.mark.parametrize("n", [1, 2000, 140_000, 140_001])
+def test_candidates_of_small_systems_in_large_grids(engine, n, side):
+    """2^23 cells lie between the grids, and 140,000 particles between the sizes, whose
+    candidates are counted beside the forces and by a kernel of their own: the oracle's
+    counts, and the ones of the same call on a finer force grid."""
+    x, y, z = ljamd.generate("clusters", n + side, n, [3, 0.1, 0.2, 0.8])
+    p = ljamd.make_params(1.0 / (side + 0.01))
+    q = po.from_lj(p)
+    want = po.candidates(q, po.bin(q, x, y, z)[0])
+    _, _, res = _forces(engine, x, y, z, p)
+    p.refine, p.refine_x = 1, 2
+    _, _, fine = _forces(engine, x, y, z, p)
+    assert int(res["n_candidates"]) == want and int(fine["n_candidates"]) == want
+    assert int(res["n_pairs"]) == int(fine["n_pairs"])
