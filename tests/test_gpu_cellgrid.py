@@ -597,3 +597,22 @@ def test_candidates_of_small_systems_in_large_grids(engine, n, side):
     _, _, fine = _forces(engine, x, y, z, p)
     assert int(res["n_candidates"]) == want and int(fine["n_candidates"]) == want
     assert int(res["n_pairs"]) == int(fine["n_pairs"])
+
+
+@pytest.mark.parametrize("pred", ["aabb", "cudalj", "triangle"])
+def test_one_lane_on_the_cell_edge_grid(engine, pred):
+    """2^20 + 1 particles, the first size that takes one lane a particle on the cell_edge
+    grid: counts, forces and energies of the FP64 oracle, in the order of the call.  The
+    outputs are 64-bit sums rounded to 32 bits; in the CUDALJ mode, whose terms all but
+    cancel, they are held against the sum of the terms' sizes."""
+    x, y, z = ljamd.generate("uniform", 77, (1 << 20) + 1)
+    p = ljamd.make_params(0.016, predicate=pred, softening2=1e-5 if pred == "cudalj" else 0.0, refine=1, refine_x=1)
+    ref = po.forces_f64(po.from_lj(p), x, y, z)
+    f, e, res = _forces(engine, x, y, z, p)
+    assert int(res["n_pairs"]) == ref["n_pairs"] and int(res["n_candidates"]) == ref["n_candidates"]
+    fin = (np.abs(ref["fx"]) < 3e38) & (np.abs(ref["fy"]) < 3e38) & (np.abs(ref["fz"]) < 3e38)
+    err = po.rel_errors([v[fin] for v in f], [ref[k][fin] for k in ("fx", "fy", "fz")], ref["cond"][fin])
+    assert err["cond"].max() <= 2.0**-22
+    if pred != "cudalj":
+        assert err["rel"].max() <= FORCE_TOL
+    assert float(res["e_total"]) == pytest.approx(ref["e_total"], rel=1e-9)

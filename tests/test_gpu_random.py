@@ -2,8 +2,9 @@
 6,000, boxes of random origin and edge with some particles outside them, uniform,
 clustered and sphere-surface positions (with exact duplicates), random cutoffs, every
 cutoff predicate (the AABB and Custom distance rules, the Sphere and Triangle ray
-models), random kernel shapes (force-grid refinement, workgroup size, LDS queue) and
-both engines (cell grid, LBVH).
+models), random kernel shapes (force-grid refinement, workgroup size, and off the
+cell_edge grid, which has none at these sizes, the LDS queue) and both engines (cell grid,
+LBVH).
 
 Bars as in the fixed-case tests: neighbour lists (CSR) bit-exact against the oracle's
 cell grid (and its O(N^2) brute force for N <= 2,000), accepted-pair counts exact, the

@@ -74,10 +74,11 @@ def test_compute_sorted_equals_compute_permuted(engine, name):
 @pytest.mark.parametrize("pred,depth", [("cudalj", 1), ("triangle", 8), ("custom", 16)])
 def test_compute_sorted_other_predicates_and_queues(engine, pred, depth):
     """The CUDALJ mode (every candidate, itself skipped by slot), a ray model and the LDS
-    queue of accepted partners give the same bits in sorted order as lj_compute's,
-    permuted."""
+    queue of accepted partners (on a refined grid: the cell_edge grid has none at this
+    size) give the same bits in sorted order as lj_compute's, permuted."""
     x, y, z = ljamd.generate("uniform", 91, 50_000)
-    p = ljamd.make_params(0.05, predicate=pred, depth=depth, block=128)
+    p = ljamd.make_params(0.05, predicate=pred, depth=depth, block=128, refine=1,
+                          refine_x=2 if depth > 1 else 1)
     if pred == "cudalj":
         p.softening2, p.sigma = 1e-5, 1.0
     n = x.size
