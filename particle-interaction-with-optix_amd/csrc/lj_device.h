@@ -35,8 +35,8 @@ inline void set_divisors(GridGeom* g) {
         g->shift[d] = L > 0 ? L - 1 : 0u;
     }
 }
-__device__ inline uint32_t div_axis(const GridGeom& g, int d, uint32_t n) {
-    return g.mul[d] ? __umulhi(n, g.mul[d]) >> g.shift[d] : n;
+__host__ __device__ inline uint32_t div_axis(const GridGeom& g, int d, uint32_t n) {
+    return g.mul[d] ? (uint32_t)(((uint64_t)n * g.mul[d]) >> 32) >> g.shift[d] : n;
 }
 
 struct PairConst {

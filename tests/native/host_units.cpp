@@ -1,7 +1,7 @@
 // Checks of the engine's host arithmetic that no call on a CPU reaches (built by
 // tests/native/Makefile with AddressSanitizer and UndefinedBehaviorSanitizer, the host side
-// only): launch sizes at the largest counts that the interface takes, where a call counts
-// its candidates.  Exit status 0 = all checks passed.
+// only): exact reciprocals, launch sizes at the largest counts that the interface takes, where
+// a call counts its candidates.  Exit status 0 = all checks passed.
 #include <cstdio>
 
 #include "lj_candidates.h"
@@ -27,7 +27,30 @@ static void check_launch(uint64_t blocks, uint64_t threads) {
     CHECK(places - blocks < g.y || blocks == 0);
 }
 
+// The quotients of cell indices by reciprocal multiplication, at every place where the
+// quotient changes near the ends of its range and at its powers of two.
+static void check_division(uint32_t v) {
+    lj::GridGeom g{};
+    g.g[0] = g.g[1] = (int32_t)v;
+    lj::set_divisors(&g);
+    const uint32_t most = 0x7fffffffu, top = most / v;
+    bool ok = true;
+    auto at = [&](uint64_t q) {
+        for (uint64_t n = q * v > 0 ? q * v - 1 : 0; n <= q * v + 1 && n <= most; ++n)
+            ok = ok && lj::div_axis(g, 0, (uint32_t)n) == n / v && lj::div_axis(g, 1, (uint32_t)n) == n / v;
+    };
+    for (uint64_t q = 0; q <= 16 && q <= top; ++q) at(q), at(top - q);
+    for (uint64_t q = 1; q <= top; q <<= 1) at(q), at(q - 1), at(q + 1 <= top ? q + 1 : top);
+    ok = ok && lj::div_axis(g, 0, most) == most / v;
+    CHECK(ok);
+}
+
 int main() {
+    // axes of a grid: up to 2^24 cells
+    for (uint32_t v = 1; v <= 30000; ++v) check_division(v);
+    for (uint32_t v = 30001; v < (1u << 24); v += 997) check_division(v);
+    for (uint32_t b = 2; b <= 24; ++b)
+        for (uint32_t v = (1u << b) - 2; v <= (1u << b) + 2 && v <= (1u << 24); ++v) check_division(v);
     const uint64_t most = 0x7fffffffull;  // particles of a call
     for (uint64_t n : {(uint64_t)0, (uint64_t)1, (uint64_t)1 << 20, ((uint64_t)1 << 28) - 1, (uint64_t)1 << 28,
                        (uint64_t)1 << 30, most - 1, most}) {
