@@ -96,7 +96,7 @@ struct BinWork {
     DevBuf offsets;      // u32 per-cell offsets (ncells+1)
     DevBuf pos;          // float4 sorted positions, w = original index bits
     DevBuf pos_alt;      // float4 ping-pong partner of pos during the sort
-    DevBuf partials;     // per-block partial sums (double) for deterministic totals
+    DevBuf partials;     // one BlockSums per workgroup of a force pass, then those of the first reduction
     DevBuf counters;     // u64 counters
     DevBuf rows;         // u64 pair-list row offsets
     DevBuf ccounts;      // u32 counts of the cell_edge grid when the force grid is refined
@@ -125,7 +125,7 @@ struct BatchWork {
     DevBuf hints;         // search hints of the plan's three base arrays (rebuilt with the plan)
     DevBuf npair;         // u32 accepted-pair count of each sorted slot in a wave shared by systems
     DevBuf ev;            // double2 energy and virial of each sorted slot in a wave shared by systems
-    DevBuf wrec;          // one WaveTotals per wave of 64 sorted slots
+    DevBuf wrec;          // one WaveTotals per wave of 64 sorted slots, then one per wave of 32 (two lanes a particle)
     DevBuf cand;          // u64 candidate count per system, counted on the second stream
     std::vector<uint8_t> plan;  // host copy of the plan last uploaded to sys
 };

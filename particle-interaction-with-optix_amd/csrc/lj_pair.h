@@ -9,13 +9,24 @@ namespace lj {
 
 constexpr int kWaveSize = 64;
 
-// The value of the lane that lane ^ d is (d = 1, 2: quad_perm) or of its mirror image in 8
-// (d = 7) or 16 lanes (d = 15), by data-parallel moves: no LDS access and no wait.
+// DPP controls of the lane exchanges inside 16 lanes, which need no LDS access and no wait.
+constexpr int kXor1 = 0xB1;         // quad_perm [1,0,3,2]
+constexpr int kXor2 = 0x4E;         // quad_perm [2,3,0,1]
+constexpr int kMirror4 = 0x1B;      // quad_perm [3,2,1,0]
+constexpr int kMirror16 = 0x140;    // row_mirror
+constexpr int kMirror8 = 0x141;     // row_half_mirror
+
+template <int CTRL>
+__device__ inline uint32_t from_lane(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+
+// The value of the lane that lane ^ d is (d = 1, 2) or of its mirror image in 8 (d = 7) or 16
+// lanes (d = 15).
 template <int D>
 __device__ inline uint32_t dpp_xor(uint32_t v) {
-    constexpr int kCtrl = D == 1 ? 0xB1 : D == 2 ? 0x4E : D == 7 ? 0x141 : 0x140;
     static_assert(D == 1 || D == 2 || D == 7 || D == 15, "lane exchanges that DPP has");
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, true);
+    return from_lane<D == 1 ? kXor1 : D == 2 ? kXor2 : D == 7 ? kMirror8 : kMirror16>(v);
 }
 template <int D, class T>
 __device__ inline T dpp_of(T v) {

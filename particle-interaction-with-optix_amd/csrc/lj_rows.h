@@ -8,6 +8,7 @@
 #pragma once
 
 #include "lj_internal.h"
+#include "lj_pair.h"
 
 namespace lj {
 
@@ -18,18 +19,6 @@ constexpr uint32_t kShortRow = 4 * kShortLanes;              // longest row that
 constexpr int kBlockRows = kSortThreads / kShortLanes;       // rows of a workgroup
 constexpr uint32_t kRegRow = 16 * kRowLanes;                 // longest row sorted in registers
 constexpr uint32_t kLdsRow = 4096;                           // longest row sorted in LDS
-
-// DPP controls of the lane exchanges inside 16 lanes.
-constexpr int kXor1 = 0xB1;         // quad_perm [1,0,3,2]
-constexpr int kXor2 = 0x4E;         // quad_perm [2,3,0,1]
-constexpr int kMirror4 = 0x1B;      // quad_perm [3,2,1,0]
-constexpr int kMirror16 = 0x140;    // row_mirror
-constexpr int kMirror8 = 0x141;     // row_half_mirror
-
-template <int CTRL>
-__device__ inline uint32_t from_lane(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
-}
 
 // One exchange across lanes: element r of a lane against element r (or, mirrored, K - 1
 // - r) of its partner; the lanes with `bit` clear keep the smaller one.

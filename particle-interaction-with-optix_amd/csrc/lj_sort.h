@@ -8,7 +8,9 @@
 //              row per tile)
 //   offsets    a digit-major exclusive scan of that table in three small kernels:
 //              hist[tile * R + d] becomes the first output slot of digit d's keys in
-//              that tile
+//              that tile; for tables of up to 512 tiles in one kernel, which leaves the
+//              digit's keys in earlier tiles there and the digits' totals beside the
+//              table, for the scatter to add the keys of smaller digits itself
 //   scatter    each wave ranks its own contiguous run of keys stably with per-wave LDS
 //              counters (no block barrier per round), the waves' counts are combined
 //              once, the tile is staged in LDS in digit order, and every digit's run

@@ -42,7 +42,7 @@ struct Shape {
 
 constexpr int kMaxBlock = 256;
 // candidates loaded and tested per iteration of the stencil's row loop (the sorted
-// positions carry kCandidates - 1 spare entries, so the loads need no clamp)
+// positions carry kPosSpare spare entries, so the loads need no clamp)
 constexpr int kCandidates = 3;
 static_assert(kCandidates - 1 <= kPosSpare, "unclamped candidate loads need spare slots");
 constexpr int kMaxDepth = 32;

@@ -40,10 +40,10 @@ static_assert((kCandidates - 1) * kPairLanes <= kPosSpare, "unclamped candidate 
 
 // The value of the even (or odd) lane of each pair of neighbouring lanes.
 __device__ inline uint32_t of_even(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xA0, 0xf, 0xf, true);  // quad_perm [0,0,2,2]
+    return from_lane<0xA0>(v);  // quad_perm [0,0,2,2]
 }
 __device__ inline uint32_t of_odd(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xF5, 0xf, 0xf, true);  // quad_perm [1,1,3,3]
+    return from_lane<0xF5>(v);  // quad_perm [1,1,3,3]
 }
 
 // Accepted partners of the particle in sorted slot k (position pi, cell `key` of the

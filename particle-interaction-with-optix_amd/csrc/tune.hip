@@ -7,7 +7,9 @@
 // overhead (more with finer cells), and occupancy against queue fill.  The best
 // choice depends on the density and distribution of the particles, so it is
 // measured, in two stages: every valid grid (K, Kx) with the default workgroup and no
-// queue, then every workgroup size and queue depth on the fastest grid.  Each shape
+// queue, then every workgroup size and queue depth on the fastest grid (where that is the
+// cell_edge grid and no system has more than kTwoLaneMax particles, a depth is without
+// effect and the times of one workgroup size differ by noise alone).  Each shape
 // runs `reps` times on the caller's positions after one untimed call, timed with
 // hipEvents on the caller's stream, and the fastest wins.
 #include <vector>
