@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kMaxBlock, LDS || AHEAD ? 4 : 8) void k_force27(con
             reinterpret_cast<f32x4*>(all)[t] = reinterpret_cast<const f32x4*>(pos)[t];
         __syncthreads();
     }
-    const uint32_t np = stencil27<PRED, AHEAD>(LDS ? all : pos, off, k, active, pi, g, 0u, active ? cell_of[k] : 0u, tr, c, acc);
+    const uint32_t np = stencil27<PRED, AHEAD, !LDS>(LDS ? all : pos, off, k, active, pi, g, 0u, active ? cell_of[k] : 0u, tr, c, acc);
     acc.template merge<kPairLanes>();
     double esum = 0.0, vsum = 0.0;
     const uint32_t ks = wbase + __lane_id() / kPairLanes;  // = k

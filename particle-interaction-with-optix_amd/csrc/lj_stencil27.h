@@ -62,7 +62,7 @@ __device__ inline uint32_t of_odd(uint32_t v) {
 // lanes): 1,000 particles 90 -> 42 (from a copy in LDS), 100,000 of 27 partners 98 -> 66, of 70 135 -> 98,
 // 300,000 clustered 248 -> 190, 131,073 CUDALJ 137 -> 87.  Splitting the rows over the lanes
 // instead, or four and eight lanes, gained less at 100,000 and cost 10-50 % at a million.
-template <int PRED, bool AHEAD, class Sink>
+template <int PRED, bool AHEAD, bool LIMITS = true, class Sink>
 __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restrict__ off, uint32_t k,
                                      bool active, const float4& pi, const GridGeom& g, uint32_t cbase, uint32_t key,
                                      const Trim& tr, const PairConst& c, Sink& acc) {
@@ -114,15 +114,17 @@ __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restri
     range(4, inz && inp, 1, 1, gz + gyp);
     uint32_t np = 0;
     const f32x4* const p4 = reinterpret_cast<const f32x4*>(pos);
-    // candidate t + q kPairLanes exists iff t < lim[q]
+    // candidate t + q kPairLanes exists iff t < lim[q] (or, without LIMITS, t + q kPairLanes <
+    // lim[0])
     auto limits = [](uint32_t e, uint32_t (&lim)[kCandidates]) {
+        lim[0] = e;
 #pragma unroll
-        for (int q = 1; q < kCandidates; ++q) lim[q] = e > (uint32_t)(q * kPairLanes) ? e - (uint32_t)(q * kPairLanes) : 0u;
+        for (int q = 1; LIMITS && q < kCandidates; ++q) lim[q] = e > (uint32_t)(q * kPairLanes) ? e - (uint32_t)(q * kPairLanes) : 0u;
     };
     auto visit = [&](uint32_t t, const uint32_t (&lim)[kCandidates], const f32x4 (&v)[kCandidates]) {
 #pragma unroll
         for (int q = 0; q < kCandidates; ++q) {
-            if (q > 0 && t >= lim[q]) continue;
+            if (q > 0 && (LIMITS ? t >= lim[q] : t + q * kPairLanes >= lim[0])) continue;
             const float4 pj = make_float4(v[q].x, v[q].y, v[q].z, v[q].w);
             const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
             const float d2 = dist2(dx, dy, dz);
@@ -136,7 +138,8 @@ __device__ inline uint32_t stencil27(const float4* pos, const uint32_t* __restri
     // One 64-bit base, the candidates at immediate offsets from it, and their limits kept
     // from step to step (a batch of 25.5M particles in systems of 2,000-60,000 of 70
     // neighbours: 9,675 us with both formed anew for each candidate, 9,472 with the one base,
-    // 9,182 with the limits too).
+    // 9,182 with the limits too).  Without LIMITS the latter are formed for each candidate
+    // (the copy in LDS: 1,000 particles 42.4 us with them, 42.1 without).
     auto load = [&](uint32_t t, f32x4 (&v)[kCandidates]) {
         const f32x4* const pt = p4 + t;
 #pragma unroll
