@@ -235,7 +235,9 @@ int lj_lbvh_compute(lj_context* ctx, const float* x, const float* y, const float
                     const lj_params* p, float* fx, float* fy, float* fz, float* e,
                     lj_result* result, void* stream);
 
-/* Device: neighbour lists through the LBVH, same contract as lj_pairs. */
+/* Device: neighbour lists through the LBVH, same contract as lj_pairs.  Up to 524,288
+ * particles the context's workspace then also holds 1 KiB a particle (at most 512 MiB)
+ * until the context is destroyed; a call that cannot allocate it goes without, slower. */
 int lj_lbvh_pairs(lj_context* ctx, const float* x, const float* y, const float* z, int64_t n,
                   const lj_params* p, unsigned long long* row_offsets, uint32_t* cols,
                   unsigned long long capacity, unsigned long long* needed, void* stream);

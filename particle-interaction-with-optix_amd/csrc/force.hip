@@ -284,11 +284,13 @@ constexpr uint32_t kPairChunk = kPairBatches * kWaveSize;
 constexpr int kListStride = (int)kRegRow + kRowLanes;
 // Runs among a workgroup's 64 slots from which on it takes them as sparse: four slots a cell.
 // lj_pairs as a whole, us, runs only -> with the sparse form (one thread per particle, with
-// its sort in the list): 1,000,000 uniform particles of 0.5 neighbours 794 -> 231 (230), of 3
-// 714 -> 264 (304), of 6 610 -> 309 (456), of 12 547 -> 403 (864), of 20 512 -> 498 (1,635);
-// on a sphere of 3 1,122 -> 694 (790).  With the line at 20 runs 235, 267, 314, 429 and 520.
-// Still behind one thread per particle at 3,000,000 uniform particles of 0.5 neighbours, 549
-// against 487, where a cell in eight holds one.
+// its sort in the list): 1,000,000 uniform particles of 0.5 neighbours 793 -> 236 (230), of 3
+// 714 -> 268 (304), of 6 613 -> 316 (456), of 12 549 -> 409 (864), of 20 514 -> 504 (1,635);
+// on a sphere of 3 1,127 -> 700 (790).  With the line at 20 runs the times of 6, 12 and 20
+// neighbours were 1, 6 and 4 % longer.  Still behind one thread per particle at 3,000,000
+// uniform particles of 0.5 and 1.5 neighbours, 550 and 569 against 490 and 512, where a cell
+// in eight or less than one in two holds a particle: a workgroup of 256 particles there
+// shared more of the offsets' lines.
 constexpr int kSparseRuns = 16;
 // A workgroup's sparse rows share its lists.
 constexpr uint32_t kSparseRow = 4 * kListStride / kPairSlots;
