@@ -279,7 +279,9 @@ __global__ __launch_bounds__(256) void k_fill_gaps(const GapPiece* __restrict__ 
 // digits, ranked as in sortk::k_scatter), the sorted keys and particles, and the cell
 // offsets.  Up to kSmallN particles and kGapNoList cells, where the four or more launches of
 // the general path (histogram, digit scan and scatter per pass, offsets) cost 3-4 us each
-// whatever they do.  1,000 particles in 64 cells: 8 us against 15.
+// whatever they do.  1,000 particles in 64 cells: 8 us against 15; lj_bin with its counts, us,
+// one workgroup and the general path: 4,096 particles in 64 cells 28 and 37, in 4,096 29 and
+// 46, in 64,000 48 and 55, clustered 51 and 64; 64 particles in 64,000 cells 58 and 70.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallItems = 4;
 constexpr int kSmallN = kSmallThreads * kSmallItems;

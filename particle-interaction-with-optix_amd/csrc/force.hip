@@ -91,10 +91,11 @@ __global__ __launch_bounds__(kMaxBlock, 8) void k_force(const float4* __restrict
 // 27-cell candidates of the same grid (none when no result is wanted): they need only the
 // offsets, and a launch of their own costs 4-5 us.
 // LDS: every workgroup first copies all the particles to LDS and walks them there: a system
-// of up to kLdsParticles leaves a SIMD one wave at most, which waits out each load (1,000
-// particles of 64 partners: 39 us from the caches, 33 us from LDS, now bound by the issue of
-// that one wave's 60 steps of three candidates).
-constexpr uint32_t kLdsParticles = 2048;
+// of up to kLdsParticles leaves a SIMD one wave at most, which waits out each load, and is
+// otherwise bound by the issue of that wave's steps.  lj_compute, us, from the caches -> from
+// LDS: 200 particles of 50 neighbours 32.2 -> 31.7, 500 of 64 44.4 -> 43.0, 1,000 42.5 -> 42.1,
+// 1,200 level, 2,048 of 30 36.3 -> 37.3, of 5 27.0 -> 27.9.
+constexpr uint32_t kLdsParticles = 1024;
 
 template <int PRED, int PREC, bool VIR, bool LDS, bool AHEAD>
 __global__ __launch_bounds__(kMaxBlock, LDS || AHEAD ? 4 : 8) void k_force27(const float4* __restrict__ pos,

@@ -480,9 +480,9 @@ def test_bin_at_the_digit_scan_sizes(engine, n, cells):
 
 
 @pytest.mark.parametrize("cells", [1, 2, 16, 40])
-@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 257, 1024, 2047, 2048, 2049, 4095, 4096, 4097])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 257, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097])
 def test_small_systems_on_both_sides_of_the_limits(engine, n, cells):
-    """Binning in one workgroup (up to 4,096 particles) and forces from LDS (up to 2,048),
+    """Binning in one workgroup (up to 4,096 particles) and forces from LDS (up to 1,024),
     keys of 0, 3, 12 and 16 bits, dense and mostly empty cells: offsets, permutation and
     counts bit-exact, forces within 1e-5 of FP64."""
     x, y, z = ljamd.generate("clusters", 7 * n + cells, n, [2, 0.15, 0.3, 0.7])
