@@ -256,6 +256,11 @@ __global__ __launch_bounds__(kWaveSize) void k_batch_force_shared(
 // their values per slot, as the waves of k_batch_force_shared do.  (One wave that took its
 // systems one after the other kept more alive across them than its 64 registers hold.)
 constexpr uint32_t kWaveSlots27 = kWaveSize / kPairLanes;
+// Threads of a workgroup where the caller names none and the call fills the chip; us, 256 ->
+// 128 threads (why the middle size wins was not found out): 32 systems of 65,536 particles on spheres 647 -> 565, 28 of 450,000 of 20 neighbours 2,632 ->
+// 2,476, 13 of a million 2,997 -> 2,786, 25.5M in systems of 2,000-60,000 6,321 -> 6,283; with
+// 64 threads 631, 2,674, 3,020 and 6,270.  Up to kAheadMax particles 256 are level or ahead.
+constexpr unsigned kBlock27 = 128;
 
 template <int PRED, int PREC, bool AHEAD>
 __global__ __launch_bounds__(kMaxBlock, AHEAD ? 4 : 8) void k_batch_force27(
@@ -563,8 +568,9 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
     const uint32_t* cell_of = B.sorted_keys();
     {
         PhaseTimer tf(ctx, LJ_PHASE_FORCE, s);
-        const unsigned nb = div_up(n, sh.block), nb27 = div_up(n * kPairLanes, sh.block);
-        const unsigned nextra = (unsigned)(extra.size() / 2), nx27 = div_up((int64_t)nextra * kWaveSize, sh.block);
+        const unsigned block27 = p0.block || n <= kAheadMax ? (unsigned)sh.block : kBlock27;
+        const unsigned nb = div_up(n, sh.block), nb27 = div_up(n * kPairLanes, block27);
+        const unsigned nextra = (unsigned)(extra.size() / 2), nx27 = div_up((int64_t)nextra * kWaveSize, block27);
         const size_t lds = sh.lds_bytes();
         const size_t lds_shared = sh.queued() ? (size_t)sh.depth * kWaveSize * sizeof(QEntry) : 0;
         if (n > 0) {
@@ -580,7 +586,7 @@ extern "C" int lj_compute_batched(lj_context* ctx, const lj_system* sys, int32_t
                                (uint32_t)sh.depth, fx, fy, fz, e, ev, npair, wrec);                                 \
     } while (0)
 #define LJ_BF27(PRED, PREC, AHEAD)                                                                                  \
-    hipLaunchKernelGGL((k_batch_force27<PRED, PREC, AHEAD>), grid_of_blocks(nb27 + nx27), dim3(sh.block), 0, s, pos, cell_of,  \
+    hipLaunchKernelGGL((k_batch_force27<PRED, PREC, AHEAD>), grid_of_blocks(nb27 + nx27), dim3(block27), 0, s, pos, cell_of,  \
                        (const uint32_t*)off, (uint32_t)n, dsys, dcbase, hcbase, (uint32_t)nsys, most, nb27, dextra,  \
                        nextra, fx, fy, fz, e, ev, npair, wrec27)
 #define LJ_BF(PRED, PREC)                                                                                          \

@@ -17,9 +17,8 @@ constexpr int kPairLanes = 2;
 // (lj_compute, us, one lane -> two): 100,000 of 27 neighbours 98 -> 66, 1,000,000 of 70 446 ->
 // 408, on a sphere 278 -> 241; at 3,000,001 uniform of 45 867 -> 851, on a sphere 670 -> 722.
 // In batches that fill the chip: 25.5M particles in systems of 2,000-60,000 of 40 and 70
-// neighbours 6,419 -> 6,270 and 9,401 -> 9,172, 28 systems of 450,000 of 40 level (3,290 and
-// 3,320); 13 of a million of 40 3,480 -> 3,670, where a wave's 32 particles share fewer of
-// the lines that its rows no longer find in the CU's cache.
+// neighbours 6,419 -> 6,270 and 9,401 -> 9,172, 28 systems of 450,000 of 40 3,288 -> 3,225, 13
+// of a million of 40 3,479 -> 3,518.
 constexpr int64_t kTwoLaneMax = (int64_t)1 << 20;
 // Calls of up to this many particles in all load a step ahead (about four waves a SIMD):
 // us without -> with, 30,000 particles of 70 partners 74 -> 66, 65,000 92 -> 83, clustered
